@@ -3,16 +3,19 @@
 //
 // Reference: gemm.rs (6x16 AVX2 micro-kernel over KC=256 packed panels,
 // parallel over 6-row C panels), linear.rs.  Here one workgroup owns a
-// BM x BN tile of C; its 4 compute waves each own a (BM/2) x (BN/2) sub-tile
-// made of 32x32 v_mfma_f32_32x32x2f32 accumulators.  The k order inside a
-// block of 8 is permuted identically for A and B (step s of group g, lane
-// half h  <->  k = 8g + 4h + s), so a k-contiguous operand gives a lane the
-// values of 4 MFMA steps with one ds_read_b128.  Two ways to stage operands:
-//   * gemm_dma_kernel (every operand whose 16-byte quads are whole): 4 more
-//     waves DMA the slabs from HBM straight into a multi-stage LDS ring;
+// BM x BN tile of C, its compute waves sub-tiles of 32x32 MFMA accumulators.
+// Two kernels:
+//   * gemm_dma_kernel (every operand whose 16-byte quads are whole): producer
+//     waves DMA the slabs from HBM straight into a multi-stage LDS ring; the
+//     products run on the bf16 matrix cores, each float in three exact parts
+//     (mfma_split.h);
 //   * gemm_kernel (any shape and alignment): the 4 waves load a slab into
 //     registers and store it k-contiguous (16 k values + 4 pad floats a row)
-//     into a double-buffered LDS tile.
+//     into a double-buffered LDS tile, multiplied by v_mfma_f32_32x32x2f32
+//     (k order inside a block of 8 permuted identically for A and B: step s
+//     of group g, lane half h  <->  k = 8g + 4h + s, so a lane gets the values
+//     of 4 MFMA steps with one ds_read_b128).
+#include "mfma_split.h"
 #include "rnn_internal.h"
 
 #include <algorithm>
@@ -217,13 +220,16 @@ struct GemmTile {
 //     of row r at position q ^ kswz(r), so the ds_read_b128 of 8 (or 16)
 //     consecutive rows at one quad hit distinct banks;
 //   * row-contiguous (A^T [k][m], B [k][n]): [BK][rows] as stored, read one
-//     float per MFMA step (32 consecutive floats per half-wave).
-// k order inside a stage matches the register-staged kernel: step s of
-// group g, lane half h <-> k = 8g + 4h + s.  Eligible when every 16-byte quad
-// is either wholly inside the operand or wholly outside (rows and k multiples
-// of 4 where they run along a quad, 16-byte aligned bases): a quad outside
-// the k range reads zero through an out-of-range offset; rows beyond M / N
-// only feed C rows / columns that are never stored.
+//     float per k (32 consecutive floats per half-wave).
+// Eligible when every 16-byte quad is either wholly inside the operand or
+// wholly outside (rows and k multiples of 4 where they run along a quad,
+// 16-byte aligned bases): a quad outside the k range reads zero through an
+// out-of-range offset; rows beyond M / N only feed C rows / columns that are
+// never stored.
+//
+// The product of two float fragments is taken on the bf16 matrix cores: each
+// float is the exact sum of three bf16 parts (mfma_split.h), and six of the
+// nine part products are summed into the fp32 accumulator.
 
 // s_waitcnt with vmcnt <= N, other counters not waited on (vmcnt bits 3:0 and
 // 15:14, expcnt 6:4, lgkmcnt 11:8).
@@ -237,81 +243,125 @@ __device__ __forceinline__ void wait_vmcnt() {
 // both 8-lane (32-bank) and 16-lane (64-bank) LDS read phases.
 template <int BK>
 __device__ __forceinline__ int kswz(int r) {
-    if constexpr (BK == 32)
+    if constexpr (BK >= 32)
         return (r ^ (r >> 3)) & 7;
     else
         return ((r >> 1) ^ (r >> 2)) & 3;
 }
 
-template <int R, int BK, bool KMAJOR>
+template <int R, int BK, bool KMAJOR, int NP>
 struct DmaOperand {
-    static constexpr int WORDS = R * BK;             // LDS floats per stage
-    static constexpr int PER = WORDS / 4 / 256;      // dwordx4 DMAs per thread
-    static_assert(WORDS % 1024 == 0, "whole DMA rows");
+    static constexpr int WORDS = R * BK;               // LDS floats per stage
+    static constexpr int PER = WORDS / 4 / (64 * NP);  // dwordx4 DMAs per producer thread
+    static_assert(WORDS % (256 * NP) == 0, "whole DMA rows");
 
-    // Issues this thread's DMAs of rows r0.. (KMAJOR) or columns r0.. of
-    // k values k0 .. k0 + BK (of kz) into lds.
-    __device__ __forceinline__ static void issue(__amdgpu_buffer_rsrc_t rs, int ld, int rows,
-                                                 int r0, int k0, int kz, float *lds, int wave,
-                                                 int lane) {
+    // This thread's source byte offsets at k = 0, per DMA of a stage: rows
+    // r0.. (KMAJOR) or columns r0.. of a stage's k values.  A stage adds its
+    // k offset in a scalar, so that an issue costs no vector arithmetic.
+    uint32_t off[PER];
+
+    // DMA u's quad of this lane in a stage's slab.
+    __device__ __forceinline__ static int quad(int u, int wave, int lane) {
+        return (u * NP + wave) * 64 + lane;
+    }
+    // First k of quad j, relative to the stage.
+    __device__ __forceinline__ static int kof(int j) {
+        if (KMAJOR) return ((j % (BK / 4)) ^ kswz<BK>(j / (BK / 4))) * 4;
+        return j / (R / 4);
+    }
+    __device__ __forceinline__ void init(int ld, int rows, int r0, int wave, int lane) {
 #pragma unroll
         for (int u = 0; u < PER; u++) {
-            const int c0 = (u * 4 + wave) * 64;  // first quad of this wave instruction
-            const int j = c0 + lane;
-            uint32_t off;
-            if (KMAJOR) {
-                constexpr int QPR = BK / 4;
-                const int r = j / QPR, q = (j % QPR) ^ kswz<BK>(r);
-                const int row = r0 + r, k = k0 + 4 * q;
-                off = (row < rows && k < kz) ? (uint32_t)(row * ld + k) * 4u : DMA_OOB;
-            } else {
-                constexpr int QPR = R / 4;
-                const int kr = j / QPR, col = r0 + (j % QPR) * 4, k = k0 + kr;
-                off = (k < kz && col < rows) ? (uint32_t)(k * ld + col) * 4u : DMA_OOB;
-            }
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(lds + 4 * c0), 16, off, 0, 0,
-                                                     0);
+            const int j = quad(u, wave, lane);
+            const int row = KMAJOR ? r0 + j / (BK / 4) : r0 + j % (R / 4) * 4;
+            off[u] = row >= rows ? DMA_OOB
+                     : KMAJOR    ? (uint32_t)(row * ld + kof(j)) * 4u
+                                 : (uint32_t)(kof(j) * ld + row) * 4u;
+        }
+    }
+    // Issues this thread's DMAs of k values k0 .. k0 + BK (of kz) into lds.
+    __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rs, int ld, int k0, int kz,
+                                          float *lds, int wave, int lane) const {
+        const uint32_t so = (uint32_t)(KMAJOR ? k0 : k0 * ld) * 4u;
+        const bool whole = k0 + BK <= kz;
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            uint32_t o = off[u];
+            if (!whole && k0 + kof(quad(u, wave, lane)) >= kz) o = DMA_OOB;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs, (lds_ptr_t)(lds + 4 * quad(u, wave, 0)), 16, o, so, 0, 0);
         }
     }
 
-    // The operand values of MFMA steps 0..3 of group g for tile row (or
-    // column) `row` and lane half h.
-    __device__ __forceinline__ static f32x4 frag(const float *lds, int row, int g, int h) {
+    // The operand values of tile row (or column) `row` at k = 16 s + 8 h + j,
+    // j = 0..7: lane half h's share of 16 k values.
+    __device__ __forceinline__ static void frag(const float *lds, int row, int s, int h,
+                                                float (&x)[8]) {
         if (KMAJOR) {
-            const int q = (2 * g + h) ^ kswz<BK>(row);
-            return *reinterpret_cast<const f32x4 *>(lds + row * BK + 4 * q);
+            const float *p = lds + row * BK;
+            const int q = 4 * s + 2 * h, w = kswz<BK>(row);
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(p + 4 * (q ^ w));
+            const f32x4 b = *reinterpret_cast<const f32x4 *>(p + 4 * ((q + 1) ^ w));
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                x[j] = a[j];
+                x[4 + j] = b[j];
+            }
         } else {
-            const float *p = lds + (8 * g + 4 * h) * R + row;
-            f32x4 v;
-            v[0] = p[0];
-            v[1] = p[R];
-            v[2] = p[2 * R];
-            v[3] = p[3 * R];
-            return v;
+            const float *p = lds + (16 * s + 8 * h) * R + row;
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[j] = p[j * R];
         }
     }
 };
 
-// One BM x BN tile of C = op(A) op(B) over kz values of k by 8 waves.
-// Waves 0..3 multiply (a 2 x 2 grid of (BM/2) x (BN/2) sub-tiles); waves
-// 4..7 only issue the DMAs, a whole stage at a time, so the compute waves
-// never wait on the memory pipeline.  One barrier per stage: when it
-// completes, stage it has landed (each producer waited for its own DMAs) and
-// every compute wave is done with stage it - 1, whose buffer the producers
-// then refill with stage it + NS - 1.  A wave with a single 32 x 32 block
-// alternates two accumulators so that consecutive MFMAs are independent.
-template <int BM, int BN, int BK, int NS, bool AT, bool BT>
+// One BM x BN tile of C = op(A) op(B) over kz values of k by NC compute waves
+// and NP producer waves.  The compute waves are a WM x WN grid of (BM/WM) x
+// (BN/WN) sub-tiles, times WK shares of each stage's k: the waves of a share
+// group hold partial sums of one sub-tile, exchanged through LDS at the end,
+// and each keeps its part of the sub-tile's accumulator groups (8 registers:
+// rows 16h + 8(e/4) + 4(lane/32) + e%4 of a 32 x 32 block).  Producer waves
+// only issue the DMAs, a whole stage at a time, so the compute waves never
+// wait on the memory pipeline.  One barrier per stage: when it completes,
+// stage it has landed (each producer waited for its own DMAs) and every
+// compute wave is done with stage it - 1, whose buffer the producers then
+// refill with stage it + NS - 1.
+template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, bool AT, bool BT>
 struct DmaTile {
-    using OA = DmaOperand<BM, BK, !AT>;
-    using OB = DmaOperand<BN, BK, BT>;
+    static constexpr int NC = WM * WN * WK;
+    using OA = DmaOperand<BM, BK, !AT, NP>;
+    using OB = DmaOperand<BN, BK, BT, NP>;
+    static constexpr int ROWS = BM, COLS = BN, THREADS = 64 * (NC + NP);
     static constexpr int STAGE = OA::WORDS + OB::WORDS;
-    static constexpr size_t LDS_BYTES = (size_t)NS * STAGE * 4;
-    static constexpr int WTM = BM / 2, WTN = BN / 2, TM = WTM / 32, TN = WTN / 32;
-    static constexpr int NACC = TM * TN == 1 ? 2 : 1;
-    f32x16 acc[TM][TN][NACC];
+    static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+    // the ring, or the exchange of partial sums (and row sums) that follows it
+    static constexpr int XWORDS = WK > 1 ? NC * (TM * TN * 1024 + TM * 128) : 0;
+    static constexpr size_t LDS_BYTES = (size_t)(NS * STAGE > XWORDS ? NS * STAGE : XWORDS) * 4;
+    // workgroups that the LDS leaves room for on a CU, as waves on a SIMD
+    static constexpr int OCC = ((int)(160 * 1024 / LDS_BYTES) * (NC + NP) + 3) / 4;
+    static constexpr int NG = TM * TN * 2 / WK;  // accumulator groups a wave keeps
+    static_assert(TM * TN * 2 % WK == 0 && BK % (16 * WK) == 0, "wave layout");
+    float acc[NG][8];
     // With rsum, the f64 sums of the A values this lane multiplies: row
-    // wm*WTM + 32i + lr at k = 8g + 4lh + s, stage by stage in k order.
+    // wm*WTM + 32i + lr, stage by stage in k order (of share 0: of all k).
     double rs[TM];
+
+    __device__ __forceinline__ static int wk() { return wave_index() / (WM * WN); }
+    __device__ __forceinline__ static int wm() { return wave_index() / WN % WM; }
+    __device__ __forceinline__ static int wn() { return wave_index() % WN; }
+    __device__ __forceinline__ static int row0() { return wm() * WTM; }
+    // Tile row and column of element 0 of kept group o (before the lane's part).
+    __device__ __forceinline__ static int grow(int o) {
+        const int g = wk() * NG + o;
+        return row0() + g / (2 * TN) * 32 + (g & 1) * 16;
+    }
+    __device__ __forceinline__ static int gcol(int o) {
+        return wn() * WTN + (wk() * NG + o) / 2 % TN * 32;
+    }
+    // The row of element e of a group, past grow(), in lane half lh.
+    __device__ __forceinline__ static int erow(int e, int lh) {
+        return 8 * (e >> 2) + 4 * lh + (e & 3);
+    }
 
     // Producer waves return false once their last DMA is issued; compute
     // waves return true with the tile in acc.  A, B: this problem's operands
@@ -320,15 +370,19 @@ struct DmaTile {
                                         int N, int kz, int m0, int n0, bool rsum, float *lds) {
         const int lane = threadIdx.x & 63, wave = wave_index();
         const int nk = (kz + BK - 1) / BK;
-        if (wave >= 4) {
-            const int pw = wave - 4;
+        if (wave >= NC) {
+            const int pw = wave - NC;
             const uint32_t abytes = (uint32_t)((AT ? (long long)kz * lda : (long long)M * lda) * 4);
             const uint32_t bbytes = (uint32_t)((BT ? (long long)N * ldb : (long long)kz * ldb) * 4);
             const __amdgpu_buffer_rsrc_t ra = make_rsrc(A, abytes), rb = make_rsrc(B, bbytes);
+            OA oa;
+            OB ob;
+            oa.init(lda, M, m0, pw, lane);
+            ob.init(ldb, N, n0, pw, lane);
             auto issue = [&](int st) {
                 float *buf = lds + (st % NS) * STAGE;
-                OA::issue(ra, lda, M, m0, st * BK, kz, buf, pw, lane);
-                OB::issue(rb, ldb, N, n0, st * BK, kz, buf + OA::WORDS, pw, lane);
+                oa.issue(ra, lda, st * BK, kz, buf, pw, lane);
+                ob.issue(rb, ldb, st * BK, kz, buf + OA::WORDS, pw, lane);
             };
 #pragma unroll
             for (int st = 0; st < NS - 1; st++)
@@ -345,9 +399,14 @@ struct DmaTile {
                 asm volatile("" ::: "memory");
                 if (it + NS - 1 < nk) issue(it + NS - 1);
             }
+            if constexpr (WK > 1) {  // the compute waves' exchange
+                __syncthreads();
+                __syncthreads();
+            }
             return false;
         }
-        const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lh = lane >> 5;
+        const int lr = lane & 31, lh = lane >> 5;
+        f32x16 sum[TM][TN];
 #pragma unroll
         for (int i = 0; i < TM; i++) rs[i] = 0.0;
 #pragma unroll
@@ -355,80 +414,167 @@ struct DmaTile {
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int a = 0; a < NACC; a++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) acc[i][j][a][v] = 0.f;
+                for (int v = 0; v < 16; v++) sum[i][j][v] = 0.f;
+        constexpr int NSTEP = BK / 16 / WK;
+        const int s0 = wk() * NSTEP, ra0 = row0() + lr, rb0 = wn() * WTN + lr;
+        // Odd shares multiply -A (subtracted in the exchange); a tile without
+        // shares turns the sign of its sums every few stages: the matrix
+        // core's rounding toward -inf cancels (mfma_split.h).
+        uint32_t neg = WK > 1 && (wk() & 1) ? 0x80000000u : 0u;
+        const int flip = min(8, max(1, nk / 4));
+        int turn = flip;
         for (int it = 0; it < nk; it++) {
+            if constexpr (WK == 1)
+                if (turn-- == 0) {
+                    turn = flip - 1;
+                    neg ^= 0x80000000u;
+                    bf3_negate<TM, TN>(sum);
+                }
             __syncthreads();
             const float *As = lds + (it % NS) * STAGE, *Bs = As + OA::WORDS;
-            f32x4 af[TM], bf[TN];
 #pragma unroll
-            for (int i = 0; i < TM; i++) af[i] = OA::frag(As, wm * WTM + i * 32 + lr, 0, lh);
+            for (int u = 0; u < NSTEP; u++) {
+                float x[TM + TN][8];
 #pragma unroll
-            for (int j = 0; j < TN; j++) bf[j] = OB::frag(Bs, wn * WTN + j * 32 + lr, 0, lh);
+                for (int i = 0; i < TM; i++) OA::frag(As, ra0 + 32 * i, s0 + u, lh, x[i]);
 #pragma unroll
-            for (int gk = 0; gk < BK / 8; gk++) {
-                f32x4 an[TM], bn[TN];
-                if (gk + 1 < BK / 8) {
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-                        an[i] = OA::frag(As, wm * WTM + i * 32 + lr, gk + 1, lh);
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        bn[j] = OB::frag(Bs, wn * WTN + j * 32 + lr, gk + 1, lh);
-                }
-                // keep the next group's reads ahead of this group's MFMAs
-                __builtin_amdgcn_sched_barrier(0);
+                for (int j = 0; j < TN; j++) OB::frag(Bs, rb0 + 32 * j, s0 + u, lh, x[TM + j]);
                 if (rsum) {
 #pragma unroll
                     for (int i = 0; i < TM; i++)
 #pragma unroll
-                        for (int s = 0; s < 4; s++) rs[i] += (double)af[i][s];
+                        for (int e = 0; e < 8; e++) rs[i] += (double)x[i][e];
                 }
 #pragma unroll
-                for (int s = 0; s < 4; s++)
+                for (int i = 0; i < TM; i++)
 #pragma unroll
-                    for (int i = 0; i < TM; i++)
+                    for (int e = 0; e < 8; e++)
+                        x[i][e] = __uint_as_float(__float_as_uint(x[i][e]) ^ neg);
+                Bf3 p[TM + TN];
 #pragma unroll
-                        for (int j = 0; j < TN; j++)
-                            acc[i][j][s % NACC] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                af[i][s], bf[j][s], acc[i][j][s % NACC], 0, 0, 0);
-                if (gk + 1 < BK / 8) {
-#pragma unroll
-                    for (int i = 0; i < TM; i++) af[i] = an[i];
-#pragma unroll
-                    for (int j = 0; j < TN; j++) bf[j] = bn[j];
-                }
+                for (int i = 0; i < TM + TN; i++) p[i] = bf3_split(x[i]);
+                bf3_mfma<TM, TN>(p, p + TM, sum);
             }
         }
+        if constexpr (WK > 1) {
+            // The ring, free once every wave is past its last stage, takes
+            // all partial sums; a wave adds its groups' over the shares (odd
+            // ones with their sign turned back), in share order.
+            __syncthreads();
+            f32x4 *x = reinterpret_cast<f32x4 *>(lds);
+            double *xr = reinterpret_cast<double *>(lds + NC * TM * TN * 1024);
+#pragma unroll
+            for (int q = 0; q < TM * TN * 4; q++) {
+                const f32x16 &t = sum[q / (4 * TN)][q / 4 % TN];
+                x[(wave * TM * TN * 4 + q) * 64 + lane] =
+                    f32x4{t[4 * (q & 3)], t[4 * (q & 3) + 1], t[4 * (q & 3) + 2], t[4 * (q & 3) + 3]};
+            }
+            if (rsum)
+#pragma unroll
+                for (int i = 0; i < TM; i++) xr[(wave * TM + i) * 64 + lane] = rs[i];
+            __syncthreads();
+            const int w0 = wave % (WM * WN), k = wk();
+#pragma unroll
+            for (int o = 0; o < NG; o++)
+#pragma unroll
+                for (int e4 = 0; e4 < 2; e4++) {
+                    const int q = (k * NG + o) * 2 + e4;
+                    f32x4 t = x[(w0 * TM * TN * 4 + q) * 64 + lane];
+#pragma unroll
+                    for (int s = 1; s < WK; s++) {
+                        const f32x4 u = x[((s * WM * WN + w0) * TM * TN * 4 + q) * 64 + lane];
+                        t = s & 1 ? t - u : t + u;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[o][4 * e4 + e] = t[e];
+                }
+            if (rsum && k == 0)
+#pragma unroll
+                for (int s = 1; s < WK; s++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+                        rs[i] += xr[((s * WM * WN + w0) * TM + i) * 64 + lane];
+        } else {
+            if (neg) bf3_negate<TM, TN>(sum);
+#pragma unroll
+            for (int o = 0; o < NG; o++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[o][e] = sum[o / (2 * TN)][o / 2 % TN][8 * (o & 1) + e];
+        }
+        // An operand's infinity has no split (its parts are inf and NaN), and
+        // part sums can overflow where the values' do not: groups that are
+        // not finite are taken again on the fp32 matrix cores.
+        bool bad = false;
+#pragma unroll
+        for (int o = 0; o < NG; o++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) bad = bad || bf3_nonfinite(acc[o][e]);
+        if (__any(bad)) slow(A, lda, M, B, ldb, N, kz, m0, n0);
         return true;
     }
 
-    // f(r, c, v) for each element of the tile this compute lane holds (tile
-    // row r = wm*WTM + 32i + 8(v/4) + 4(lane/32) + v%4, column wn*WTN + 32j +
-    // lane%32: the 32x32 MFMA accumulator layout).
+    // acc over all of kz with fp32 MFMAs, from global memory.
+    __device__ __forceinline__ void slow(const float *A, int lda, int M, const float *B, int ldb,
+                                         int N, int kz, int m0, int n0) {
+        const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+#pragma unroll
+        for (int o = 0; o < NG; o++) {
+            const int hi = grow(o) & 16, r = m0 + (grow(o) & ~16) + lr, c = n0 + gcol(o) + lr;
+            f32x16 t;
+#pragma unroll
+            for (int v = 0; v < 16; v++) t[v] = 0.f;
+            for (int k0 = 0; k0 < kz; k0 += 2) {
+                const int k = k0 + lh;
+                const long long ao = AT ? (long long)k * lda + r : (long long)r * lda + k;
+                const long long bo = BT ? (long long)c * ldb + k : (long long)k * ldb + c;
+                const float a = k < kz && r < M ? A[ao] : 0.f, b = k < kz && c < N ? B[bo] : 0.f;
+                t = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, t, 0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[o][e] = hi ? t[8 + e] : t[e];
+        }
+    }
+
+    // f(r, c, v) for each element of the tile that this compute lane keeps.
     template <typename F>
     __device__ __forceinline__ void each(F f) const {
-        const int lane = threadIdx.x & 63, wave = wave_index();
-        const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lh = lane >> 5;
+        const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+        for (int o = 0; o < NG; o++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    float val = acc[i][j][0][v];
-                    if (NACC == 2) val += acc[i][j][NACC - 1][v];
-                    f(wm * WTM + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3), wn * WTN + j * 32 + lr,
-                      val);
-                }
+            for (int e = 0; e < 8; e++) f(grow(o) + erow(e, lh), gcol(o) + lr, acc[o][e]);
     }
 };
 
-template <int BM, int BN, int BK, int NS, bool AT, bool BT, bool RS>
-__global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs g) {
+// The tiles.  Producers issue one DMA instruction a KiB, and that rate bounds
+// a stage when too few waves share it: 8192 x 256 x 768 with one / two / four
+// producer waves on the 64 x 64 tile 27.4 / 26.5 / 26.6 us, on a 64 x 64 x 64
+// stage 37.8 / 29.5 / 25.9; so four each.  Sub-tiles of 32 x 64 and 64 x 64
+// per wave keep the splitting (44 VALU instructions per fragment) at 11 and
+// 7.3 instructions an MFMA, of which about 4 hide behind it in one wave.
+// Measured (us; fp32-pipe kernel before -> 32 x 64 / 64 x 64 / 128 x 128 /
+// 256 x 128): 512^3 12.8 -> 8.1 / 12.8 / 26.6 / 44; 2048 x 384 x 384 10.1 ->
+// 8.6 / 9.9 / 21 / 36; 8192 x 768 x 256 34.6 -> 38 / 30.2 / 37 / 32; 8192 x
+// 256 x 768 32.1 -> 29 / 26.6 / 38 / 63; 16384 x 768 x 256 69.2 -> 78 / 56.4 /
+// 62 / 63; 2048^3 148 -> 148 / 113 / 103 / 156; 4096^3 1280 -> 1202 / 918 /
+// 818 / 766 (179 TFLOP/s).  The tiles with two or four shares of k also
+// shorten the accumulation chains (K = 256 error 2.05e-7 -> 1.76e-7).
+template <bool AT, bool BT>
+using Tile32 = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, AT, BT>;
+template <bool AT, bool BT>
+using Tile64 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, AT, BT>;
+template <bool AT, bool BT>
+using Tile128 = DmaTile<128, 128, 32, 3, 2, 2, 2, 4, AT, BT>;
+template <bool AT, bool BT>
+using Tile256 = DmaTile<256, 128, 16, 4, 4, 2, 1, 4, AT, BT>;
+// Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile.
+template <bool AT, bool BT>
+using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, AT, BT>;
+
+template <class Tile, bool RS>
+__global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(GemmArgs g) {
     extern __shared__ float lds[];
-    using Tile = DmaTile<BM, BN, BK, NS, AT, BT>;
+    constexpr int BM = Tile::ROWS, BN = Tile::COLS;
     const long long z = blockIdx.z;
     const int kz = min(g.kchunk, g.ktotal - (int)z * g.kchunk);
     // XCD-aware tile order, as in gemm_kernel
@@ -438,8 +584,8 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs g) {
     const int tl = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
     const int m0 = (tl / gx) * BM, n0 = (tl % gx) * BN;
     // RS: the compute waves of the first column tile also sum A's values
-    const int lane = threadIdx.x & 63, wave = wave_index(), lr = lane & 31, lh = lane >> 5;
-    const bool rsum = RS && n0 == 0 && (wave & 1) == 0;
+    const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+    const bool rsum = RS && n0 == 0 && Tile::wn() == 0;
     Tile t;
     if (!t.run(g.a + zoff(g, z, g.stride_a, g.stride_a2), g.lda, g.M,
                g.b + zoff(g, z, g.stride_b, g.stride_b2), g.ldb, g.N, kz, m0, n0,
@@ -451,8 +597,8 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs g) {
             // the two lane halves' sums, added in half order on both halves
             const double o = __shfl_xor(t.rs[i], 32, 64);
             const double s = lh == 0 ? t.rs[i] + o : o + t.rs[i];
-            const int row = m0 + (wave >> 1) * Tile::WTM + i * 32 + lr;
-            if (lh == 0 && row < g.M) {
+            const int row = m0 + Tile::row0() + i * 32 + lr;
+            if (lh == 0 && Tile::wk() == 0 && row < g.M) {
                 if (g.rsum_part)
                     g.rsum_part[z * g.M + row] = s;
                 else
@@ -466,11 +612,8 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs g) {
     // or the residual's old value and mask (res) -- is loaded before the
     // stores, eight elements at a time, so the loads are in flight together
     // instead of each waiting behind the stores before it (eight: the
-    // registers keep three 64 x 64 workgroups a CU).  Element (i, j, v):
-    // tile row wm*WTM + 32i + 8(v/4) + 4(lane/32) + v%4, column
-    // wn*WTN + 32j + lane%32 (the 32x32 MFMA accumulator layout).
+    // registers keep three 64 x 64 workgroups a CU).
     const bool acc = g.acc != 0, res = g.res != nullptr, bias = g.bias != nullptr;
-    const int wm = wave >> 1, wn = wave & 1;
     if (!acc && !res) {
         // (the plain store, written this way, measured faster than the
         // loop below with the bias preloaded: 5.84 vs 5.92 ms rustvit step)
@@ -484,43 +627,33 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs g) {
         return;
     }
 #pragma unroll
-    for (int j = 0; j < Tile::TN; j++) {
-        const int col = n0 + wn * Tile::WTN + j * 32 + lr, colc = min(col, g.N - 1);
+    for (int o = 0; o < Tile::NG; o++) {
+        const int col = n0 + Tile::gcol(o) + lr, colc = min(col, g.N - 1);
+        const int row0 = m0 + Tile::grow(o);
         const float bj = bias ? g.bias[colc] : 0.f, lj = res ? g.res_l[colc] : 0.f;
+        float old[8], mv[8];
 #pragma unroll
-        for (int i = 0; i < Tile::TM; i++)
+        for (int e = 0; e < 8; e++) {
+            const int rowc = min(row0 + Tile::erow(e, lh), g.M - 1);
+            const long long off = (long long)rowc * g.ldc + colc;
+            old[e] = acc ? Cp[off] : g.res[off];
+            mv[e] = (res && g.res_mask) ? g.res_mask[rowc >> g.res_shift] : 1.0f;
+        }
 #pragma unroll
-            for (int h = 0; h < 16; h += 8) {
-                float old[8], mv[8];
-                if (acc || res) {
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const int v = h + u;
-                        const int row = m0 + wm * Tile::WTM + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                        const long long o = (long long)min(row, g.M - 1) * g.ldc + colc;
-                        old[u] = acc ? Cp[o] : g.res[o];
-                        mv[u] = (res && g.res_mask) ? g.res_mask[min(row, g.M - 1) >> g.res_shift]
-                                                    : 1.0f;
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const int v = h + u;
-                    const int row = m0 + wm * Tile::WTM + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                    if (row < g.M && col < g.N) {
-                        float val = t.acc[i][j][0][v];
-                        if constexpr (Tile::NACC == 2) val += t.acc[i][j][1][v];
-                        if (bias) val += bj;
-                        const long long o = (long long)row * g.ldc + col;
-                        Cp[o] = acc ? old[u] + val : val;
-                        if (res) {
-                            float tr = val * lj;
-                            if (g.res_mask) tr = tr * mv[u];
-                            g.res[o] = old[u] + tr;
-                        }
-                    }
+        for (int e = 0; e < 8; e++) {
+            const int row = row0 + Tile::erow(e, lh);
+            if (row < g.M && col < g.N) {
+                float val = t.acc[o][e];
+                if (bias) val += bj;
+                const long long off = (long long)row * g.ldc + col;
+                Cp[off] = acc ? old[e] + val : val;
+                if (res) {
+                    float tr = val * lj;
+                    if (g.res_mask) tr = tr * mv[e];
+                    g.res[off] = old[e] + tr;
                 }
             }
+        }
     }
 }
 
@@ -629,7 +762,7 @@ template <bool AT, bool BT>
 __device__ __forceinline__ void ns_tile_dma(const NsGemmProb &p, uint32_t z, int ti, int tj,
                                             float alpha, float beta, float *lds) {
 #pragma clang fp contract(off)
-    using Tile = DmaTile<64, 64, 32, 3, AT, BT>;
+    using Tile = TileNs<AT, BT>;
     const int m0 = ti * 64, n0 = tj * 64;
     Tile t;
     if (!t.run(p.a + z * p.stride_a, p.lda, p.M, p.b + z * p.stride_b, p.ldb, p.N, p.K, m0, n0,
@@ -649,9 +782,9 @@ __device__ __forceinline__ void ns_tile_dma(const NsGemmProb &p, uint32_t z, int
     });
 }
 
-constexpr size_t NS_DMA_LDS = DmaTile<64, 64, 32, 3, false, false>::LDS_BYTES;
+using NsTile = TileNs<false, false>;
 
-__global__ __launch_bounds__(512) void ns_gemm_dma_kernel(const NsGemmProb *__restrict__ probs,
+__global__ __launch_bounds__(NsTile::THREADS, 3) void ns_gemm_dma_kernel(const NsGemmProb *__restrict__ probs,
                                                           int nprob, float alpha, float beta) {
     extern __shared__ float lds[];
     int lo = 0, hi = nprob - 1;
@@ -749,33 +882,33 @@ int launch_t(rnn_ctx *ctx, const GemmArgs &g, int count, bool vec) {
     return RNN_OK;
 }
 
-template <int BM, int BN, int BK, int NS, bool AT, bool BT, bool RS>
+template <class Tile, bool RS>
 int launch_dma_t(rnn_ctx *ctx, const GemmArgs &g, int count) {
-    constexpr size_t lds = DmaTile<BM, BN, BK, NS, AT, BT>::LDS_BYTES;
     static bool attr = false;
     if (!attr) {
         attr = true;
-        (void)hipFuncSetAttribute((const void *)gemm_dma_kernel<BM, BN, BK, NS, AT, BT, RS>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute((const void *)gemm_dma_kernel<Tile, RS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)Tile::LDS_BYTES);
     }
-    dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, count);
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, BK, NS, AT, BT, RS>), grid, dim3(512), lds,
+    dim3 grid((g.N + Tile::COLS - 1) / Tile::COLS, (g.M + Tile::ROWS - 1) / Tile::ROWS, count);
+    hipLaunchKernelGGL((gemm_dma_kernel<Tile, RS>), grid, dim3(Tile::THREADS), Tile::LDS_BYTES,
                        ctx->stream, g);
     RNN_LAUNCHED(ctx);
     return RNN_OK;
 }
 
 // The row sums of op(A) ride along only in the weight-gradient layout (A^T B).
-template <int BM, int BN, int BK, int NS>
-int launch_dma_bm(rnn_ctx *ctx, const GemmArgs &g, int count, bool at, bool bt) {
+template <template <bool, bool> class Tile>
+int launch_dma(rnn_ctx *ctx, const GemmArgs &g, int count, bool at, bool bt) {
     if (g.rsum_out || g.rsum_part) {
         if (!at || bt) return rnn_fail(ctx, RNN_E_INVALID, "gemm: row sums need the A^T B layout");
-        return launch_dma_t<BM, BN, BK, NS, true, false, true>(ctx, g, count);
+        return launch_dma_t<Tile<true, false>, true>(ctx, g, count);
     }
-    if (!at && !bt) return launch_dma_t<BM, BN, BK, NS, false, false, false>(ctx, g, count);
-    if (!at && bt) return launch_dma_t<BM, BN, BK, NS, false, true, false>(ctx, g, count);
-    if (at && !bt) return launch_dma_t<BM, BN, BK, NS, true, false, false>(ctx, g, count);
-    return launch_dma_t<BM, BN, BK, NS, true, true, false>(ctx, g, count);
+    if (!at && !bt) return launch_dma_t<Tile<false, false>, false>(ctx, g, count);
+    if (!at && bt) return launch_dma_t<Tile<false, true>, false>(ctx, g, count);
+    if (at && !bt) return launch_dma_t<Tile<true, false>, false>(ctx, g, count);
+    return launch_dma_t<Tile<true, true>, false>(ctx, g, count);
 }
 
 template <int BM, int BN>
@@ -876,13 +1009,20 @@ static int gemm_enqueue(rnn_ctx *ctx, size_t count, size_t m, size_t n, size_t k
     size_t tiles128 = rnn_div_up(m, 128) * rnn_div_up(n, 128) * count;
     if (dma_enabled() && stride_a2 % 4 == 0 && stride_b2 % 4 == 0 &&
         dma_ok(count, m, n, kchunk, ktotal, a, stride_a, lda, at, b, stride_b, ldb, bt)) {
-        // 128 x 128 tiles only from four tiles per CU: below that the 64 x 64
-        // grid's extra workgroups hide more latency than the larger tile's
-        // operand reuse saves (measured on MI355X: 8192x768x256 99 vs 79
-        // TFLOP/s, 4096^3 124 vs 136)
-        if (m >= 128 && n >= 128 && tiles128 >= 4 * (size_t)ctx->num_cus)
-            return launch_dma_bm<128, 128, 16, 4>(ctx, g, (int)count, at, bt);
-        return launch_dma_bm<64, 64, 32, 3>(ctx, g, (int)count, at, bt);
+        // The largest tile that still fills the chip (times at the tiles'
+        // definitions): 256 x 128 from two tiles a CU (at 1.5, 16384 x 768,
+        // the 64 x 64 grid is faster), 128 x 128 from one a CU where k is
+        // long enough to pay for its ramp, 32 x 64 where 64 x 64 tiles would
+        // leave CUs without one.
+        const size_t cus = (size_t)ctx->num_cus;
+        const size_t tiles256 = rnn_div_up(m, 256) * rnn_div_up(n, 128) * count;
+        const size_t tiles64 = rnn_div_up(m, 64) * rnn_div_up(n, 64) * count;
+        if (m >= 256 && n >= 128 && tiles256 >= 2 * cus)
+            return launch_dma<Tile256>(ctx, g, (int)count, at, bt);
+        if (m >= 128 && n >= 128 && tiles128 >= cus && kchunk >= 1024)
+            return launch_dma<Tile128>(ctx, g, (int)count, at, bt);
+        if (tiles64 < cus) return launch_dma<Tile32>(ctx, g, (int)count, at, bt);
+        return launch_dma<Tile64>(ctx, g, (int)count, at, bt);
     }
     if (rs_out || rs_part) return rnn_fail(ctx, RNN_E_INVALID, "gemm: row sums need the DMA path");
     const bool big = m >= 128 && n >= 128 && tiles128 >= (size_t)ctx->num_cus;
@@ -908,10 +1048,11 @@ int rnn_ns_gemm_launch(rnn_ctx *ctx, const NsGemmProb *probs, int nprob, size_t 
         if (!attr) {
             attr = true;
             (void)hipFuncSetAttribute((const void *)ns_gemm_dma_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)NS_DMA_LDS);
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)NsTile::LDS_BYTES);
         }
-        hipLaunchKernelGGL(ns_gemm_dma_kernel, grid, dim3(512), NS_DMA_LDS, ctx->stream, probs,
-                           nprob, alpha, beta);
+        hipLaunchKernelGGL(ns_gemm_dma_kernel, grid, dim3(NsTile::THREADS), NsTile::LDS_BYTES,
+                           ctx->stream, probs, nprob, alpha, beta);
     } else if (vec)
         hipLaunchKernelGGL(ns_gemm_kernel<true>, grid, dim3(256), 0, ctx->stream, probs, nprob,
                            alpha, beta);

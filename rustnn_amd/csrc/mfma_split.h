@@ -1,0 +1,88 @@
+// fp32 products on the bf16 matrix cores.
+//
+// A float with 24 significant bits is the exact sum of three bf16 values of 8
+// bits each: its leading 8 bits, those of the remainder, and the rest (cut
+// off, not rounded, so that the largest float's leading part stays finite).
+// Of the nine part products of a x b the three smallest (mid lo, lo mid, lo
+// lo: below 2^-23 of the product) are left out; the other six are exact in
+// the matrix core and summed in its fp32 accumulator, sixteen k values and
+// two roundings an instruction where v_mfma_f32_32x32x2f32 takes two.
+//
+// Measured on MI355X.  Rate: the bf16 pipe sustains 1.79 PFLOP/s from
+// registers, six products 298 TFLOP/s of fp32 work against the fp32 pipe's
+// 154; with the splitting of both operands in the same wave 200-220.  Error
+// against f64 over random normal operands (fp32 pipe / split): K = 16 8.0e-8
+// / 7.0e-8, K = 256 3.1e-7 / 2.4e-7, K = 4096 1.20e-6 / 1.11e-6, the same for
+// operands scaled down to 1e-33.  The sum inside one instruction is cut off
+// toward -inf, which leaves a mean error of -1.4e-8 (K = 256) to -5e-8 (K =
+// 1024) of the result's size where the fp32 pipe has none above 3e-9: it adds
+// up where many results are summed (a bias gradient over 8192 rows was 4
+// times further off).  So a kernel lets half of its k steps accumulate the
+// negated product: the mean goes below 2e-9, and the K = 256 error to 1.8e-7.
+// Below 2^-110 (8e-34) the lowest part of a
+// value is denormal and reads as zero: an absolute error under 2^-126.
+#pragma once
+
+#include "rnn_internal.h"
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// The parts of 8 floats, as operands of v_mfma_f32_32x32x16_bf16.
+struct Bf3 {
+    u32x4 hi, mid, lo;
+};
+
+// Two floats' leading 16 bits in one register.
+__device__ __forceinline__ uint32_t bf3_top2(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float bf3_rest(float a) {
+    return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+}
+
+__device__ __forceinline__ Bf3 bf3_split(const float (&x)[8]) {
+    Bf3 p;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float a = x[2 * j], b = x[2 * j + 1];
+        p.hi[j] = bf3_top2(a, b);
+        const float ra = bf3_rest(a), rb = bf3_rest(b);
+        p.mid[j] = bf3_top2(ra, rb);
+        p.lo[j] = bf3_top2(bf3_rest(ra), bf3_rest(rb));
+    }
+    return p;
+}
+
+__device__ __forceinline__ f32x16 bf3_mfma1(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// acc[i][j] += a[i] b[j] over 16 k values, the smallest part products first.
+template <int TM, int TN>
+__device__ __forceinline__ void bf3_mfma(const Bf3 *a, const Bf3 *b, f32x16 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const u32x4 u = q == 0 || q == 4 ? a[i].mid : q == 2 ? a[i].lo : a[i].hi;
+                const u32x4 w = q == 0 || q == 3 ? b[j].mid : q == 1 ? b[j].lo : b[j].hi;
+                acc[i][j] = bf3_mfma1(u, w, acc[i][j]);
+            }
+}
+
+template <int TM, int TN>
+__device__ __forceinline__ void bf3_negate(f32x16 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = -acc[i][j];
+}
+
+// Whether a value is an infinity or a NaN.
+__device__ __forceinline__ bool bf3_nonfinite(float c) {
+    return __builtin_amdgcn_classf(c, 0x207);
+}

@@ -250,3 +250,40 @@ def test_destroy_flushes_deferred_reductions(rnn, orc):
     assert np.array_equal(got[0][0], got[1][0])
     assert np.array_equal(got[0][1], got[1][1])
     assert got[1][1].any()
+
+
+# The direct-to-LDS tiles at their edges: a quad past the last whole tile, one
+# short of it, the shortest k, k off a stage; 32 x 64, 64 x 64, 128 x 128 and
+# 256 x 128 tiles by size.
+@pytest.mark.parametrize("m,n,k", [(4, 4, 4), (36, 68, 12), (516, 2052, 132), (2044, 2180, 1028),
+                                   (16388, 1028, 36)])
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+def test_matmul_split_tiles(rnn, m, n, k, at, bt):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn((k, m) if at else (m, k), generator=g, device="cuda")
+    b = torch.randn((n, k) if bt else (k, n), generator=g, device="cuda")
+    c = torch.full((m, n), 7.0, device="cuda")
+    rnn.matmul(m, n, k, a, at, b, bt, c)
+    want = (a.T if at else a).double() @ (b.T if bt else b).double()
+    # k sums of rounded products, each rounding 2^-24 of a partial sum: as a
+    # random walk 2^-24 sqrt(k) of the result, with 2^-23 for the part
+    # products left out
+    assert rel_frob(to_host(c), to_host(want)) < 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 64, 64), (512, 2048, 256), (2048, 2176, 1024),
+                                   (16384, 1024, 32)])
+def test_matmul_split_special_values(rnn, m, n, k):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randint(-3, 4, (m, k), generator=g, device="cuda").float()
+    b = torch.randint(-3, 4, (k, n), generator=g, device="cuda").float()
+    a[5, 3], a[17, 1], b[2, 9] = float("inf"), float("nan"), float("-inf")
+    a[40], a[40, 7], b[7] = 0.0, torch.finfo(torch.float32).max, 1.0
+    c = torch.empty((m, n), device="cuda")
+    rnn.matmul(m, n, k, a, False, b, False, c)
+    # infinities and NaN land where IEEE products and sums put them, finite
+    # integer results are exact, the largest float comes through whole
+    want = (a.double() @ b.double()).float()
+    assert np.array_equal(to_host(c), to_host(want), equal_nan=True)
