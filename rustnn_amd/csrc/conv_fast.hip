@@ -3,27 +3,34 @@
 //
 // Persistent workgroups walk a list of work items -- (tile of output
 // positions, group of MB blocks of 32 output channels) -- and, per item, the
-// source channels in chunks of CH.  Each (item, chunk) stage is staged into
-// one of two LDS buffers by DMA (buffer_load ... lds, no registers) while the
-// previous stage is computed:
-//   * the zero-padded source window (x for forward, dY for dX), stored
-//     [channel quad][position][4]: the 4 channels of a quad are adjacent, so
-//     one ds_read_b128 gives a lane the B operand of 4 MFMA k-steps;
-//   * the weight slab, gathered straight from W into MFMA fragment order
-//     [mb][quad][tap][lane][4] (one ds_read_b128 per 4 k-steps for A).
-// MFMA mapping (v_mfma_f32_32x32x2f32): M = output channels, N = output
-// positions (32 per group), K = (channel, tap) with lane half h carrying
-// channel h*CH/2 + 4q + i, so one per-tap offset serves all 64 lanes.  The
-// operands of the next (quad, tap) step are read while the MFMAs of the
-// current one run.
+// source channels in chunks of CH.  Producer waves stage each (item, chunk)
+// into one of two LDS buffers -- the zero-padded source window (x for
+// forward, dY for dX) and the chunk's weights -- while the compute waves
+// multiply the previous one; M = output channels, N = output positions (32
+// per group), K = (channel, tap):
+//   * 3x3: on the bf16 matrix cores, each float in three exact parts
+//     (mfma_split.h); the producers load through registers and split;
+//   * 1x1 (bound by memory): v_mfma_f32_32x32x2f32; the producers DMA
+//     (buffer_load ... lds) the window as [channel quad][position][4] and the
+//     weights in fragment order [mb][quad][tap][lane][4], one ds_read_b128
+//     per 4 k-steps, lane half h carrying channel h*CH/2 + 4q + i.
 //
 // For dX with stride s the workgroup computes all s*s parity classes of its
 // block positions from the same dY window, each tap feeding exactly one class
 // accumulator (gather-form col2im: no atomics, every dX element written once).
 //
+// 3x3 at batch 128, packed weights, fp32 pipe -> here (us, forward / dX):
+// 32 -> 32 @32x32 29.8 / 28.4 -> 23.4 / 22.9; 64 -> 64 @16x16 28.3 / 28.0 ->
+// 20.3 / 20.5; 128 -> 128 @8x8 28.4 / 28.5 -> 23.6 / 23.3; 96 -> 96 @16x16
+// 69.1 / 68.9 -> 37.5 / 37.7; stride 2 64 -> 128 @16x16 18.7 / 29.6 -> 20.4 /
+// 26.3.  Without loads and splitting 17-21 us are left of the stride-1 ones:
+// the ramp, LDS reads and MFMAs.  Errors against 64 bits 2-3 times smaller
+// (32 -> 32 2.1e-7 / 3.0e-7 -> 0.9e-7 / 1.1e-7).
+//
 // Reference: conv.rs forward_image (168-203), dx_image (205-246) and the
 // Conv2d batch drivers (nn.rs:166-250).
 #include "conv_common.h"
+#include "mfma_split.h"
 
 #include <algorithm>
 #include <cstdio>
@@ -54,17 +61,20 @@ struct FastArgs {
     int CD, HD, WD;
     int GA, GB;        // output block grid per image
     int TR, tiles_a, ntiles, ngroups;
-    int CH, nchunks;   // source channels per stage (multiple of 8)
+    int CH, nchunks;   // source channels per stage (multiple of 8; 3x3: 8)
     int sm, sc;        // weight strides of output row m and source channel ch
     int wbytes;        // bytes of W
     int dymin, dxmin;  // smallest tap offsets (window origin)
     int lrow, lcol;    // window rows / columns per output row / column step
-    int plane;         // window positions per channel quad (multiple of 64)
-    int ppw;           // plane / 64: window rows per quad and wave
-    int xwords;        // LDS words of the window: CH * plane
+    int plane;         // window positions (multiple of 64) per channel quad or bf16 part
+    int ppw;           // plane / 64: window rows per quad and wave, or 64-position groups
+    int xwords;        // LDS words of the window: CH * plane (3x3: 3 parts of 8 bf16: 12 * plane)
     int stage;         // LDS words of one stage: window, then weight slabs
     TileGeo geo;       // window geometry in positions (chs unused)
     int tapoff[9];     // window-position offset of each tap
+    // 3x3: the two taps of each k step (one per lane half; -1 none) and their
+    // window-position offsets
+    int ptap[10], poff[10];
     uint32_t m_imgs, m_tiwp;  // FastDiv multipliers of geo.imgs and geo.TIWP
     int npart;         // store-pass statistics: partials per channel (= ntiles)
     ConvStats stats;   // store-pass statistics (forward with EPI = 1)
@@ -167,6 +177,273 @@ __device__ __forceinline__ void item_rows(const FastArgs &g, const StageDMA &d, 
         const int ty = L.tmeta[u] & 255, img = L.tmeta[u] >> 8;
         const bool rowok = (unsigned)(ty - d.ylo) < (unsigned)(d.yhi - d.ylo) && img < d.nimg;
         L.roff[u] = rowok ? (uint32_t)(L.toff[u] + d.ebase) * 4u : 0x80000000u;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// 3x3 convolutions: products on the bf16 matrix cores (mfma_split.h).  A stage
+// is 8 source channels; a k step of 16 is those 8 channels under two taps of
+// one parity class, one tap per lane half (nine taps: the tenth half step
+// meets zero weights).  The producers load the window and the weights into
+// registers, split each float into its three bf16 parts and store the parts
+// in operand order -- window [part][position][8 channels], weights [mb][tap
+// pair][part][lane][8 channels] -- so that the compute waves only read
+// operands (one ds_read_b128 each) and multiply, and a value is split once
+// and not once per tap.
+template <int S, int P, bool DX>
+struct ConvPairs {
+    using T = ConvTaps<3, S, P, DX>;
+    static constexpr int N = 5;
+    int t[2 * N] = {}, cls[N] = {};
+    constexpr ConvPairs() {
+        int n = 0;
+        for (int c = 0; c < T::NCLS; c++) {
+            int k = 0;
+            for (int i = 0; i < 9; i++)
+                if (T::cls(i) == c) {
+                    if (k % 2 == 0) {
+                        cls[n] = c;
+                        t[2 * n] = i;
+                        t[2 * n + 1] = -1;
+                        n++;
+                    } else {
+                        t[2 * n - 1] = i;
+                    }
+                    k++;
+                }
+        }
+    }
+};
+
+// s_waitcnt lgkmcnt(0) / vmcnt(0) alone, and a barrier that waits for this
+// wave's LDS accesses only (loads into registers stay in flight across it).
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    wait_lds();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+constexpr int SPLIT_U = 3;  // 64-position window groups per producer wave
+
+// A producer wave's share of a stage: window groups dw, dw + 4, .. and weight
+// tasks (mb, tap pair), dealt from the wave after the last window group.
+template <int SL, int U, bool PK>
+struct SplitStage {
+    static constexpr int TW = (5 * SL + FAST_NW - 1) / FAST_NW;
+    int toff[U], tmeta[U];  // as LaneDMA's, for channel 0
+    uint32_t roff[U];       // byte offset for the work item, >= 2^31: none
+    uint32_t woff[TW];      // byte offset of weight task u at chunk 0
+    // Two stages in flight.  Every load is issued, past the end with an offset
+    // out of range, so that the wait for one stage leaves the next in flight.
+    float v[2][U][8], wv[2][TW][8];
+
+    __device__ __forceinline__ static int wtask(const FastArgs &g, int u, int dw) {
+        return ((dw - g.ppw) & (FAST_NW - 1)) + FAST_NW * u;
+    }
+
+    __device__ __forceinline__ void init(const FastArgs &g, int dw, int lane) {
+        const TileGeo &t = g.geo;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int pos = (dw + FAST_NW * u) * 64 + lane;
+            const uint32_t mi = g.m_imgs, mt = g.m_tiwp;
+            const int img = (int)(mi ? __umulhi((uint32_t)pos, mi) : (uint32_t)pos);
+            const int rem = pos - img * t.imgs;
+            const int ty = (int)(mt ? __umulhi((uint32_t)rem, mt) : (uint32_t)rem);
+            const int col = rem - ty * t.TIWP;
+            const int tx = t.deint ? (col < t.HALF ? 2 * col : 2 * (col - t.HALF) + 1) : col;
+            const int x = g.dxmin + tx * t.colstep;
+            const bool ok = pos < g.plane && img < t.IMGS && ty < t.TIH && tx < t.TIW && x >= 0 &&
+                            x < g.WS;
+            toff[u] = (img * g.CS * g.HS + ty * t.rowstep) * g.WS + x;
+            tmeta[u] = ok ? (ty | (img << 8)) : 255;
+        }
+    }
+
+    __device__ __forceinline__ void item(const FastArgs &g, const StageDMA &d, int dw, int lane) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int ty = tmeta[u] & 255, img = tmeta[u] >> 8;
+            const bool ok = (unsigned)(ty - d.ylo) < (unsigned)(d.yhi - d.ylo) && img < d.nimg;
+            roff[u] = ok ? (uint32_t)(toff[u] + d.ebase) * 4u : 0x80000000u;
+        }
+#pragma unroll
+        for (int u = 0; u < TW; u++) {
+            const int t = wtask(g, u, dw), mb = t / 5, pair = t - 5 * mb;
+            const int blk = d.grp * SL + mb, m = blk * 32 + (lane & 31);
+            if (t >= 5 * SL) {
+                woff[u] = DMA_OOB;
+            } else if (PK) {
+                woff[u] = (uint32_t)(blk * g.nchunks * 2560 + pair * 512 + lane * 8) * 4u;
+            } else {
+                const int tap = lane < 32 ? g.ptap[2 * pair] : g.ptap[2 * pair + 1];
+                woff[u] = tap >= 0 && m < g.CD ? (uint32_t)(m * g.sm + tap) * 4u : DMA_OOB;
+            }
+        }
+    }
+
+    // Loads the share of the item's `chunk` into register set B.
+    template <int B>
+    __device__ __forceinline__ void load(const FastArgs &g, const StageDMA &d, int chunk,
+                                         __amdgpu_buffer_rsrc_t rs_w) {
+        const uint32_t hsws4 = (uint32_t)(g.HS * g.WS) * 4u;
+        const int c0 = chunk * 8;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const bool live = c0 + c < g.CS;
+            const uint32_t so = live ? (uint32_t)(c0 + c) * hsws4 : 0u;
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                v[B][u][c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    d.rs, live ? roff[u] : 0x80000000u, so, 0));
+            if constexpr (!PK) {
+                const uint32_t sw = live ? (uint32_t)((c0 + c) * g.sc) * 4u : 0u;
+#pragma unroll
+                for (int u = 0; u < TW; u++)
+                    wv[B][u][c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        rs_w, live ? woff[u] : DMA_OOB, sw, 0));
+            }
+        }
+        if constexpr (PK) {
+            const uint32_t so = (uint32_t)chunk * 10240u;
+#pragma unroll
+            for (int u = 0; u < TW; u++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const u32x4 a =
+                        __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff[u] + 16 * q, so, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) wv[B][u][4 * q + i] = __uint_as_float(a[i]);
+                }
+        }
+    }
+
+    // Splits register set B into the stage buffer.
+    template <int B>
+    __device__ __forceinline__ void store(const FastArgs &g, float *buf, int dw, int lane) const {
+        u32x4 *x = reinterpret_cast<u32x4 *>(buf), *w = reinterpret_cast<u32x4 *>(buf + g.xwords);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (dw + FAST_NW * u < g.ppw) {
+                const Bf3 p = bf3_split(v[B][u]);
+                u32x4 *q = x + (dw + FAST_NW * u) * 64 + lane;
+                q[0] = p.hi;
+                q[g.plane] = p.mid;
+                q[2 * g.plane] = p.lo;
+                __builtin_amdgcn_sched_barrier(0);  // one group's parts live at a time
+            }
+#pragma unroll
+        for (int u = 0; u < TW; u++) {
+            const int t = wtask(g, u, dw);
+            if (t < 5 * SL) {
+                const Bf3 p = bf3_split(wv[B][u]);
+                u32x4 *q = w + t * 192 + lane;
+                q[0] = p.hi;
+                q[64] = p.mid;
+                q[128] = p.lo;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+};
+
+// A stage on the compute waves: vb the lane's window position of each
+// 32-position group, po the offset of each pair's tap in its lane half.
+template <int S, int P, bool DX, int NPW, int MB, int WM>
+__device__ __forceinline__ void compute_split(
+    const FastArgs &g, const float *__restrict__ buf, const int (&vb)[NPW], const int (&po)[5],
+    f32x16 (&acc)[ConvTaps<3, S, P, DX>::NCLS][MB][NPW][2], int wave, int lane) {
+    constexpr ConvPairs<S, P, DX> CP;
+    constexpr int WP = FAST_NW / WM;
+    const u32x4 *xs = reinterpret_cast<const u32x4 *>(buf);
+    const u32x4 *ws = reinterpret_cast<const u32x4 *>(buf + g.xwords) + wave / WP * MB * 960 + lane;
+    Bf3 a[MB], b[NPW];
+    auto fetch = [&](int i, Bf3 (&fa)[MB], Bf3 (&fb)[NPW]) {
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            const u32x4 *q = ws + (mb * 5 + i) * 192;
+            fa[mb] = Bf3{q[0], q[64], q[128]};
+        }
+#pragma unroll
+        for (int j = 0; j < NPW; j++) {
+            const u32x4 *q = xs + vb[j] + po[i];
+            fb[j] = Bf3{q[0], q[g.plane], q[2 * g.plane]};
+        }
+    };
+    // With one block a wave there are registers to read the next pair while
+    // this one is multiplied; with more, the MFMAs of a pair outlast the reads.
+    constexpr bool AHEAD = NPW * MB == 1;
+    if constexpr (AHEAD) fetch(0, a, b);
+    static_for<0, 5>([&](auto pc) {
+        constexpr int i = decltype(pc)::value, c = CP.cls[i];
+        Bf3 na[MB], nb[NPW];
+        if constexpr (!AHEAD)
+            fetch(i, a, b);
+        else if constexpr (i + 1 < 5)
+            fetch(i + 1, na, nb);
+        if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+        bf3_products([&](auto pick, auto kind) {
+            constexpr int A = decltype(kind)::value;
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                for (int j = 0; j < NPW; j++)
+                    acc[c][mb][j][A] = pick(a[mb], b[j], acc[c][mb][j][A]);
+        });
+        if constexpr (AHEAD && i + 1 < 5) {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) a[mb] = na[mb];
+#pragma unroll
+            for (int j = 0; j < NPW; j++) b[j] = nb[j];
+        }
+    });
+}
+
+// The item's sums with fp32 MFMAs from global memory: for values that are not
+// finite in the split (see bf3_nonfinite).
+template <int S, int P, bool DX, int NPW, int MB, int WM>
+__device__ __forceinline__ void compute_slow(
+    const FastArgs &g, f32x16 (&acc)[ConvTaps<3, S, P, DX>::NCLS][MB][NPW][2], int wave, int lane,
+    int grp, int a0, int n0) {
+    using T = ConvTaps<3, S, P, DX>;
+    constexpr int WP = FAST_NW / WM, SL = WM * MB;
+    const int h = lane >> 5, l32 = lane & 31, tpix = g.TR * g.GB;
+#pragma unroll
+    for (int j = 0; j < NPW; j++) {
+        const int p = ((wave % WP) * NPW + j) * 32 + l32;
+        const int img = p / tpix, rem = p - img * tpix, r = rem / g.GB, cb = rem - r * g.GB;
+        const int n = n0 + img, a = a0 + r;
+        const bool live = p < g.geo.IMGS * tpix && n < g.N && a < g.GA;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            const int m = (grp * SL + (wave / WP) * MB + mb) * 32 + l32;
+#pragma unroll
+            for (int c = 0; c < T::NCLS; c++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[c][mb][j][0][v] = 0.f;
+#pragma unroll
+            for (int c = 0; c < T::NCLS; c++)
+#pragma unroll 1
+                for (int t = 0; t < 9; t++) {
+                    if (T::cls(t) != c) continue;
+                    const int sy = a * T::IS + T::dy(t), sx = cb * T::IS + T::dx(t);
+                    const bool in = live && sy >= 0 && sy < g.HS && sx >= 0 && sx < g.WS;
+                    const float *xp = g.src + (((long long)n * g.CS + h) * g.HS + sy) * g.WS + sx;
+                    const float *wp = g.w + (long long)m * g.sm + (long long)h * g.sc + t;
+#pragma unroll 1
+                    for (int k = h; k < g.CS + h; k += 2) {
+                        const float b = in && k < g.CS ? *xp : 0.f;
+                        const float wt = m < g.CD && k < g.CS ? *wp : 0.f;
+                        acc[c][mb][j][0] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(wt, b, acc[c][mb][j][0], 0, 0, 0);
+                        xp += 2ll * g.HS * g.WS;
+                        wp += 2ll * g.sc;
+                    }
+                }
+        }
     }
 }
 
@@ -310,7 +587,7 @@ __device__ __forceinline__ void store_stats(
 #pragma unroll
             for (int mb = 0; mb < MB; mb++) {
                 f32x16 v16 = acc[0][mb][j][0];
-                if constexpr (NACC == 2) v16 += acc[0][mb][j][1];
+                if constexpr (K == 1 && NACC == 2) v16 += acc[0][mb][j][1];
                 static_for<0, VG>([&](auto uc) {
                     constexpr int u = decltype(uc)::value, v = vbase + u;
                     const int m = (grp * SL + (wave / WP) * MB + mb) * 32 + 8 * (v >> 2) + 4 * h +
@@ -347,14 +624,16 @@ __device__ __forceinline__ void store_stats(
 // EPI = 1: the forward's store pass also takes the batch statistics
 // (store_stats, ConvStats), with one more barrier per work item that the
 // producers match.
-template <int K, int S, int P, bool DX, int NPW, int MB, int WM, int EPI>
+// 3x3 only: U window groups per producer wave, PK packed weights.
+template <int K, int S, int P, bool DX, int NPW, int MB, int WM, int EPI, int U, bool PK>
 __global__ __launch_bounds__(64 * FAST_NW * 2)
-__attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs g) {
+__attribute__((amdgpu_waves_per_eu(EPI || (K == 3 && !(DX && S == 2)) ? 4 : 1))) void conv_fast_kernel(FastArgs g) {
     using T = ConvTaps<K, S, P, DX>;
     constexpr int NCLS = T::NCLS;
-    // A wave with a single output block alternates two accumulators so that
-    // consecutive MFMAs do not depend on each other.
-    constexpr int NACC = NCLS * NPW * MB == 1 ? 2 : 1;
+    // 1x1: a wave with a single output block alternates two accumulators so
+    // that consecutive MFMAs do not depend on each other.  3x3: the products
+    // of leading parts in one, the smaller ones in the other.
+    constexpr int NACC = K == 3 || NCLS * NPW * MB == 1 ? 2 : 1;
     constexpr int WP = FAST_NW / WM, SL = WM * MB;
     extern __shared__ float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
@@ -367,6 +646,48 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
     if (wave >= FAST_NW) {
         // producer
         const int dw = wave - FAST_NW;
+        if constexpr (K == 3) {
+            const __amdgpu_buffer_rsrc_t rs_w =
+                make_rsrc(PK ? g.wp : g.w, (uint32_t)(PK ? g.wpbytes : g.wbytes));
+            SplitStage<SL, U, PK> L;
+            L.init(g, dw, lane);
+            // the cursor of the next stage to load; it stays on the last one
+            int item = blockIdx.x, chunk = 0;
+            StageDMA d = stage_dma<K, S, P, DX, SL>(g, item, 0, smem);
+            L.item(g, d, dw, lane);
+            auto next = [&]() {
+                if (chunk + 1 < g.nchunks) {
+                    chunk++;
+                } else if (item + (int)gridDim.x < nitems) {
+                    item += gridDim.x;
+                    chunk = 0;
+                    d = stage_dma<K, S, P, DX, SL>(g, item, 0, smem);
+                    L.item(g, d, dw, lane);
+                }
+            };
+            const int nst = (nitems - 1 - (int)blockIdx.x) / (int)gridDim.x * g.nchunks + g.nchunks;
+            L.template load<0>(g, d, 0, rs_w);
+            next();
+            L.template load<1>(g, d, chunk, rs_w);
+            int sc = 0;  // the stored stage's chunk
+            auto stage = [&](auto bc) {
+                constexpr int B = decltype(bc)::value;
+                // buffer B: every wave is past the stage before last
+                L.template store<B>(g, smem + B * g.stage, dw, lane);
+                next();
+                L.template load<B>(g, d, chunk, rs_w);
+                lds_barrier();
+                if (++sc == g.nchunks) {
+                    sc = 0;
+                    if constexpr (EPI != 0) lds_barrier();  // the compute waves' store-pass sums
+                }
+            };
+            for (int s = 0; s < nst; s += 2) {
+                stage(std::integral_constant<int, 0>{});
+                if (s + 1 < nst) stage(std::integral_constant<int, 1>{});
+            }
+            return;
+        } else {
         const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(g.w, (uint32_t)g.wbytes);
         LaneDMA<T::KK> L;
         lane_dma_init<T::KK>(g, L, dw, lane);
@@ -389,18 +710,25 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
             if constexpr (EPI != 0) __syncthreads();  // the compute waves' store-pass sums
         }
         return;
+        }
     }
 
     // LDS word offset of this lane's channel half and window position for
-    // each 32-position group (tile-relative: the same for every work item).
+    // each 32-position group (tile-relative: the same for every work item);
+    // 3x3: the window position alone.
     int vb[NPW];
 #pragma unroll
     for (int j = 0; j < NPW; j++) {
         int p = ((wave % WP) * NPW + j) * 32 + l32;
         if (p >= npix) p = 0;
         const int img = p / tpix, rem = p - img * tpix, r = rem / g.GB, c = rem - r * g.GB;
-        vb[j] = (h * CQ * g.plane + img * g.geo.imgs + r * g.lrow * g.geo.TIWP + c * g.lcol) * 4;
+        const int pos = img * g.geo.imgs + r * g.lrow * g.geo.TIWP + c * g.lcol;
+        vb[j] = K == 3 ? pos : (h * CQ * g.plane + pos) * 4;
     }
+    int po[5];
+    if constexpr (K == 3)
+#pragma unroll
+        for (int i = 0; i < 5; i++) po[i] = h ? g.poff[2 * i + 1] : g.poff[2 * i];
 
     f32x16 acc[NCLS][MB][NPW][NACC];
     int s = 0;
@@ -418,13 +746,35 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
         for (int chunk = 0; chunk < g.nchunks; chunk++, s++) {
             // Stage s has landed and every wave is done with stage s-1, whose
             // buffer the producers fill with stage s+1 while stage s is computed.
+            if constexpr (K == 3) {
+                lds_barrier();
+                compute_split<S, P, DX, NPW, MB, WM>(g, smem + (s & 1) * g.stage, vb, po, acc,
+                                                     wave, lane);
+                continue;
+            } else {
             dma_wait_barrier();
             compute_stage<K, S, P, DX, NPW, MB, WM, NACC>(g, smem + (s & 1) * g.stage, vb, acc,
                                                           wave, lane);
+            }
         }
         // acc row 8*(v/4) + 4*h + v%4 = output channel in the block, column = position.
         const int tile = item % g.ntiles, grp = item / g.ntiles;
         const int a0 = (tile % g.tiles_a) * g.TR, n0 = (tile / g.tiles_a) * g.geo.IMGS;
+        if constexpr (K == 3) {
+            bool bad = false;
+#pragma unroll
+            for (int c = 0; c < NCLS; c++)
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                    for (int j = 0; j < NPW; j++) {
+                        acc[c][mb][j][0] += acc[c][mb][j][1];
+#pragma unroll
+                        for (int v = 0; v < 16; v++)
+                            bad = bad || bf3_nonfinite(acc[c][mb][j][0][v]);
+                    }
+            if (__any(bad)) compute_slow<S, P, DX, NPW, MB, WM>(g, acc, wave, lane, grp, a0, n0);
+        }
         if constexpr (EPI != 0) {
             // Store pass with the statistics' sums; then the WP position
             // waves' totals of each channel, summed in wave order, make partial
@@ -433,7 +783,10 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
             constexpr int NCH = 32 * SL;
             double *red = reinterpret_cast<double *>(smem + 2 * g.stage);
             store_stats<K, S, P, NPW, MB, WM, NACC>(g, acc, wave, lane, grp, a0, n0, red);
-            __syncthreads();
+            if constexpr (K == 3)
+                lds_barrier();
+            else
+                __syncthreads();
             for (int t = tid; t < 2 * NCH; t += 64 * FAST_NW) {
                 const int cl = t >> 1, m = grp * NCH + cl;
                 if (m >= g.CD) continue;
@@ -463,7 +816,7 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
 #pragma unroll
                     for (int mb = 0; mb < MB; mb++) {
                         f32x16 v0 = acc[2 * py][mb][j][0], v1 = acc[2 * py + 1][mb][j][0];
-                        if constexpr (NACC == 2) {
+                        if constexpr (K == 1 && NACC == 2) {
                             v0 += acc[2 * py][mb][j][1];
                             v1 += acc[2 * py + 1][mb][j][1];
                         }
@@ -489,7 +842,7 @@ __attribute__((amdgpu_waves_per_eu(EPI ? 4 : 1))) void conv_fast_kernel(FastArgs
 #pragma unroll
                     for (int mb = 0; mb < MB; mb++) {
                         f32x16 v16 = acc[c][mb][j][0];
-                        if constexpr (NACC == 2) v16 += acc[c][mb][j][1];
+                        if constexpr (K == 1 && NACC == 2) v16 += acc[c][mb][j][1];
 #pragma unroll
                         for (int v = 0; v < 16; v++) {
                             const int m = (grp * SL + (wave / WP) * MB + mb) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
@@ -536,9 +889,10 @@ static size_t plan_geometry(const FastPlan &p, int GB, FastArgs &a) {
     t.imgs = t.TIH * t.TIWP;
     t.chs = 0;
     tilegeo_finish(t);
-    a.plane = (p.IMGS * t.imgs + 16 * FAST_NW - 1) / (16 * FAST_NW) * (16 * FAST_NW);
-    a.ppw = a.plane / (16 * FAST_NW);
-    if (a.ppw > WinRows<T::KK>::MAX || t.TIH > 254 || p.IMGS > 255) return 0;
+    a.plane = (p.IMGS * t.imgs + 63) / 64 * 64;
+    a.ppw = a.plane / 64;
+    if (a.ppw > (K == 3 ? SPLIT_U * FAST_NW : WinRows<T::KK>::MAX) || t.TIH > 254 || p.IMGS > 255)
+        return 0;
     a.dymin = dymin;
     a.dxmin = dxmin;
     for (int i = 0; i < 9; i++) {
@@ -550,8 +904,18 @@ static size_t plan_geometry(const FastPlan &p, int GB, FastArgs &a) {
     }
     a.m_imgs = t.fd_imgstr.m;
     a.m_tiwp = t.fd_tiwp.m;
-    a.xwords = p.CH * a.plane;
-    a.stage = a.xwords + p.WM * p.MB * p.CH * T::KK * 32;
+    if constexpr (K == 3) {
+        constexpr ConvPairs<S, P, DX> cp;
+        for (int i = 0; i < 10; i++) {
+            a.ptap[i] = cp.t[i];
+            a.poff[i] = a.tapoff[cp.t[i] >= 0 ? cp.t[i] : cp.t[i & ~1]];
+        }
+        a.xwords = 12 * a.plane;
+        a.stage = a.xwords + p.WM * p.MB * 5 * 3 * 256;
+    } else {
+        a.xwords = p.CH * a.plane;
+        a.stage = a.xwords + p.WM * p.MB * p.CH * T::KK * 32;
+    }
     return (size_t)2 * a.stage * 4;
 }
 
@@ -559,13 +923,13 @@ template <int K, int S, int P, bool DX>
 static bool plan_ok(FastPlan &p, int CS, int GA, int GB, FastArgs &a) {
     using T = ConvTaps<K, S, P, DX>;
     const int CSe = std::max(8, (CS + 7) & ~7);
-    p.CH = std::min(p.CH, std::min(32, CSe));
+    p.CH = K == 3 ? 8 : std::min(p.CH, std::min(32, CSe));
     p.TR = std::min(p.TR, GA);
     if (p.TR <= 0 || p.IMGS <= 0 || p.CH < 8 || p.CH % 8) return false;
     if (p.WM <= 0) p.WM = 1;
     const int nwm = p.NPW * 100 + p.MB * 10 + p.WM;
-    const bool shape_ok = T::NCLS == 1 ? (nwm == 211 || nwm == 111 || nwm == 121 || nwm == 112)
-                                       : (nwm == 111 || nwm == 112);
+    const bool shape_ok = nwm == 111 || (nwm == 211 && T::NCLS == 1 && !(K == 3 && T::IS == 2)) ||
+                          ((nwm == 112 || nwm == 212) && K == 3 && T::IS == 2);
     if (!shape_ok || p.IMGS * p.TR * GB > (FAST_NW / p.WM) * p.NPW * 32) return false;
     p.lds = plan_geometry<K, S, P, DX>(p, GB, a);
     return p.lds > 0 && p.lds <= 160 * 1024;
@@ -573,16 +937,17 @@ static bool plan_ok(FastPlan &p, int CS, int GA, int GB, FastArgs &a) {
 
 // Tile choice.  RNN_CONV_PLAN="TR,IMGS,CH,NPW,MB[,WM[,WPC]]" overrides
 // (tuning sweeps).  Otherwise rules fitted to measured sweeps on MI355X:
-// channel chunks of a quarter of the source channels (8..32; 32 for 1x1);
-// stride-1 3x3 and 1x1 forward take 256 positions in two 32-position groups
-// per wave when an image has 256 or more positions, else 128 positions (whole
-// images); strided 3x3 forward takes 64 positions with the waves split two
-// ways along output channels, so every wave has a 32x32 block.  A plan that
-// does not fit falls back to shrinking the tile; a strided 3x3 forward gives
-// up channels per chunk before positions (at 96 source channels, 24-channel
-// chunks with 32 positions ran at half the rate of 8-channel chunks with 64).
+// chunks of 8 channels (3x3) or 32 (1x1); stride-1 3x3 takes 256 positions in
+// two 32-position groups per wave where that leaves two items a CU (32 -> 32
+// @32x32, 512 items: 23.4 us), else 128 positions (64 -> 64 @16x16, 256 or 512
+// items: 23.5 / 20.3; 48 -> 80 @23x29, 37 images: 25.2 / 21.2; one 32x32 image
+// 13.9 / 9.5); 1x1 forward takes 256 positions when an image has as many;
+// strided 3x3 forward takes 64 positions with the waves split two ways along
+// output channels, so every wave has a 32x32 block.  A plan that does not fit
+// falls back to shrinking the tile.
 template <int K, int S, int P, bool DX>
-static bool choose_plan(int CS, int CD, int GA, int GB, FastPlan &best, FastArgs &a) {
+static bool choose_plan(int CS, int CD, int GA, int GB, size_t n, size_t cus, FastPlan &best,
+                        FastArgs &a) {
     using T = ConvTaps<K, S, P, DX>;
     if (const char *env = getenv("RNN_CONV_PLAN")) {
         FastPlan p{};
@@ -594,7 +959,7 @@ static bool choose_plan(int CS, int CD, int GA, int GB, FastPlan &best, FastArgs
         }
     }
     if (GB > 256) return false;
-    const int ch = T::KK == 1 ? 32 : std::max(8, std::min(32, (CS / 4 + 7) & ~7));
+    const int ch = T::KK == 1 ? 32 : 8;
     const bool strided = T::KK == 9 && T::IS == 2;
     FastPlan r{};
     r.CH = ch;
@@ -603,7 +968,8 @@ static bool choose_plan(int CS, int CD, int GA, int GB, FastPlan &best, FastArgs
     r.WM = 1;
     int npos = 128;
     if (T::KK == 9 && T::NCLS == 1 && T::IS == 1) {
-        if (GA * GB >= 256) {
+        const size_t tiles = n * (size_t)((GA + std::max(1, 256 / GB) - 1) / std::max(1, 256 / GB));
+        if (GA * GB >= 256 && tiles * ((CD + 31) / 32) >= 2 * cus) {
             r.NPW = 2;
             npos = 256;
         }
@@ -629,8 +995,6 @@ static bool choose_plan(int CS, int CD, int GA, int GB, FastPlan &best, FastArgs
         }
         if (r.IMGS > 1)
             r.IMGS /= 2;
-        else if (strided && r.CH > 8)
-            r.CH = std::max(8, (r.CH / 2) & ~7);
         else if (r.TR > 1)
             r.TR = (r.TR + 1) / 2;
         else if (r.CH > 8)
@@ -648,19 +1012,11 @@ static size_t epi_lds(const FastPlan &p) {
     return (size_t)(FAST_NW / p.WM) * 32 * p.WM * p.MB * 2 * sizeof(double);
 }
 
-template <int K, int S, int P, bool DX, int NPW, int MB, int WM>
-static void set_attr() {
-    (void)hipFuncSetAttribute((const void *)conv_fast_kernel<K, S, P, DX, NPW, MB, WM, 0>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if constexpr (!DX)
-        (void)hipFuncSetAttribute((const void *)conv_fast_kernel<K, S, P, DX, NPW, MB, WM, 1>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-}
 
 // Operand roles, geometry and tile plan of a (k, stride, pad) forward / dX
 // convolution; false when no plan fits.
 template <int K, int S, int P, bool DX>
-static bool setup(const rnn_conv_spec *sp, FastArgs &a, FastPlan &p) {
+static bool setup(const rnn_conv_spec *sp, size_t n, size_t cus, FastArgs &a, FastPlan &p) {
     using T = ConvTaps<K, S, P, DX>;
     std::memset(&a, 0, sizeof(a));
     const int cin = sp->cin, cout = sp->cout;
@@ -687,7 +1043,7 @@ static bool setup(const rnn_conv_spec *sp, FastArgs &a, FastPlan &p) {
         a.sm = T::KK;  // W^T: m = cin, ch = cout
         a.sc = cin * T::KK;
     }
-    if (!choose_plan<K, S, P, DX>(a.CS, a.CD, a.GA, a.GB, p, a)) return false;
+    if (!choose_plan<K, S, P, DX>(a.CS, a.CD, a.GA, a.GB, n, cus, p, a)) return false;
     if (getenv("RNN_CONV_DEBUG"))
         fprintf(stderr, "conv k%d s%d p%d %s %dx%d->%d: plan %d,%d,%d,%d,%d,%d lds %zu\n", K, S, P,
                 DX ? "dx" : "fwd", a.CS, a.GA, a.CD, p.TR, p.IMGS, p.CH, p.NPW, p.MB, p.WM, p.lds);
@@ -709,6 +1065,8 @@ static PackGeo pack_geo(const FastArgs &a) {
     pg.nmblk = (a.CD + 31) / 32;
     pg.sm = a.sm;
     pg.sc = a.sc;
+    pg.ptap = 0;
+    for (int i = 0; i < 10; i++) pg.ptap |= (uint64_t)(a.ptap[i] & 15) << 4 * i;
     return pg;
 }
 
@@ -716,19 +1074,9 @@ template <int K, int S, int P, bool DX>
 static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src, const float *w,
                   const float *wp, float *dst, const ConvStats *cs) {
     using T = ConvTaps<K, S, P, DX>;
-    static bool attr = false;
-    if (!attr) {
-        attr = true;
-        set_attr<K, S, P, DX, 1, 1, 1>();
-        set_attr<K, S, P, DX, 1, 1, 2>();
-        if constexpr (T::NCLS == 1) {
-            set_attr<K, S, P, DX, 2, 1, 1>();
-            set_attr<K, S, P, DX, 1, 2, 1>();
-        }
-    }
     FastArgs a;
     FastPlan p;
-    if (!setup<K, S, P, DX>(sp, a, p))
+    if (!setup<K, S, P, DX>(sp, (size_t)n, (size_t)ctx->num_cus, a, p))
         return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: no LDS tiling for a %dx%d grid", a.GA, a.GB);
     a.src = src;
     a.w = w;
@@ -759,6 +1107,8 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
     }
     // Persistent grid: as many workgroups as fit on the chip at once.
     auto run = [&](auto kern) -> int {
+        (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  160 * 1024);
         int occ = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, 64 * FAST_NW * 2, p.lds) !=
                 hipSuccess ||
@@ -773,12 +1123,31 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
     };
     auto pick = [&](auto ec) -> int {
         constexpr int E = decltype(ec)::value;
-        if constexpr (T::NCLS == 1) {
-            if (p.NPW == 2) return run(conv_fast_kernel<K, S, P, DX, 2, 1, 1, E>);
-            if (p.MB == 2) return run(conv_fast_kernel<K, S, P, DX, 1, 2, 1, E>);
+        if constexpr (K == 3) {
+            auto split = [&](auto nc, auto mc) -> int {  // groups per wave, blocks of channels
+                constexpr int N = decltype(nc)::value, M = decltype(mc)::value;
+                const int u = (a.ppw + FAST_NW - 1) / FAST_NW;
+                if (wp)
+                    return u == 1   ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, true>)
+                           : u == 2 ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, true>)
+                                    : run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, true>);
+                return u == 1   ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, false>)
+                       : u == 2 ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, false>)
+                                : run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, false>);
+            };
+            using one = std::integral_constant<int, 1>;
+            using two = std::integral_constant<int, 2>;
+            if constexpr (T::IS == 2) {
+                if (p.WM == 2) return p.NPW == 2 ? split(two{}, two{}) : split(one{}, two{});
+            } else if constexpr (T::NCLS == 1) {
+                if (p.NPW == 2) return split(two{}, one{});
+            }
+            return split(one{}, one{});
+        } else {
+            if constexpr (T::NCLS == 1)
+                if (p.NPW == 2) return run(conv_fast_kernel<K, S, P, DX, 2, 1, 1, E, 1, false>);
+            return run(conv_fast_kernel<K, S, P, DX, 1, 1, 1, E, 1, false>);
         }
-        if (p.WM == 2) return run(conv_fast_kernel<K, S, P, DX, 1, 1, 2, E>);
-        return run(conv_fast_kernel<K, S, P, DX, 1, 1, 1, E>);
     };
     if constexpr (!DX)
         if (stats) return pick(std::integral_constant<int, 1>{});
@@ -786,10 +1155,10 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
 }
 
 template <int K, int S, int P>
-static int parts_of(const rnn_conv_spec *sp, size_t n) {
+static int parts_of(const rnn_ctx *ctx, const rnn_conv_spec *sp, size_t n) {
     FastArgs a;
     FastPlan p;
-    if (!setup<K, S, P, false>(sp, a, p)) return -1;
+    if (!setup<K, S, P, false>(sp, n, (size_t)ctx->num_cus, a, p)) return -1;
     if (p.lds + epi_lds(p) > 160 * 1024) return -1;
     const long long np = (long long)a.tiles_a * (((long long)n + p.IMGS - 1) / p.IMGS);
     return np > 0x3fffffffll ? -1 : (int)np;
@@ -831,7 +1200,8 @@ template <int K, int S, int P, bool DX>
 static int geo_of(const rnn_conv_spec *sp, PackGeo *pg) {
     FastArgs a;
     FastPlan p;
-    if (!setup<K, S, P, DX>(sp, a, p)) return RNN_E_UNSUPPORTED;
+    // (the packed layout does not depend on the batch: 3x3 plans share CH)
+    if (!setup<K, S, P, DX>(sp, 1, 1, a, p)) return RNN_E_UNSUPPORTED;
     *pg = pack_geo<K, S, P, DX>(a);
     return RNN_OK;
 }
@@ -859,11 +1229,11 @@ int rnn_conv_fast(rnn_ctx *ctx, int dx, const rnn_conv_spec *sp, size_t n, const
     return RNN_E_UNSUPPORTED;
 }
 
-int rnn_conv_fast_parts(const rnn_conv_spec *sp, size_t n) {
+int rnn_conv_fast_parts(const rnn_ctx *ctx, const rnn_conv_spec *sp, size_t n) {
     if (getenv("RNN_CONV_GENERIC") || n == 0 || n > 0x7fffffff) return -1;
     const int k = sp->k, s = sp->stride, p = sp->pad;
 #define RNN_CONV_CASE(K_, S_, P_) \
-    if (k == K_ && s == S_ && p == P_) return parts_of<K_, S_, P_>(sp, n);
+    if (k == K_ && s == S_ && p == P_) return parts_of<K_, S_, P_>(ctx, sp, n);
     RNN_CONV_CASE(3, 1, 1)
     RNN_CONV_CASE(3, 2, 1)
     RNN_CONV_CASE(1, 2, 0)

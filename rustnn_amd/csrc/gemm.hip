@@ -326,7 +326,8 @@ struct DmaOperand {
 // stage it has landed (each producer waited for its own DMAs) and every
 // compute wave is done with stage it - 1, whose buffer the producers then
 // refill with stage it + NS - 1.
-template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, bool AT, bool BT>
+template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, int NACC, bool AT,
+          bool BT>
 struct DmaTile {
     static constexpr int NC = WM * WN * WK;
     using OA = DmaOperand<BM, BK, !AT, NP>;
@@ -406,7 +407,7 @@ struct DmaTile {
             return false;
         }
         const int lr = lane & 31, lh = lane >> 5;
-        f32x16 sum[TM][TN];
+        f32x16 sum[TM][TN], part[TM][TN];  // NACC = 2: part takes the smaller part products
 #pragma unroll
         for (int i = 0; i < TM; i++) rs[i] = 0.0;
 #pragma unroll
@@ -414,17 +415,17 @@ struct DmaTile {
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) sum[i][j][v] = 0.f;
+                for (int v = 0; v < 16; v++) sum[i][j][v] = part[i][j][v] = 0.f;
         constexpr int NSTEP = BK / 16 / WK;
         const int s0 = wk() * NSTEP, ra0 = row0() + lr, rb0 = wn() * WTN + lr;
         // Odd shares multiply -A (subtracted in the exchange); a tile without
         // shares turns the sign of its sums every few stages: the matrix
         // core's rounding toward -inf cancels (mfma_split.h).
-        uint32_t neg = WK > 1 && (wk() & 1) ? 0x80000000u : 0u;
+        uint32_t neg = NACC == 1 && WK > 1 && (wk() & 1) ? 0x80000000u : 0u;
         const int flip = min(8, max(1, nk / 4));
         int turn = flip;
         for (int it = 0; it < nk; it++) {
-            if constexpr (WK == 1)
+            if constexpr (NACC == 1 && WK == 1)
                 if (turn-- == 0) {
                     turn = flip - 1;
                     neg ^= 0x80000000u;
@@ -445,17 +446,30 @@ struct DmaTile {
 #pragma unroll
                         for (int e = 0; e < 8; e++) rs[i] += (double)x[i][e];
                 }
+                if constexpr (NACC == 1)
 #pragma unroll
-                for (int i = 0; i < TM; i++)
+                    for (int i = 0; i < TM; i++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        x[i][e] = __uint_as_float(__float_as_uint(x[i][e]) ^ neg);
+                        for (int e = 0; e < 8; e++)
+                            x[i][e] = __uint_as_float(__float_as_uint(x[i][e]) ^ neg);
                 Bf3 p[TM + TN];
 #pragma unroll
                 for (int i = 0; i < TM + TN; i++) p[i] = bf3_split(x[i]);
-                bf3_mfma<TM, TN>(p, p + TM, sum);
+                bf3_products([&](auto pick, auto kind) {
+                    auto &t = NACC == 2 && decltype(kind)::value ? part : sum;
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++)
+                            t[i][j] = pick(p[i], p[TM + j], t[i][j]);
+                });
             }
         }
+        if constexpr (NACC == 2)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) sum[i][j] += part[i][j];
         if constexpr (WK > 1) {
             // The ring, free once every wave is past its last stage, takes
             // all partial sums; a wave adds its groups' over the shares (odd
@@ -483,7 +497,7 @@ struct DmaTile {
 #pragma unroll
                     for (int s = 1; s < WK; s++) {
                         const f32x4 u = x[((s * WM * WN + w0) * TM * TN * 4 + q) * 64 + lane];
-                        t = s & 1 ? t - u : t + u;
+                        t = NACC == 1 && (s & 1) ? t - u : t + u;
                     }
 #pragma unroll
                     for (int e = 0; e < 4; e++) acc[o][4 * e4 + e] = t[e];
@@ -557,19 +571,20 @@ struct DmaTile {
 // 8.6 / 9.9 / 21 / 36; 8192 x 768 x 256 34.6 -> 38 / 30.2 / 37 / 32; 8192 x
 // 256 x 768 32.1 -> 29 / 26.6 / 38 / 63; 16384 x 768 x 256 69.2 -> 78 / 56.4 /
 // 62 / 63; 2048^3 148 -> 148 / 113 / 103 / 156; 4096^3 1280 -> 1202 / 918 /
-// 818 / 766 (179 TFLOP/s).  The tiles with two or four shares of k also
-// shorten the accumulation chains (K = 256 error 2.05e-7 -> 1.76e-7).
+// 818 / 766 (179 TFLOP/s).  NACC: a second accumulator for the smaller part
+// products (mfma_split.h) where the registers allow it; on the 64 x 64 tile
+// it costs a workgroup a CU (8192 x 768 x 256 31.7 -> 32.5 us).
 template <bool AT, bool BT>
-using Tile32 = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, AT, BT>;
+using Tile32 = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, AT, BT>;
 template <bool AT, bool BT>
-using Tile64 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, AT, BT>;
+using Tile64 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, AT, BT>;
 template <bool AT, bool BT>
-using Tile128 = DmaTile<128, 128, 32, 3, 2, 2, 2, 4, AT, BT>;
+using Tile128 = DmaTile<128, 128, 32, 3, 2, 2, 2, 4, 1, AT, BT>;
 template <bool AT, bool BT>
-using Tile256 = DmaTile<256, 128, 16, 4, 4, 2, 1, 4, AT, BT>;
+using Tile256 = DmaTile<256, 128, 16, 4, 4, 2, 1, 4, 1, AT, BT>;
 // Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile.
 template <bool AT, bool BT>
-using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, AT, BT>;
+using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, AT, BT>;
 
 template <class Tile, bool RS>
 __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(GemmArgs g) {

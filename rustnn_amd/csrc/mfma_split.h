@@ -17,13 +17,17 @@
 // toward -inf, which leaves a mean error of -1.4e-8 (K = 256) to -5e-8 (K =
 // 1024) of the result's size where the fp32 pipe has none above 3e-9: it adds
 // up where many results are summed (a bias gradient over 8192 rows was 4
-// times further off).  So a kernel lets half of its k steps accumulate the
-// negated product: the mean goes below 2e-9, and the K = 256 error to 1.8e-7.
+// times further off).  Two ways out, both with a mean error below 2e-9: a
+// second accumulator for the five smaller products (K = 256 1.1e-7, K = 1024
+// 1.9e-7 against the fp32 pipe's 5.6e-7), or, where registers are short, half
+// of the k steps accumulating the negated product (K = 256 1.8e-7).
 // Below 2^-110 (8e-34) the lowest part of a
 // value is denormal and reads as zero: an absolute error under 2^-126.
 #pragma once
 
 #include "rnn_internal.h"
+
+#include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -59,19 +63,19 @@ __device__ __forceinline__ f32x16 bf3_mfma1(u32x4 a, u32x4 b, f32x16 c) {
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// acc[i][j] += a[i] b[j] over 16 k values, the smallest part products first.
-template <int TM, int TN>
-__device__ __forceinline__ void bf3_mfma(const Bf3 *a, const Bf3 *b, f32x16 (&acc)[TM][TN]) {
-#pragma unroll
-    for (int q = 0; q < 6; q++)
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const u32x4 u = q == 0 || q == 4 ? a[i].mid : q == 2 ? a[i].lo : a[i].hi;
-                const u32x4 w = q == 0 || q == 3 ? b[j].mid : q == 1 ? b[j].lo : b[j].hi;
-                acc[i][j] = bf3_mfma1(u, w, acc[i][j]);
-            }
+// Calls f(pick, small) for each of the six part products, smallest first;
+// pick(a, b, c) adds that product of two fragments to accumulator c; small is
+// 0 for the product of the leading parts, 1 for the others.
+template <typename F>
+__device__ __forceinline__ void bf3_products(F &&f) {
+    const std::integral_constant<int, 0> lead;
+    const std::integral_constant<int, 1> small;
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.mid, b.mid, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.lo, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.lo, b.hi, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.mid, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.mid, b.hi, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.hi, c); }, lead);
 }
 
 template <int TM, int TN>

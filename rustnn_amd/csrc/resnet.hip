@@ -290,7 +290,7 @@ int plan(rnn_resnet *r, size_t n, size_t H, size_t W) {
     auto ep = [&](NetConv &c, size_t hh, size_t ww) -> int {
         if (!r->fuse_bn) return -1;
         rnn_conv_spec sp = c.spec((uint32_t)hh, (uint32_t)ww);
-        return rnn_conv_fast_parts(&sp, n);
+        return rnn_conv_fast_parts(r->ctx, &sp, n);
     };
     r->stem.epf = ep(r->stem, H, W);
     for (auto &b : r->blocks) {

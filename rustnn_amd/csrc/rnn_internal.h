@@ -479,29 +479,41 @@ int rnn_conv_fast(rnn_ctx *ctx, int dx, const rnn_conv_spec *sp, size_t n, const
                   const float *w, const float *wp, float *dst, const ConvStats *stats = nullptr);
 // Partials per channel of the store-pass statistics of a forward of (sp, n);
 // -1 when the shape has no specialised plan.
-int rnn_conv_fast_parts(const rnn_conv_spec *sp, size_t n);
+int rnn_conv_fast_parts(const rnn_ctx *ctx, const rnn_conv_spec *sp, size_t n);
 
-// Packed weights of one direction: [m-block][chunk][quad][tap][lane 64][4]
-// with lane L of slab (quad q, tap t) holding rows m = 32*mblk + L%32 and
-// source channels c = chunk*CH + (L/32)*CH/2 + 4q + i of W[m*sm + c*sc + t],
-// zero beyond CD rows or CS channels.
+// Packed weights of one direction, W[m*sm + c*sc + t] in the order the kernel
+// stages it, zero beyond CD rows or CS channels.  1x1: [m-block][chunk][quad]
+// [lane 64][4], lane L of quad q holding row m = 32*mblk + L%32 and source
+// channels c = chunk*CH + (L/32)*CH/2 + 4q + i.  3x3: [m-block][chunk of 8]
+// [tap pair][lane 64][8], lane L holding row 32*mblk + L%32 and the chunk's
+// channels under tap ptap[2*pair + L/32].
 struct PackGeo {
     int CS, CD, KK, CH, nchunks, nmblk, sm, sc;
-    __host__ __device__ size_t floats() const {
-        return (size_t)nmblk * nchunks * CH * KK * 32;
-    }
-    // 256-float slabs: slab r = ((mblk*nchunks + chunk)*CH/8 + q)*KK + t
-    __host__ __device__ int slabs() const { return nmblk * nchunks * (CH >> 3) * KK; }
-    // word j = 4L + i of slab r
+    // 3x3: the taps of each pair's lane halves, a nibble each (15: zeros); one
+    // word, as an array indexed per lane would go through scratch memory
+    // (packing the ResNet-20 14 -> 50 us)
+    uint64_t ptap;
+    // 256-float slabs of an (m-block, chunk)
+    __host__ __device__ int per() const { return KK == 9 ? 10 : (CH >> 3) * KK; }
+    __host__ __device__ int slabs() const { return nmblk * nchunks * per(); }
+    __host__ __device__ size_t floats() const { return (size_t)slabs() * 256; }
+    // word j of slab r
     __device__ float value(const float *w, int r, int j) const {
-        const int cq = CH >> 3;
-        const int t = r % KK, rq = r / KK;
-        const int q = rq % cq, rc = rq / cq;
+        const int n = per(), q = r % n, rc = r / n;
         const int chunk = rc % nchunks, mblk = rc / nchunks;
-        const int i = j & 3, L = j >> 2;
-        const int m = mblk * 32 + (L & 31);
-        const int c = chunk * CH + (L >> 5) * (CH >> 1) + 4 * q + i;
-        return (m < CD && c < CS) ? w[(size_t)m * sm + (size_t)c * sc + t] : 0.0f;
+        int m, c, t;
+        if (KK == 9) {
+            const int f = (q & 1) * 256 + j, L = f >> 3;
+            t = (int)(ptap >> 4 * ((q & ~1) + (L >> 5))) & 15;
+            m = mblk * 32 + (L & 31);
+            c = chunk * 8 + (f & 7);
+        } else {
+            const int L = j >> 2;
+            t = q % KK;
+            m = mblk * 32 + (L & 31);
+            c = chunk * CH + (L >> 5) * (CH >> 1) + 4 * (q / KK) + (j & 3);
+        }
+        return t < 9 && m < CD && c < CS ? w[(size_t)m * sm + (size_t)c * sc + t] : 0.0f;
     }
 };
 // The packing of `sp` in direction dx (RNN_E_UNSUPPORTED: no specialised

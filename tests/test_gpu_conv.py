@@ -278,3 +278,51 @@ def test_conv_layercheck_gpu(rnn, orc):
     assert len(res) == 6
     bad = [(t, e) for t, e in res if not e < refcheck.TOL]
     assert not bad, res
+
+
+# The split 3x3 kernels at their edges: fewer than 8 channels and one past a
+# chunk, channel blocks one short of and past 32, tiles with a last row, a
+# window of the widest plan, one pixel.
+@pytest.mark.parametrize("n,cin,cout,s,h,w", [(1, 1, 1, 1, 1, 1), (2, 9, 33, 1, 17, 31),
+                                              (3, 7, 31, 2, 9, 33), (1, 8, 64, 1, 3, 250),
+                                              (1, 16, 40, 2, 40, 127), (64, 24, 32, 1, 32, 32)])
+def test_conv_split_matches_float64(rnn, n, cin, cout, s, h, w):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + cin + cout)
+    sp = rnn.ConvSpec.make(cin, cout, 3, s, 1, h, w)
+    x = torch.randn((n, cin, h, w), generator=g, device="cuda")
+    wt = torch.randn((cout, cin, 3, 3), generator=g, device="cuda")
+    dy = torch.randn((n, cout, sp.oh, sp.ow), generator=g, device="cuda")
+    xd, wd = x.double().requires_grad_(True), wt.double()
+    cols = torch.nn.functional.unfold(xd, 3, padding=1, stride=s)
+    y = (wd.reshape(cout, -1) @ cols).view(dy.shape)
+    dx, = torch.autograd.grad(y, xd, dy.double())
+    # k sums of rounded products as a random walk: 2^-24 sqrt(k) of the result,
+    # with 2^-23 for the part products left out
+    tol = lambda k: 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23
+    for p in (False, True):
+        wp = [rnn.conv_pack_weights(sp, d, wt.view(-1)) for d in (0, 1)] if p else None
+        a = (rnn.conv2d_forward_packed(sp, n, x, wt.view(-1), wp[0]) if p
+             else rnn.conv2d_forward(sp, n, x, wt.view(-1)))
+        b = (rnn.conv2d_backward_x_packed(sp, n, dy, wt.view(-1), wp[1]) if p
+             else rnn.conv2d_backward_x(sp, n, dy, wt.view(-1)))
+        assert rel_frob(to_host(a), to_host(y)) < tol(9 * cin)
+        assert rel_frob(to_host(b), to_host(dx)) < tol(9 * cout)
+
+
+@pytest.mark.parametrize("s", [1, 2])
+def test_conv_split_special_values(rnn, s):
+    """Infinities and NaN reach the outputs that IEEE products and sums give,
+    and no others; the largest float comes through whole."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(5)
+    n, cin, cout, h = 3, 12, 36, 16
+    sp = rnn.ConvSpec.make(cin, cout, 3, s, 1, h, h)
+    x = torch.randint(1, 4, (n, cin, h, h), generator=g, device="cuda").float()
+    wt = torch.randint(1, 4, (cout, cin, 3, 3), generator=g, device="cuda").float()
+    x[0, 2, 3, 4], x[1, 5, 8, 8] = float("inf"), float("nan")
+    x[2] = 0.0
+    x[2, 1, 5, 5], wt[:, 1] = torch.finfo(torch.float32).max, 1.0
+    want = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), stride=s, padding=1)
+    got = rnn.conv2d_forward(sp, n, x, wt.view(-1))
+    assert np.array_equal(to_host(got), want.float().numpy().ravel(), equal_nan=True)
