@@ -1,4 +1,5 @@
-// Convolution weight gradient, deterministic split-K on fp32 MFMA.
+// Convolution weight gradient, deterministic split-K on MFMA (3x3: the bf16
+// cores, each float in three exact parts; 1x1: the fp32 ones).
 //
 // dW[co][ci][kh][kw] += sum over (n, oy, ox) of dY[n][co][oy][ox] *
 //                       X[n][ci][oy*s + kh - pad][ox*s + kw - pad]
@@ -22,12 +23,19 @@
 // Compute: a wave takes 8-pixel groups of a tile row; lane half h reads the 4
 // pixels 4h..4h+3 of the group with one ds_read_b128 for dY and, per kernel
 // row kh, the 6 (or 5 + 4) X values those pixels touch, so the three kw taps
-// are register offsets into the same read.  MFMA k-step i takes pixels i and
-// 4 + i; a wave's tap accumulators (5 or 4) are independent chains.  The 4
+// are register offsets into the same read.  3x3: two groups make a k step of
+// 16 pixels, split in registers (44 VALU instructions per operand, hidden
+// behind the other MFMA wave of the SIMD).  Measured, fp32 pipe -> here: the
+// grouped launch of the ResNet-20 step 337 -> 241 us; alone with its slab sum
+// at batch 128 32 -> 32 @32x32 33.3 -> 29.0 us, 96 -> 96 @16x16 59.0 -> 45.6,
+// 48 -> 80 @23x29 (37 images) 46.1 -> 33.7; errors against 64 bits 1.9e-7 ->
+// 1.6e-7, 2.2e-7 -> 1.4e-7, 1.8e-7 -> 1.3e-7.  1x1: k-step i takes pixels i
+// and 4 + i.  The 4
 // waves of a tap set add their sums through LDS in a fixed pairwise order and the workgroup
 // writes one partial slab; slabs are added in slab order by one reduction
 // launch (no atomics: the result is bit-reproducible).
 #include "conv_common.h"
+#include "mfma_split.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -373,41 +381,68 @@ __device__ __forceinline__ void dw_issue_tile4(const DwArgs &g, const DwLane4<S>
                 rd, (lds_ptr_t)(buf + g.xwords + (pw + DW_NP * kk) * 256), 16, L.dof[kk], 0, 0, 0);
 }
 
-// MFMAs of one 8-pixel group for taps T0 .. T0 + NT - 1 (a 1x1 kernel: the
-// four k-steps into four accumulators): k-step i takes pixels i and 4 + i.
-template <int K, int S, bool X4, int T0, int NT>
-__device__ __forceinline__ void dw_mma(const DwOps<K, S, X4> &o, f32x16 (&acc)[NT]) {
+// MFMAs of one 8-pixel group of a 1x1 kernel: k-step i takes pixels i and
+// 4 + i, the four k-steps into four accumulators.
+template <int S>
+__device__ __forceinline__ void dw_mma1(const DwOps<1, S, false> &o, f32x16 (&acc)[4]) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if constexpr (K == 1) {
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.a[i], dw_bval<K, S, X4>(o, 0, 0, i),
-                                                          acc[i], 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                    o.a[i], dw_bval<K, S, X4>(o, (T0 + j) / K, (T0 + j) % K, i), acc[j], 0, 0, 0);
-        }
-    }
+    for (int i = 0; i < 4; i++)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.a[i], dw_bval<1, S, false>(o, 0, 0, i),
+                                                      acc[i], 0, 0, 0);
 }
 
 // Scheduling hint for one step: the LDS reads of the next group go out
 // among the first MFMAs of this one, so their latency hides under the rest.
-template <int K, int S, bool X4, int NT>
-__device__ __forceinline__ void dw_step_schedule() {
-    constexpr int NMF = K == 1 ? 4 : 4 * NT;
-    constexpr int NRD = 1 + (K == 1 ? 1 : K * (S == 2 || X4 ? 3 : 2));
-    static_for<0, NRD>([&](auto) {
+__device__ __forceinline__ void dw_step_schedule1() {
+    static_for<0, 2>([&](auto) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
     });
-    __builtin_amdgcn_sched_group_barrier(0x008, NMF - NRD, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 }
 
-// The GEMM steps of one staged tile: 8-pixel groups wave, wave + NW, ...;
-// two operand sets alternate so that the reads of group n+1 overlap the
-// MFMAs of group n.  Reads past the tile's last group are clamped to group
-// `wave` (in range; their values are not used).
+// MFMAs of two 8-pixel groups of a 3x3 kernel for taps T0 .. T0 + NT - 1: one
+// k step of 16 pixels (lane half h: pixels 4h .. 4h+3 of both), the operands
+// split into bf16 parts in registers (mfma_split.h).  The smaller part
+// products are summed from zero each step: accumulators of their own would
+// take 80 registers more than three waves a SIMD have, and in acc itself they
+// cost it accuracy (32 -> 32 @32x32, 128 images: 2.1e-7 against 64 bits).
+template <int S, bool X4, int T0, int NT>
+__device__ __forceinline__ void dw_mma3(const DwOps<3, S, X4> &oa, const DwOps<3, S, X4> &ob,
+                                        bool both, f32x16 (&acc)[NT]) {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        y[i] = oa.a[i];
+        y[4 + i] = both ? ob.a[i] : 0.f;
+    }
+    const Bf3 a = bf3_split_round(y);  // once for all taps
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int kh = (T0 + j) / 3, kw = (T0 + j) % 3;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            y[i] = dw_bval<3, S, X4>(oa, kh, kw, i);
+            y[4 + i] = dw_bval<3, S, X4>(ob, kh, kw, i);
+        }
+        const Bf3 b = bf3_split(y);
+        f32x16 t;
+#pragma unroll
+        for (int v = 0; v < 16; v++) t[v] = 0.f;
+        bf3_products([&](auto pick, auto small) {
+            if constexpr (decltype(small)::value)
+                t = pick(a, b, t);
+            else
+                acc[j] = pick(a, b, acc[j]);
+        });
+        acc[j] += t;
+    }
+}
+
+// The GEMM steps of one staged tile: 8-pixel groups wave, wave + NW, ... (3x3:
+// two at a time; 1x1: two operand sets alternate so that the reads of group
+// n+1 overlap the MFMAs of group n).  Reads past the tile's last group are
+// clamped to group `wave` (in range; their values are not used).
 template <int K, int S, bool X4, int T0, int NT>
 __device__ __forceinline__ void dw_compute(const DwArgs &g, const float *__restrict__ cur,
                                            int wave, int lane, f32x16 (&acc)[NT]) {
@@ -418,16 +453,60 @@ __device__ __forceinline__ void dw_compute(const DwArgs &g, const float *__restr
         return gi < g.ngroups ? gi : min(wave, g.ngroups - 1);
     };
     DwOps<K, S, X4> oa, ob;
-    dw_fetch<K, S, X4>(g, xs, ds, grp(0), lane, oa);
+    if constexpr (K == 3) {
 #pragma unroll 1
-    for (int s = 0; s < nsteps; s += 2) {
-        dw_fetch<K, S, X4>(g, xs, ds, grp(s + 1), lane, ob);
-        dw_mma<K, S, X4, T0, NT>(oa, acc);
-        dw_step_schedule<K, S, X4, NT>();
-        if (s + 1 >= nsteps) break;
-        dw_fetch<K, S, X4>(g, xs, ds, grp(s + 2), lane, oa);
-        dw_mma<K, S, X4, T0, NT>(ob, acc);
-        dw_step_schedule<K, S, X4, NT>();
+        for (int s = 0; s < nsteps; s += 2) {
+            dw_fetch<K, S, X4>(g, xs, ds, grp(s), lane, oa);
+            dw_fetch<K, S, X4>(g, xs, ds, grp(s + 1), lane, ob);
+            dw_mma3<S, X4, T0, NT>(oa, ob, s + 1 < nsteps, acc);
+        }
+    } else {
+        dw_fetch<K, S, X4>(g, xs, ds, grp(0), lane, oa);
+#pragma unroll 1
+        for (int s = 0; s < nsteps; s += 2) {
+            dw_fetch<K, S, X4>(g, xs, ds, grp(s + 1), lane, ob);
+            dw_mma1<S>(oa, acc);
+            dw_step_schedule1();
+            if (s + 1 >= nsteps) break;
+            dw_fetch<K, S, X4>(g, xs, ds, grp(s + 2), lane, oa);
+            dw_mma1<S>(ob, acc);
+            dw_step_schedule1();
+        }
+    }
+}
+
+// A 3x3 wave's sums again with fp32 MFMAs from global memory: for values that
+// are not finite in the split (see bf3_nonfinite).
+template <int S, int T0, int NT>
+__device__ __forceinline__ void dw_slow(const DwArgs &g, int z, int cob, int cib, int wave,
+                                        int lane, f32x16 (&acc)[NT]) {
+    const int h = lane >> 5, co = cob * 32 + (lane & 31), ci = cib * 32 + (lane & 31);
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[j][v] = 0.f;
+    for (int tile = z; tile < g.ntiles; tile += g.nz) {
+        const int n0 = (tile / g.tiles_a) * g.IMGS, a0 = (tile % g.tiles_a) * g.TR;
+        for (int grp = wave; grp < g.ngroups; grp += DW_NW) {
+            const int rr = grp / g.gpr, cq = grp - rr * g.gpr;
+            const int n = n0 + rr / g.TR, oy = a0 + rr % g.TR;
+#pragma unroll 1
+            for (int i = 0; i < 4; i++) {
+                const int ox = 8 * cq + 4 * h + i;
+                const bool live = n < g.N && oy < g.OH && ox < g.OW;
+                const float a = live && co < g.CO ? g.dy[(long long)n * g.cohw +
+                                                         (long long)co * g.ohw + oy * g.OW + ox]
+                                                  : 0.f;
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const int y = oy * S + (T0 + j) / 3 - g.pad, x = ox * S + (T0 + j) % 3 - g.pad;
+                    const bool in = live && ci < g.CI && y >= 0 && y < g.H && x >= 0 && x < g.W;
+                    const float b =
+                        in ? g.x[(long long)n * g.cihw + (long long)ci * g.hw + y * g.W + x] : 0.f;
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[j], 0, 0, 0);
+                }
+            }
+        }
     }
 }
 
@@ -460,7 +539,7 @@ __device__ __forceinline__ void dw_red_add(const float *src, int lbase, f32x16 *
 // the same slices at once.
 template <int K, int S, bool X4, int NB, int T0, int NT>
 __device__ __forceinline__ void dw_mfma_wave(const DwArgs &g, float *smem, float *red, int z,
-                                             int wq, int lane) {
+                                             int cob, int cib, int wq, int lane) {
     constexpr int KK = K * K, SL = KK * 1024, NR = K == 1 ? 1 : NT;
     f32x16 acc[NT];
 #pragma unroll
@@ -476,6 +555,14 @@ __device__ __forceinline__ void dw_mfma_wave(const DwArgs &g, float *smem, float
             dw_compute<K, S, X4, T0, NT>(g, smem, wq, lane, acc);
             __syncthreads();
         }
+    }
+    if constexpr (K == 3) {
+        bool bad = false;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) bad = bad || bf3_nonfinite(acc[t][v]);
+        if (__any(bad)) dw_slow<S, T0, NT>(g, z, cob, cib, wq, lane, acc);
     }
     if constexpr (K == 1) {
 #pragma unroll
@@ -547,11 +634,11 @@ __device__ __forceinline__ void dw_body(const DwArgs &g, int z, int cob, int cib
         __syncthreads();
         __syncthreads();
     } else if constexpr (K == 1) {
-        dw_mfma_wave<K, S, X4, NB, 0, 4>(g, smem, red, z, wave, lane);
+        dw_mfma_wave<K, S, X4, NB, 0, 4>(g, smem, red, z, cob, cib, wave, lane);
     } else if (wave < DW_NW) {
-        dw_mfma_wave<K, S, X4, NB, 0, 5>(g, smem, red, z, wave, lane);
+        dw_mfma_wave<K, S, X4, NB, 0, 5>(g, smem, red, z, cob, cib, wave, lane);
     } else {
-        dw_mfma_wave<K, S, X4, NB, 5, KK - 5>(g, smem, red, z, wave - DW_NW, lane);
+        dw_mfma_wave<K, S, X4, NB, 5, KK - 5>(g, smem, red, z, cob, cib, wave - DW_NW, lane);
     }
     const int ckk = g.CI * KK, rowlen = 32 * KK;
     float *slab = g.part + (long long)z * g.CO * ckk + cib * 32 * KK;

@@ -58,6 +58,28 @@ __device__ __forceinline__ Bf3 bf3_split(const float (&x)[8]) {
     return p;
 }
 
+// The parts rounded to nearest instead of cut off: with one operand of a
+// product split this way the part products left out have no common sign (cut
+// off, they make results 3.3e-8 smaller).  Slower (bf16 conversions), and
+// values within 2^-9 of the largest float overflow to infinity.
+__device__ __forceinline__ Bf3 bf3_split_round(const float (&x)[8]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    Bf3 p;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float a = x[2 * j], b = x[2 * j + 1];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const bf16x2 v = {(__bf16)a, (__bf16)b};
+            const uint32_t u = __builtin_bit_cast(uint32_t, v);
+            (q == 0 ? p.hi : q == 1 ? p.mid : p.lo)[j] = u;
+            a -= __uint_as_float(u << 16);
+            b -= __uint_as_float(u & 0xFFFF0000u);
+        }
+    }
+    return p;
+}
+
 __device__ __forceinline__ f32x16 bf3_mfma1(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);

@@ -326,3 +326,32 @@ def test_conv_split_special_values(rnn, s):
     want = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), stride=s, padding=1)
     got = rnn.conv2d_forward(sp, n, x, wt.view(-1))
     assert np.array_equal(to_host(got), want.float().numpy().ravel(), equal_nan=True)
+
+
+# dW on the split kernel: one pixel, an odd count of 8-pixel groups a wave,
+# rows that are no whole groups, channels off the 32-blocks, both stagings.
+@pytest.mark.parametrize("n,cin,cout,s,h,w", [(1, 5, 1, 1, 1, 1), (3, 33, 31, 1, 9, 13),
+                                              (2, 40, 70, 2, 17, 22), (9, 36, 32, 1, 16, 16),
+                                              (5, 64, 32, 2, 32, 32)])
+def test_conv_dw_split(rnn, n, cin, cout, s, h, w):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + cin + cout)
+    sp = rnn.ConvSpec.make(cin, cout, 3, s, 1, h, w)
+    x = torch.randn((n, cin, h, w), generator=g, device="cuda")
+    dy = torch.randn((n, cout, sp.oh, sp.ow), generator=g, device="cuda")
+    cols = torch.nn.functional.unfold(x.double(), 3, padding=1, stride=s)
+    want = dy.double().reshape(n, cout, -1).permute(1, 0, 2).reshape(cout, -1) @ (
+        cols.permute(0, 2, 1).reshape(-1, 9 * cin))
+    dw = torch.zeros(cout * cin * 9, device="cuda")
+    rnn.conv2d_backward_w(sp, n, dy, x, dw)
+    # as the forward's bound, over n oh ow pixels
+    tol = 2.0 ** -24 * np.sqrt(n * sp.hw) + 2.0 ** -23
+    assert rel_frob(to_host(dw), to_host(want)) < tol
+    if h > 1:  # an infinity reaches the weights its pixel touches, and only those
+        x[0, 2, h // 2, w // 2] = float("inf")
+        x, dy = x.abs().round(), dy.abs().round() + 1.0
+        dw.zero_()
+        rnn.conv2d_backward_w(sp, n, dy, x, dw)
+        got = to_host(dw).reshape(cout, cin, 9)
+        assert np.isfinite(np.delete(got, 2, axis=1)).all() and not np.isnan(got[:, 2, 4]).any()
+        assert (~np.isfinite(got[:, 2])).any()
