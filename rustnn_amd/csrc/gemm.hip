@@ -5,11 +5,11 @@
 // parallel over 6-row C panels), linear.rs.  Here one workgroup owns a
 // BM x BN tile of C, its compute waves sub-tiles of 32x32 MFMA accumulators.
 // Two kernels:
-//   * gemm_dma_kernel (every operand whose 16-byte quads are whole): producer
-//     waves DMA the slabs from HBM straight into a multi-stage LDS ring; the
-//     products run on the bf16 matrix cores, each float in three exact parts
-//     (mfma_split.h);
-//   * gemm_kernel (any shape and alignment): the 4 waves load a slab into
+//   * gemm_dma_kernel (operands under 2 GiB): producer waves DMA the slabs
+//     from HBM straight into a multi-stage LDS ring, 16 bytes a lane where
+//     every operand quad is whole, else one float; the products run on the
+//     bf16 matrix cores, each float in three exact parts (mfma_split.h);
+//   * gemm_kernel (any shape): the 4 waves load a slab into
 //     registers and store it k-contiguous (16 k values + 4 pad floats a row)
 //     into a double-buffered LDS tile, multiplied by v_mfma_f32_32x32x2f32
 //     (k order inside a block of 8 permuted identically for A and B: step s
@@ -221,11 +221,11 @@ struct GemmTile {
 //     consecutive rows at one quad hit distinct banks;
 //   * row-contiguous (A^T [k][m], B [k][n]): [BK][rows] as stored, read one
 //     float per k (32 consecutive floats per half-wave).
-// Eligible when every 16-byte quad is either wholly inside the operand or
+// 16 bytes a lane when every quad is either wholly inside the operand or
 // wholly outside (rows and k multiples of 4 where they run along a quad,
-// 16-byte aligned bases): a quad outside the k range reads zero through an
-// out-of-range offset; rows beyond M / N only feed C rows / columns that are
-// never stored.
+// 16-byte aligned bases), else one float: a quad or float outside the k range
+// reads zero through an out-of-range offset; rows beyond M / N only feed C
+// rows / columns that are never stored.
 //
 // The product of two float fragments is taken on the bf16 matrix cores: each
 // float is the exact sum of three bf16 parts (mfma_split.h), and six of the
@@ -249,31 +249,32 @@ __device__ __forceinline__ int kswz(int r) {
         return ((r >> 1) ^ (r >> 2)) & 3;
 }
 
-template <int R, int BK, bool KMAJOR, int NP>
+// VW: floats a lane moves per DMA, 4 where every 16-byte quad is whole, else 1.
+template <int R, int BK, bool KMAJOR, int NP, int VW>
 struct DmaOperand {
-    static constexpr int WORDS = R * BK;               // LDS floats per stage
-    static constexpr int PER = WORDS / 4 / (64 * NP);  // dwordx4 DMAs per producer thread
-    static_assert(WORDS % (256 * NP) == 0, "whole DMA rows");
+    static constexpr int WORDS = R * BK;                // LDS floats per stage
+    static constexpr int PER = WORDS / VW / (64 * NP);  // DMAs per producer thread
+    static_assert(WORDS % (64 * VW * NP) == 0, "whole DMA rows");
 
     // This thread's source byte offsets at k = 0, per DMA of a stage: rows
     // r0.. (KMAJOR) or columns r0.. of a stage's k values.  A stage adds its
     // k offset in a scalar, so that an issue costs no vector arithmetic.
     uint32_t off[PER];
 
-    // DMA u's quad of this lane in a stage's slab.
-    __device__ __forceinline__ static int quad(int u, int wave, int lane) {
-        return (u * NP + wave) * 64 + lane;
+    // First word of DMA u of this lane in a stage's slab.
+    __device__ __forceinline__ static int word(int u, int wave, int lane) {
+        return ((u * NP + wave) * 64 + lane) * VW;
     }
-    // First k of quad j, relative to the stage.
+    // The k of word j, relative to the stage.
     __device__ __forceinline__ static int kof(int j) {
-        if (KMAJOR) return ((j % (BK / 4)) ^ kswz<BK>(j / (BK / 4))) * 4;
-        return j / (R / 4);
+        if (KMAJOR) return ((j % BK / 4) ^ kswz<BK>(j / BK)) * 4 + j % 4;
+        return j / R;
     }
     __device__ __forceinline__ void init(int ld, int rows, int r0, int wave, int lane) {
 #pragma unroll
         for (int u = 0; u < PER; u++) {
-            const int j = quad(u, wave, lane);
-            const int row = KMAJOR ? r0 + j / (BK / 4) : r0 + j % (R / 4) * 4;
+            const int j = word(u, wave, lane);
+            const int row = r0 + (KMAJOR ? j / BK : j % R);
             off[u] = row >= rows ? DMA_OOB
                      : KMAJOR    ? (uint32_t)(row * ld + kof(j)) * 4u
                                  : (uint32_t)(kof(j) * ld + row) * 4u;
@@ -287,9 +288,12 @@ struct DmaOperand {
 #pragma unroll
         for (int u = 0; u < PER; u++) {
             uint32_t o = off[u];
-            if (!whole && k0 + kof(quad(u, wave, lane)) >= kz) o = DMA_OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rs, (lds_ptr_t)(lds + 4 * quad(u, wave, 0)), 16, o, so, 0, 0);
+            if (!whole && k0 + kof(word(u, wave, lane)) >= kz) o = DMA_OOB;
+            const lds_ptr_t to = (lds_ptr_t)(lds + word(u, wave, 0));
+            if constexpr (VW == 4)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, to, 16, o, so, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, to, 4, o, so, 0, 0);
         }
     }
 
@@ -326,12 +330,12 @@ struct DmaOperand {
 // stage it has landed (each producer waited for its own DMAs) and every
 // compute wave is done with stage it - 1, whose buffer the producers then
 // refill with stage it + NS - 1.
-template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, int NACC, bool AT,
-          bool BT>
+template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, int NACC, int VW,
+          bool AT, bool BT>
 struct DmaTile {
     static constexpr int NC = WM * WN * WK;
-    using OA = DmaOperand<BM, BK, !AT, NP>;
-    using OB = DmaOperand<BN, BK, BT, NP>;
+    using OA = DmaOperand<BM, BK, !AT, NP, VW>;
+    using OB = DmaOperand<BN, BK, BT, NP, VW>;
     static constexpr int ROWS = BM, COLS = BN, THREADS = 64 * (NC + NP);
     static constexpr int STAGE = OA::WORDS + OB::WORDS;
     static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
@@ -575,16 +579,25 @@ struct DmaTile {
 // products (mfma_split.h) where the registers allow it; on the 64 x 64 tile
 // it costs a workgroup a CU (8192 x 768 x 256 31.7 -> 32.5 us).
 template <bool AT, bool BT>
-using Tile32 = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, AT, BT>;
+using Tile32 = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, 4, AT, BT>;
 template <bool AT, bool BT>
-using Tile64 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, AT, BT>;
+using Tile64 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, 4, AT, BT>;
 template <bool AT, bool BT>
-using Tile128 = DmaTile<128, 128, 32, 3, 2, 2, 2, 4, 1, AT, BT>;
+using Tile128 = DmaTile<128, 128, 32, 3, 2, 2, 2, 4, 1, 4, AT, BT>;
 template <bool AT, bool BT>
-using Tile256 = DmaTile<256, 128, 16, 4, 4, 2, 1, 4, 1, AT, BT>;
+using Tile256 = DmaTile<256, 128, 16, 4, 4, 2, 1, 4, 1, 4, AT, BT>;
+// Operands whose 16-byte quads are not whole: one float a lane and DMA.  Four
+// times the DMA instructions, but no scalar loads into registers and no LDS
+// writes as in gemm_kernel, which took these before: 1003 x 517 x 771 (A B^T)
+// 48.3 -> 20.3 us, 33 x 77 x 4095 27.2 -> 14.4, 8191 x 255 x 257 23.3 -> 16.7,
+// 2047 x 2049 x 511 112 -> 49.
+template <bool AT, bool BT>
+using Tile32u = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, 1, AT, BT>;
+template <bool AT, bool BT>
+using Tile64u = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, 1, AT, BT>;
 // Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile.
 template <bool AT, bool BT>
-using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, AT, BT>;
+using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, 4, AT, BT>;
 
 template <class Tile, bool RS>
 __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(GemmArgs g) {
@@ -938,14 +951,21 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
-// Whether every operand quad of the direct-to-LDS kernel is wholly inside or
-// wholly outside its operand, and every problem's operand spans under 2^31
-// bytes (buffer offsets).
+// Whether every problem's operand spans under 2^31 bytes (buffer offsets of
+// the direct-to-LDS kernel).
+static bool dma_extent_ok(size_t m, size_t n, size_t kchunk, size_t ktotal, int lda, int at,
+                          int ldb, int bt) {
+    const size_t lim = 0x7FFF0000u / 4, kz = std::min(kchunk, ktotal);
+    const size_t ea = at ? kz * (size_t)lda : m * (size_t)lda;
+    const size_t eb = bt ? n * (size_t)ldb : kz * (size_t)ldb;
+    return ea < lim && eb < lim;
+}
+
+// Whether, besides, every operand quad is wholly inside or wholly outside its
+// operand (16 bytes a lane and DMA).
 static bool dma_ok(size_t count, size_t m, size_t n, size_t kchunk, size_t ktotal, const float *a,
                    size_t stride_a, int lda, int at, const float *b, size_t stride_b, int ldb,
                    int bt) {
-    const size_t lim = 0x7FFF0000u / 4;
-    const size_t kz = std::min(kchunk, ktotal);
     auto aligned = [](const void *p, size_t stride, int ld) {
         return ((uintptr_t)p & 15) == 0 && stride % 4 == 0 && ld % 4 == 0;
     };
@@ -954,9 +974,7 @@ static bool dma_ok(size_t count, size_t m, size_t n, size_t kchunk, size_t ktota
     if ((!at || bt) && (kchunk % 4 || ktotal % 4)) return false;
     if (at && m % 4) return false;
     if (!bt && n % 4) return false;
-    const size_t ea = at ? kz * (size_t)lda : m * (size_t)lda;
-    const size_t eb = bt ? n * (size_t)ldb : kz * (size_t)ldb;
-    return ea < lim && eb < lim;
+    return dma_extent_ok(m, n, kchunk, ktotal, lda, at, ldb, bt);
 }
 
 // Enqueues `count` GEMMs C_z = op(A_z) op(B_z) (+C_z) (+bias) with problem z
@@ -974,8 +992,8 @@ static bool dma_enabled() {
 
 // Whether C += A^T B (A [k x m], B [k x n]) takes the direct-to-LDS kernel,
 // which can then also sum A's columns (the row sums of A^T).
-static bool dw_rowsum_ok(size_t m, size_t n, size_t k, const float *a, const float *b) {
-    return dma_enabled() && dma_ok(1, m, n, k, k, a, 0, (int)m, 1, b, 0, (int)n, 0);
+static bool dw_rowsum_ok(size_t m, size_t n, size_t k) {
+    return dma_enabled() && dma_extent_ok(m, n, k, k, (int)m, 1, (int)n, 0);
 }
 
 // rs_out / rs_part: the row sums of op(A) (A^T B layout and the direct-to-LDS
@@ -1038,6 +1056,12 @@ static int gemm_enqueue(rnn_ctx *ctx, size_t count, size_t m, size_t n, size_t k
             return launch_dma<Tile128>(ctx, g, (int)count, at, bt);
         if (tiles64 < cus) return launch_dma<Tile32>(ctx, g, (int)count, at, bt);
         return launch_dma<Tile64>(ctx, g, (int)count, at, bt);
+    }
+    if (dma_enabled() && dma_extent_ok(m, n, kchunk, ktotal, lda, at, ldb, bt)) {
+        // quads that are not whole: the aligned rule's line between the tiles
+        if (rnn_div_up(m, 64) * rnn_div_up(n, 64) * count < (size_t)ctx->num_cus)
+            return launch_dma<Tile32u>(ctx, g, (int)count, at, bt);
+        return launch_dma<Tile64u>(ctx, g, (int)count, at, bt);
     }
     if (rs_out || rs_part) return rnn_fail(ctx, RNN_E_INVALID, "gemm: row sums need the DMA path");
     const bool big = m >= 128 && n >= 128 && tiles128 >= (size_t)ctx->num_cus;
@@ -1278,7 +1302,7 @@ int rnn_linear_backward_ex(rnn_ctx *ctx, size_t rows, size_t fin, size_t fout, c
     // (linear.rs:70-89), summed in f64 by the dW GEMM itself when it takes
     // the direct-to-LDS kernel, else by the column-sum kernels
     int rc;
-    if (db && rows && fout && fin && dw_rowsum_ok(fout, fin, rows, dy, x)) {
+    if (db && rows && fout && fin && dw_rowsum_ok(fout, fin, rows)) {
         rc = gemm_splitk(ctx, fout, fin, rows, dy, 1, x, 0, dw, 1, db, true);
         if (rc == -1)
             rc = gemm_enqueue(ctx, 1, fout, fin, rows, rows, dy, 0, (int)fout, 1, x, 0, (int)fin,

@@ -255,8 +255,10 @@ def test_destroy_flushes_deferred_reductions(rnn, orc):
 # The direct-to-LDS tiles at their edges: a quad past the last whole tile, one
 # short of it, the shortest k, k off a stage; 32 x 64, 64 x 64, 128 x 128 and
 # 256 x 128 tiles by size.
+# Then sizes that no 16-byte quad divides (one float a lane and DMA).
 @pytest.mark.parametrize("m,n,k", [(4, 4, 4), (36, 68, 12), (516, 2052, 132), (2044, 2180, 1028),
-                                   (16388, 1028, 36)])
+                                   (16388, 1028, 36), (1, 1, 1), (33, 65, 67), (1001, 1030, 35),
+                                   (70, 31, 2051)])
 @pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
 def test_matmul_split_tiles(rnn, m, n, k, at, bt):
     import torch
@@ -287,3 +289,21 @@ def test_matmul_split_special_values(rnn, m, n, k):
     # integer results are exact, the largest float comes through whole
     want = (a.double() @ b.double()).float()
     assert np.array_equal(to_host(c), to_host(want), equal_nan=True)
+
+
+@pytest.mark.parametrize("rows,fin,fout", [(35, 33, 31), (2050, 130, 67), (5, 513, 2)])
+def test_linear_backward_ragged_bias(rnn, rows, fin, fout):
+    """db rides in the dW product for ragged sizes too, also split over rows."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    dy = torch.randn((rows, fout), generator=g, device="cuda")
+    x = torch.randn((rows, fin), generator=g, device="cuda")
+    w = torch.randn((fout, fin), generator=g, device="cuda")
+    dw, db = torch.ones(fout * fin, device="cuda"), torch.ones(fout, device="cuda")
+    dx = rnn.linear_backward(rows, fin, fout, dy, x, w, dw, db)
+    # sums of at most `rows` rounded products (test_matmul_split_tiles); db in f64
+    tol = lambda k: 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23
+    d = dy.double()
+    assert rel_frob(to_host(dw) - 1, to_host(d.T @ x.double())) < 2 * tol(rows)
+    assert rel_frob(to_host(db), to_host(d.sum(0) + 1)) < 2.0 ** -23
+    assert rel_frob(to_host(dx), to_host(d @ w.double())) < tol(fout)
