@@ -339,7 +339,7 @@ struct SplitStage {
         for (int u = 0; u < TW; u++) {
             const int t = wtask(g, u, dw);
             if (t < 5 * SL) {
-                const Bf3 p = bf3_split(wv[B][u]);
+                const Bf3 p = bf3_split_near(wv[B][u]);
                 u32x4 *q = w + t * 192 + lane;
                 q[0] = p.hi;
                 q[64] = p.mid;

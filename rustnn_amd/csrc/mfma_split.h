@@ -80,8 +80,34 @@ __device__ __forceinline__ Bf3 bf3_split_round(const float (&x)[8]) {
     return p;
 }
 
+// The same with the leading part alone rounded, which already takes the common
+// sign away, for one integer add a float more than bf3_split.  On the weights
+// of the 3x3 convolutions: logits of 17 ResNets of 8 to 20 layers 1.047 times
+// the fp32 pipe's error against 64 bits cut off, 0.996 this way, for 1% of the
+// time (a ResNet-20 step 1953 -> 1973 us).
+// An infinity's or NaN's remainder is a NaN.
+__device__ __forceinline__ Bf3 bf3_split_near(const float (&x)[8]) {
+    Bf3 p;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float a = __uint_as_float(__float_as_uint(x[2 * j]) + 0x8000u);
+        const float b = __uint_as_float(__float_as_uint(x[2 * j + 1]) + 0x8000u);
+        p.hi[j] = bf3_top2(a, b);
+        const float ra = x[2 * j] - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+        const float rb = x[2 * j + 1] - __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
+        p.mid[j] = bf3_top2(ra, rb);
+        p.lo[j] = bf3_top2(bf3_rest(ra), bf3_rest(rb));
+    }
+    return p;
+}
+
 __device__ __forceinline__ f32x16 bf3_mfma1(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 bf3_mfma1(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
@@ -92,12 +118,12 @@ template <typename F>
 __device__ __forceinline__ void bf3_products(F &&f) {
     const std::integral_constant<int, 0> lead;
     const std::integral_constant<int, 1> small;
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.mid, b.mid, c); }, small);
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.lo, c); }, small);
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.lo, b.hi, c); }, small);
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.mid, c); }, small);
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.mid, b.hi, c); }, small);
-    f([](const Bf3 &a, const Bf3 &b, f32x16 c) { return bf3_mfma1(a.hi, b.hi, c); }, lead);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.mid, b.mid, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.hi, b.lo, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.lo, b.hi, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.hi, b.mid, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.mid, b.hi, c); }, small);
+    f([](const Bf3 &a, const Bf3 &b, auto c) { return bf3_mfma1(a.hi, b.hi, c); }, lead);
 }
 
 template <int TM, int TN>
