@@ -28,6 +28,7 @@
 // writes its (image, head) partial -- drel through an inverse index (for
 // every bias slot, the positions that map to it, in ascending order) -- and a
 // second kernel adds the partials over images in image order.
+#include "mfma_split.h"
 #include "rnn_internal.h"
 
 #include <algorithm>
@@ -40,8 +41,6 @@ constexpr int MAXT = 64;   // tq, tk limit of the workgroup kernels
 constexpr int MAXDH = 64;  // head-dim limit
 constexpr int TS = 68;     // LDS row stride of the [64]-wide transposed tiles
 constexpr int LT = 4096;   // u32 entries of the lane-order relidx table
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct AttnArgs {
     const float *q, *kv, *tau, *rel, *p, *dout;
@@ -927,38 +926,99 @@ attn_bwd_long_q_kernel(AttnArgs g, float *__restrict__ s2) {
     }
 }
 
+// The 16-byte slots of a [head dim][64 queries] bf16 row in LDS: 8 of 8
+// queries and one of padding, so that 16 consecutive rows' b128 accesses at
+// one slot hit distinct banks.
+constexpr int KSLOT = 9;
+
+// One operand of attn_bwd_long_k_kernel: src's rows (queries) transposed into
+// LDS as their three bf16 parts, [part][head dim][KSLOT]; a thread loads 8
+// queries of a head dim.
+template <int DHP>
+struct SplitTile {
+    static constexpr int TASKS = DHP * 8 / 256;
+    float v[TASKS][8];
+    __device__ __forceinline__ void load(const float *src, long long stride, int nrows, int tid) {
+#pragma unroll
+        for (int t = 0; t < TASKS; t++) {
+            const int i = tid + 256 * t, d = i % DHP, r = i / DHP * 8;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                v[t][j] = src[(long long)min(r + j, nrows - 1) * stride + d];
+        }
+    }
+    __device__ __forceinline__ void store(u32x4 *dst, int nrows, int tid) {
+#pragma unroll
+        for (int t = 0; t < TASKS; t++) {
+            const int i = tid + 256 * t, d = i % DHP, s = i / DHP;
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[t][j] = keep(v[t][j], 8 * s + j < nrows);
+            const Bf3 p = bf3_split(v[t]);
+            dst[d * KSLOT + s] = p.hi;
+            dst[(DHP + d) * KSLOT + s] = p.mid;
+            dst[(2 * DHP + d) * KSLOT + s] = p.lo;
+        }
+    }
+    __device__ __forceinline__ static Bf3 frag(const u32x4 *src, int d, int s) {
+        return Bf3{src[d * KSLOT + s], src[(DHP + d) * KSLOT + s], src[(2 * DHP + d) * KSLOT + s]};
+    }
+};
+
+template <int DHP>
+constexpr size_t bwd_long_k_bytes() {
+    return (size_t)2 * 3 * DHP * KSLOT * 16;
+}
+
 // Core::backward's key half for the same shapes: dV = P^T dO and
 // dK = (tau dS)^T Q over the (image, head)'s queries, set or added (ACC);
-// wave w on keys [TK/4 w, TK/4 (w + 1)), 16 at a time, as attn_bwd_kernel's
-// phase 2: dO^T and Q^T staged in LDS, the A operands (P and tau dS for the
-// lane's key and four queries) read from HBM.
+// wave w on keys [TK/4 w, TK/4 (w + 1)), 16 at a time.  The products run on
+// the bf16 matrix cores (mfma_split.h; 28 us of a 37.1 us launch at 128 images,
+// 4 heads, 64 x 256 tokens, dh 64 were fp32 MFMAs; 34.4 us this way, its 151
+// MB at 4.4 TB/s of the 4.9 that a copy reaches): dO^T and Q^T split once into LDS, the A operands (P and tau dS for
+// the lane's key and eight queries a k step of 32) read from HBM a key tile
+// ahead and split in registers, the smaller part products in accumulators of
+// their own.
 template <int DHP, int NT, bool ACC>
 __global__ __launch_bounds__(256) void attn_bwd_long_k_kernel(AttnArgs g,
                                                               const float *__restrict__ s2) {
     constexpr int NDT = DHP / 16, TK = 16 * NT, KPW = NT / 4;  // key tiles a wave
+    using T = SplitTile<DHP>;
     extern __shared__ float smem[];
-    float *Qt = smem;            // [DHP][TS]
-    float *Ot = Qt + DHP * TS;   // [DHP][TS] dO^T
+    u32x4 *Ot = reinterpret_cast<u32x4 *>(smem), *Qt = Ot + 3 * DHP * KSLOT;
     const int tid = threadIdx.x, lane = tid & 63, w = wave_index();
     const int l16 = lane & 15, grp = lane >> 4;
     const int img = blockIdx.x / g.h, hd = blockIdx.x % g.h;
     const int tq = g.tq, dh = g.dh, c = g.h * dh;
-    const int QT = (tq + 15) >> 4;
     const float *qb = g.q + (long long)img * tq * g.qstride + g.qoff + (long long)hd * dh;
     const float *ob = g.dout + (long long)img * tq * c + (long long)hd * dh;
     float *dki = g.dkv + (long long)img * TK * g.kvstride + g.koff + (long long)hd * dh;
     float *dvi = g.dkv + (long long)img * TK * g.kvstride + g.voff + (long long)hd * dh;
     const long long prow = ((long long)img * g.h + hd) * tq;
     const float *pb = g.p + prow * TK, *sb = s2 + prow * TK;
-    Tile<DHP> ot, qt;
-    ot.template load<true>(ob, c, tq, dh, tid);
-    qt.template load<true>(qb, g.qstride, tq, dh, tid);
-    ot.template store<true>(Ot, tq, dh, tid);
-    qt.template store<true>(Qt, tq, dh, tid);
+    T ot, qt;
+    ot.load(ob, c, tq, tid);
+    qt.load(qb, g.qstride, tq, tid);
+    // the lane's key of tile kt, queries 32 u + 8 grp + j (rows past tq read
+    // row tq - 1 and are zeroed)
+    float pn[2][8], sn[2][8];
+    auto ahead = [&](int kt) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const long long o = (long long)min(32 * u + 8 * grp + j, tq - 1) * TK +
+                                    16 * (KPW * w + kt) + l16;
+                pn[u][j] = pb[o];
+                sn[u][j] = sb[o];
+            }
+    };
+    ahead(0);
+    ot.store(Ot, tq, tid);
+    qt.store(Qt, tq, tid);
     __syncthreads();
 #pragma unroll 1
     for (int kt = 0; kt < KPW; kt++) {
-        const int k0 = 16 * (KPW * w + kt), kr = k0 + l16, r0 = k0 + 4 * grp;
+        const int k0 = 16 * (KPW * w + kt), r0 = k0 + 4 * grp;
         float ov[NDT][4], ok[NDT][4];
         if constexpr (ACC) {
 #pragma unroll
@@ -967,53 +1027,77 @@ __global__ __launch_bounds__(256) void attn_bwd_long_k_kernel(AttnArgs g,
                 old4(ok[dt], dki, g.kvstride, r0, TK, 16 * dt + l16, dh);
             }
         }
-        // the lane's key, queries 16 ta + 4 grp + v (rows past tq read row
-        // tq - 1 and are zeroed)
-        float pa[4][4], sa[4][4];
+        Bf3 fp[2], fs[2];
 #pragma unroll
-        for (int ta = 0; ta < 4; ta++)
+        for (int u = 0; u < 2; u++) {
+            float x[8], y[8];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int q = 16 * ta + 4 * grp + v;
-                const long long o = (long long)min(q, tq - 1) * TK + kr;
-                pa[ta][v] = pb[o];
-                sa[ta][v] = sb[o];
+            for (int j = 0; j < 8; j++) {
+                const bool live = 32 * u + 8 * grp + j < tq;
+                x[j] = keep(pn[u][j], live);
+                y[j] = keep(sn[u][j], live);
             }
-        f32x4 av[NDT], ak[NDT];
+            fp[u] = bf3_split_near(x);
+            fs[u] = bf3_split_near(y);
+        }
+        if (kt + 1 < KPW) ahead(kt + 1);
+        f32x4 av[NDT][2], ak[NDT][2];  // [1]: the smaller part products
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) av[dt][s] = ak[dt][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (32 * u >= tq) break;
+#pragma unroll
+            for (int d2 = 0; d2 < NDT; d2 += 2) {  // two head-dim tiles: four chains
+                Bf3 fo[2], fq[2];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    fo[e] = T::frag(Ot, 16 * (d2 + e) + l16, 4 * u + grp);
+                    fq[e] = T::frag(Qt, 16 * (d2 + e) + l16, 4 * u + grp);
+                }
+                bf3_products([&](auto pick, auto kind) {
+                    constexpr int s = decltype(kind)::value;
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        av[d2 + e][s] = pick(fp[u], fo[e], av[d2 + e][s]);
+                        ak[d2 + e][s] = pick(fs[u], fq[e], ak[d2 + e][s]);
+                    }
+                });
+            }
+        }
+        bool bad = false;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
-            av[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            ak[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            av[dt][0] += av[dt][1];
+            ak[dt][0] += ak[dt][1];
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                bad = bad || bf3_nonfinite(av[dt][0][v]) || bf3_nonfinite(ak[dt][0][v]);
         }
-#pragma unroll
-        for (int ta = 0; ta < 4; ta++) {
-            if (ta >= QT) break;
-            const int q0 = 16 * ta + 4 * grp;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                pa[ta][v] = keep(pa[ta][v], q0 + v < tq);
-                sa[ta][v] = keep(sa[ta][v], q0 + v < tq);
-            }
+        if (__any(bad)) {  // values that have no split: again with fp32 MFMAs
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
                 const int d = 16 * dt + l16;
-                const float4 ob4 = lds4(Ot + d * TS + q0);
-                const float4 qb4 = lds4(Qt + d * TS + q0);
-                av[dt] = mfma16(pa[ta][0], ob4.x, av[dt]);
-                ak[dt] = mfma16(sa[ta][0], qb4.x, ak[dt]);
-                av[dt] = mfma16(pa[ta][1], ob4.y, av[dt]);
-                ak[dt] = mfma16(sa[ta][1], qb4.y, ak[dt]);
-                av[dt] = mfma16(pa[ta][2], ob4.z, av[dt]);
-                ak[dt] = mfma16(sa[ta][2], qb4.z, ak[dt]);
-                av[dt] = mfma16(pa[ta][3], ob4.w, av[dt]);
-                ak[dt] = mfma16(sa[ta][3], qb4.w, ak[dt]);
+                av[dt][0] = ak[dt][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int q0 = 0; q0 < tq; q0 += 4) {
+                    const int q = q0 + grp;
+                    const long long qc = min(q, tq - 1);
+                    const bool live = q < tq;
+                    av[dt][0] = mfma16(keep(pb[qc * TK + k0 + l16], live),
+                                       keep(ob[qc * c + d], live), av[dt][0]);
+                    ak[dt][0] = mfma16(keep(sb[qc * TK + k0 + l16], live),
+                                       keep(qb[qc * g.qstride + d], live), ak[dt][0]);
+                }
             }
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
             const int d = 16 * dt + l16;
-            store4<ACC>(dvi, g.kvstride, r0, TK, d, dh, ov[dt], av[dt], 1.0f);
-            store4<ACC>(dki, g.kvstride, r0, TK, d, dh, ok[dt], ak[dt], 1.0f);
+            store4<ACC>(dvi, g.kvstride, r0, TK, d, dh, ov[dt], av[dt][0], 1.0f);
+            store4<ACC>(dki, g.kvstride, r0, TK, d, dh, ok[dt], ak[dt][0], 1.0f);
         }
     }
 }
@@ -1512,7 +1596,7 @@ LongBwd bwd_long_kernels(const rnn_attn_desc *d, bool vec, bool acc_q, bool acc_
     r.kk = acc_kv ? (const void *)attn_bwd_long_k_kernel<DH_, NT_, true>                        \
                   : (const void *)attn_bwd_long_k_kernel<DH_, NT_, false>;                      \
     words = bwd_long_words<DH_, NT_>();                                                         \
-    r.klds = (size_t)2 * DH_ * TS * 4;
+    r.klds = bwd_long_k_bytes<DH_>();
     if (d->dh == 64 && d->tk == 256) {
         RNN_LONG_PAIR(64, 16)
     } else if (d->dh == 64) {

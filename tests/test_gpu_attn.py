@@ -202,3 +202,42 @@ def test_attn_unsupported_shape_raises(rnn, orc):
     with pytest.raises(rnn.RnnError):
         core.forward(1, q, 80, 0, kv, 160, 0, 80, to_dev(np.ones(1, np.float32)),
                      to_dev(np.zeros(nrel, np.float32)))
+
+
+# The long-key backward's key half: one query, a whole k step of 32, one more,
+# a partial second one; an infinity and a NaN in dO (which have no split).
+@pytest.mark.parametrize("h,dh,th,tw,mh,mw,acc,special", [
+    (2, 64, 1, 1, 16, 16, False, False), (3, 32, 4, 8, 8, 16, True, False),
+    (2, 64, 3, 11, 16, 16, False, False), (1, 64, 7, 9, 8, 16, True, False),
+    (3, 32, 5, 6, 16, 16, False, False), (2, 64, 8, 8, 16, 16, False, True),
+    (2, 32, 5, 8, 8, 16, True, True)])
+def test_attn_long_key_gradients(rnn, h, dh, th, tw, mh, mw, acc, special):
+    import torch
+    n, tq, tk, c = 3, th * tw, mh * mw, h * dh
+    idx, nrel = rnn.rel_index(th, tw, mh, mw)
+    core = rnn.Core(h, dh, tq, tk, idx, nrel, False)
+    gen = torch.Generator(device="cuda").manual_seed(tq + tk)
+    rnd = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+    q, kv, do = rnd(n, tq, c), rnd(n, tk, 2 * c), rnd(n, tq, c)
+    tau, rel = torch.full((h,), dh ** -0.5, device="cuda"), rnd(h * nrel) * 0.2
+    if special:
+        do[0, tq - 1, 1], do[1, 0, c - 1] = float("inf"), float("nan")
+    lay = (c, 0, kv, 2 * c, 0, c)
+    p, _ = core.forward(n, q, *lay, tau, rel)
+    dq, dtau, drel = torch.zeros_like(q), torch.zeros_like(tau), torch.zeros_like(rel)
+    dkv = torch.full_like(kv, 1.0 if acc else float("nan"))
+    core.backward(n, q, *lay, tau, p, do, dq, dkv, dtau, drel, set_dkv=not acc)
+    heads = lambda t, at: t[..., at:at + c].reshape(n, -1, h, dh).transpose(1, 2).double()
+    P, O, Q = p.view(n, h, tq, tk).double(), heads(do, 0), heads(q, 0)
+    dp = O @ heads(kv, c).transpose(2, 3).contiguous()
+    ds = P * (dp - (P * dp).sum(-1, keepdim=True)) * tau.view(1, h, 1, 1)
+    for at, a, b in ((c, P, O), (0, ds, Q)):
+        got = to_host(heads(dkv, at)) - (1.0 if acc else 0.0)
+        want = to_host(a.transpose(2, 3).contiguous() @ b)
+        fine = np.isfinite(want)
+        assert np.array_equal(got[~fine], want[~fine], equal_nan=True)
+        # sums of tq rounded products, each rounding 2^-24 of a partial sum; dS
+        # from a dP of dh such terms; the added 1 is far larger than dK
+        tol = 2.0 ** -24 * (np.sqrt(tq) + 4 * np.sqrt(dh) + 8)
+        size = np.linalg.norm(want[fine]) + (np.sqrt(fine.sum()) if acc else 0.0)
+        assert np.linalg.norm(got[fine] - want[fine]) < tol * size
