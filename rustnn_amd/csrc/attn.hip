@@ -293,22 +293,206 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs g) {
     }
 }
 
+// K (or V) of one (image, head) for the long-key kernels, TK keys in halves of
+// 128 staged one after the other in LDS as their three bf16 parts
+// (mfma_split.h), split once for all four waves: two workgroups' halves fit a
+// CU.  A thread holds both halves in registers from their loads on.
+//   * rows: [part][key][DHP/8 + 1 slots of 8 head dims], the A operand of the
+//     products over head dims;
+//   * columns: [part][head dim][16 + 1 slots of 8 keys], slot 4u + g with keys
+//     32u + 4g + {0..3, 16..19}: lane group g's P (or dS) registers of key
+//     tiles 2u and 2u + 1 are the other operand.
+// The slot of padding puts 16 consecutive rows' b128 reads on distinct banks.
+template <int DHP, int NT>
+struct LongTile {
+    static constexpr int HK = 128, NH = NT / 8;  // keys of a half, halves
+    static constexpr int G = DHP / 4, CPH = HK * G / 256, RS = DHP / 8 + 1, CS = HK / 8 + 1;
+    static constexpr size_t WORDS = (size_t)3 * 4 * (HK * RS > DHP * CS ? HK * RS : DHP * CS);
+    float v[NH][4 * CPH];
+
+    __device__ __forceinline__ void load_rows(int hh, const float *src, long long stride, int tid) {
+#pragma unroll
+        for (int j = 0; j < CPH; j++) {
+            const int i = tid + 256 * j;
+            const float4 x = *reinterpret_cast<const float4 *>(
+                src + (long long)(HK * hh + i / G) * stride + (i % G) * 4);
+            v[hh][4 * j] = x.x;
+            v[hh][4 * j + 1] = x.y;
+            v[hh][4 * j + 2] = x.z;
+            v[hh][4 * j + 3] = x.w;
+        }
+    }
+    __device__ __forceinline__ void store_rows(int hh, float *lds, int tid) const {
+#pragma unroll
+        for (int j = 0; j < CPH; j++) {
+            const int i = tid + 256 * j;
+            const float *x = &v[hh][4 * j];
+            uint2 *d = reinterpret_cast<uint2 *>(lds) + (i / G) * RS * 2 + i % G;
+            float r[4], q[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                r[e] = bf3_rest(x[e]);
+                q[e] = bf3_rest(r[e]);
+            }
+            d[0] = make_uint2(bf3_top2(x[0], x[1]), bf3_top2(x[2], x[3]));
+            d[HK * RS * 2] = make_uint2(bf3_top2(r[0], r[1]), bf3_top2(r[2], r[3]));
+            d[2 * HK * RS * 2] = make_uint2(bf3_top2(q[0], q[1]), bf3_top2(q[2], q[3]));
+        }
+    }
+    __device__ __forceinline__ void load_cols(int hh, const float *src, long long stride, int tid) {
+#pragma unroll
+        for (int t = 0; t < CPH / 2; t++) {
+            const int i = tid + 256 * t, d = i % DHP, sl = i / DHP;
+            const int k = HK * hh + 32 * (sl >> 2) + 4 * (sl & 3);
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[hh][8 * t + e] = src[(long long)(k + (e & 3) + 16 * (e >> 2)) * stride + d];
+        }
+    }
+    __device__ __forceinline__ void store_cols(int hh, float *lds, int tid) const {
+        u32x4 *w = reinterpret_cast<u32x4 *>(lds);
+#pragma unroll
+        for (int t = 0; t < CPH / 2; t++) {
+            const int i = tid + 256 * t, d = i % DHP, sl = i / DHP;
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = v[hh][8 * t + e];
+            const Bf3 p = bf3_split(x);
+            w[d * CS + sl] = p.hi;
+            w[(DHP + d) * CS + sl] = p.mid;
+            w[(2 * DHP + d) * CS + sl] = p.lo;
+        }
+    }
+    // Head dims 8 (4u + g) .. of key row `row` of the half.
+    __device__ __forceinline__ static Bf3 row(const float *lds, int row, int sl) {
+        const u32x4 *w = reinterpret_cast<const u32x4 *>(lds) + row * RS + sl;
+        return Bf3{w[0], w[HK * RS], w[2 * HK * RS]};
+    }
+    __device__ __forceinline__ static Bf3 col(const float *lds, int d, int sl) {
+        const u32x4 *w = reinterpret_cast<const u32x4 *>(lds) + d * CS + sl;
+        return Bf3{w[0], w[DHP * CS], w[2 * DHP * CS]};
+    }
+
+    // The lane's operand of the products over head dims: row `r` of src (zero
+    // unless live), head dims 32u + 8g + 0..7.
+    __device__ __forceinline__ static void lane_row(const float *src, bool live, int grp,
+                                                    Bf3 (&f)[DHP / 32]) {
+#pragma unroll
+        for (int u = 0; u < DHP / 32; u++) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const float4 t = *reinterpret_cast<const float4 *>(src + 32 * u + 8 * grp + 4 * e);
+                x[4 * e] = keep(t.x, live);
+                x[4 * e + 1] = keep(t.y, live);
+                x[4 * e + 2] = keep(t.z, live);
+                x[4 * e + 3] = keep(t.w, live);
+            }
+            f[u] = bf3_split_near(x);
+        }
+    }
+    // out[t] = rows of key tile t times the lane's row, for the half's tiles.
+    __device__ __forceinline__ static void times_rows(const float *lds, int hh, int l16, int grp,
+                                                      const Bf3 (&f)[DHP / 32],
+                                                      f32x4 (&out)[NT]) {
+#pragma unroll
+        for (int t = 0; t < 8; t += 2) {
+            f32x4 c[2][2];
+#pragma unroll
+            for (int e = 0; e < 4; e++) c[e >> 1][e & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < DHP / 32; u++) {
+                const Bf3 a0 = row(lds, 16 * t + l16, 4 * u + grp);
+                const Bf3 a1 = row(lds, 16 * (t + 1) + l16, 4 * u + grp);
+                bf3_products([&](auto pick, auto kind) {
+                    constexpr int k = decltype(kind)::value;
+                    c[0][k] = pick(a0, f[u], c[0][k]);
+                    c[1][k] = pick(a1, f[u], c[1][k]);
+                });
+            }
+            out[8 * hh + t] = c[0][0] + c[0][1];
+            out[8 * hh + t + 1] = c[1][0] + c[1][1];
+        }
+    }
+    // acc[dt] += st (the lane's row, the half's keys) times columns 16 dt ..;
+    // acc[dt][1] the smaller part products.
+    __device__ __forceinline__ static void times_cols(const float *lds, int hh, int l16, int grp,
+                                                      const f32x4 (&st)[NT],
+                                                      f32x4 (&acc)[DHP / 16][2]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = st[8 * hh + 2 * u + (e >> 2)][e & 3];
+            const Bf3 a = bf3_split_near(x);
+#pragma unroll
+            for (int d2 = 0; d2 < DHP / 16; d2 += 2) {
+                const Bf3 b0 = col(lds, 16 * d2 + l16, 4 * u + grp);
+                const Bf3 b1 = col(lds, 16 * (d2 + 1) + l16, 4 * u + grp);
+                bf3_products([&](auto pick, auto kind) {
+                    constexpr int k = decltype(kind)::value;
+                    acc[d2][k] = pick(a, b0, acc[d2][k]);
+                    acc[d2 + 1][k] = pick(a, b1, acc[d2 + 1][k]);
+                });
+            }
+        }
+    }
+    // The same products with fp32 MFMAs from global memory, for values that
+    // have no split: src the [TK] rows, x the lane's row.
+    __device__ __forceinline__ static void slow_rows(const float *src, long long stride,
+                                                     const float *x, bool live, int l16, int grp,
+                                                     f32x4 (&out)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            out[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = grp; k < DHP + grp; k += 4)
+                out[t] = mfma16(src[(long long)(16 * t + l16) * stride + k], keep(x[k], live),
+                                out[t]);
+        }
+    }
+    __device__ __forceinline__ static void slow_cols(const float *src, long long stride, int l16,
+                                                     int grp, const f32x4 (&st)[NT],
+                                                     f32x4 (&acc)[DHP / 16][2]) {
+#pragma unroll
+        for (int dt = 0; dt < DHP / 16; dt++) {
+            acc[dt][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[dt][0] = mfma16(
+                        st[t][v],
+                        src[(long long)(16 * t + 4 * grp + v) * stride + 16 * dt + l16],
+                        acc[dt][0]);
+        }
+    }
+    template <int N>
+    __device__ __forceinline__ static bool nonfinite(const f32x4 (&x)[N]) {
+        bool bad = false;
+#pragma unroll
+        for (int t = 0; t < N; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) bad = bad || bf3_nonfinite(x[t][v]);
+        return __any(bad);
+    }
+};
+
 // Core::forward for tq <= 64 and tk = 16 NT keys above 64 (the rustvit's
 // cross-attention over 256 memory tokens), one workgroup per (image, head),
-// as attn_fwd_kernel with float4 accesses: K rows staged in LDS [tk][DHP+4];
-// V loaded into registers while the scores run and stored transposed
-// ([DHP][tk+4]) over the K rows once every wave is done with them; the
-// relidx entries of the lane's query and keys read from the composed path's
-// [tq][tk] table.  Two workgroups fit a CU.
+// wave w on queries [16w, 16w + 16) as attn_fwd_kernel; both products on the
+// bf16 matrix cores (LongTile; on fp32 MFMAs, which took 28 us of it, 128
+// images, 4 heads, 64 x 256 tokens, dh 64 41.9 us, so 33.3: the loads, 117 MB
+// in 24 us at a copy's rate, and what of the products they do not hide).  V's loads go out as K's halves are stored, so
+// that they overlap the scores; the relidx entries of the lane's query and
+// keys are read from the composed path's [tq][tk] table.
 template <int DHP, int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
 attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
-    constexpr int KSL = DHP / 4, TK = 16 * NT, KS = DHP + 4, VS = TK + 4;
-    constexpr int AW = TK * KS > DHP * VS ? TK * KS : DHP * VS;
-    constexpr int G = DHP / 4, CPT = TK * G / 256;  // float4 chunks of K (or V) per thread
+    constexpr int TK = 16 * NT;
+    using T = LongTile<DHP, NT>;
     extern __shared__ float smem[];
-    float *A = smem;          // K rows [TK][KS], then V^T [DHP][VS]
-    float *rels = smem + AW;  // [nrel]
+    float *rels = smem + T::WORDS;  // [nrel]
     const int tid = threadIdx.x, lane = tid & 63, w = wave_index();
     const int l16 = lane & 15, grp = lane >> 4;
     const int img = blockIdx.x / g.h, hd = blockIdx.x % g.h;
@@ -317,61 +501,31 @@ attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
     const float *kb = g.kv + (long long)img * TK * g.kvstride + g.koff + (long long)hd * dh;
     const float *vb = g.kv + (long long)img * TK * g.kvstride + g.voff + (long long)hd * dh;
     const int qi = 16 * w + l16;
+    const bool qlive = qi < tq;
     const float tau = g.tau[hd];
-    float4 qraw[KSL / 4];
+    const float *qr = qb + (long long)min(qi, tq - 1) * g.qstride;
+    T kv;
 #pragma unroll
-    for (int i = 0; i < KSL; i += 4)
-        qraw[i / 4] = load4<true>(qb, g.qstride, qi, tq, grp * KSL + i, dh);
+    for (int hh = 0; hh < T::NH; hh++) kv.load_rows(hh, kb, g.kvstride, tid);
+    Bf3 qf[DHP / 32];
+    T::lane_row(qr, qlive, grp, qf);
+    const float *relh = g.rel + (long long)hd * g.nrel;
+    for (int e = tid; e < g.nrel; e += 256) rels[e] = relh[e];
     const uint32_t *rq = relidx + (long long)min(qi, tq - 1) * TK + 4 * grp;
     uint4 ri[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) ri[t] = *reinterpret_cast<const uint4 *>(rq + 16 * t);
-    float4 kv4[CPT];
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, c = (i % G) * 4;
-        kv4[j] = load4<true>(kb, g.kvstride, r, TK, c, dh);
-    }
-    const float *relh = g.rel + (long long)hd * g.nrel;
-    const float rel0 = relh[min(tid, g.nrel - 1)];
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, c = (i % G) * 4;
-        *reinterpret_cast<float4 *>(A + r * KS + c) = kv4[j];
-    }
-    // V next: only O = P V needs it, so its latency overlaps the scores
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, c = (i % G) * 4;
-        kv4[j] = load4<true>(vb, g.kvstride, r, TK, c, dh);
-    }
-    if (tid < g.nrel) rels[tid] = rel0;
-    for (int e = tid + 256; e < g.nrel; e += 256) rels[e] = relh[e];
-    __syncthreads();
-
-    float qs[KSL];
-#pragma unroll
-    for (int i = 0; i < KSL; i += 4) {
-        const float4 t4 = mask4(qraw[i / 4], qi < tq, grp * KSL + i, dh);
-        qs[i] = t4.x;
-        qs[i + 1] = t4.y;
-        qs[i + 2] = t4.z;
-        qs[i + 3] = t4.w;
-    }
     f32x4 st[NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        st[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const float *kr = A + (16 * t + l16) * KS + grp * KSL;
+    for (int hh = 0; hh < T::NH; hh++) {
+        if (hh) __syncthreads();  // every wave is done with the half before
+        kv.store_rows(hh, smem, tid);
+        if (hh == 0)
 #pragma unroll
-        for (int s = 0; s < KSL; s += 4) {
-            const float4 a = lds4(kr + s);
-            st[t] = mfma16(a.x, qs[s], st[t]);
-            st[t] = mfma16(a.y, qs[s + 1], st[t]);
-            st[t] = mfma16(a.z, qs[s + 2], st[t]);
-            st[t] = mfma16(a.w, qs[s + 3], st[t]);
-        }
+            for (int t = 0; t < NT; t++) ri[t] = *reinterpret_cast<const uint4 *>(rq + 16 * t);
+        kv.load_cols(hh, vb, g.kvstride, tid);
+        __syncthreads();
+        T::times_rows(smem, hh, l16, grp, qf, st);
     }
+    if (T::nonfinite(st)) T::slow_rows(kb, g.kvstride, qr, qlive, l16, grp, st);
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < NT; t++) {
@@ -396,7 +550,6 @@ attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
     const float inv = 1.0f / sum;
-    const bool qlive = qi < tq;
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -408,37 +561,34 @@ attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
             *reinterpret_cast<float4 *>(pr + 16 * t) =
                 make_float4(st[t][0], st[t][1], st[t][2], st[t][3]);
     }
-    __syncthreads();  // every wave is done with the K rows
+    f32x4 acc[DHP / 16][2];
 #pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, c = (i % G) * 4;
-        A[(c + 0) * VS + r] = kv4[j].x;
-        A[(c + 1) * VS + r] = kv4[j].y;
-        A[(c + 2) * VS + r] = kv4[j].z;
-        A[(c + 3) * VS + r] = kv4[j].w;
+    for (int dt = 0; dt < DHP / 16; dt++)
+        acc[dt][0] = acc[dt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int hh = 0; hh < T::NH; hh++) {
+        __syncthreads();  // every wave is done with K, or V's half before
+        kv.store_cols(hh, smem, tid);
+        __syncthreads();
+        T::times_cols(smem, hh, l16, grp, st, acc);
     }
-    __syncthreads();
+    f32x4 o[DHP / 16];
+#pragma unroll
+    for (int dt = 0; dt < DHP / 16; dt++) o[dt] = acc[dt][0] + acc[dt][1];
+    if (T::nonfinite(o)) {
+        T::slow_cols(vb, g.kvstride, l16, grp, st, acc);
+#pragma unroll
+        for (int dt = 0; dt < DHP / 16; dt++) o[dt] = acc[dt][0];
+    }
     const int c = g.h * dh;
     float *od = g.o + (long long)img * tq * c + (long long)hd * dh;
 #pragma unroll
-    for (int dt = 0; dt < DHP / 16; dt++) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        const float *vr = A + (16 * dt + l16) * VS + 4 * grp;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const float4 b = lds4(vr + 16 * t);
-            acc = mfma16(st[t][0], b.x, acc);
-            acc = mfma16(st[t][1], b.y, acc);
-            acc = mfma16(st[t][2], b.z, acc);
-            acc = mfma16(st[t][3], b.w, acc);
-        }
-        const int d = 16 * dt + l16;
+    for (int dt = 0; dt < DHP / 16; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int q = 16 * w + 4 * grp + v;
-            if (q < tq) od[(long long)q * c + d] = acc[v];
+            if (q < tq) od[(long long)q * c + 16 * dt + l16] = o[dt][v];
         }
-    }
 }
 
 template <int DHP, int NT>
@@ -450,8 +600,7 @@ constexpr size_t bwd_long_words() {
 
 template <int DHP, int NT>
 constexpr size_t fwd_long_words() {
-    return (size_t)((16 * NT) * (DHP + 4) > DHP * (16 * NT + 4) ? (16 * NT) * (DHP + 4)
-                                                               : DHP * (16 * NT + 4));
+    return LongTile<DHP, NT>::WORDS;
 }
 
 // dst[r][d] = old[v] + scale * val[v] (ACC) or scale * val[v] for the 4

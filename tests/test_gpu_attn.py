@@ -241,3 +241,37 @@ def test_attn_long_key_gradients(rnn, h, dh, th, tw, mh, mw, acc, special):
         tol = 2.0 ** -24 * (np.sqrt(tq) + 4 * np.sqrt(dh) + 8)
         size = np.linalg.norm(want[fine]) + (np.sqrt(fine.sum()) if acc else 0.0)
         assert np.linalg.norm(got[fine] - want[fine]) < tol * size
+
+
+# The long-key forward: one query, a query past a wave's 16, a partial last
+# wave; infinities and a NaN in K and V (which have no split).
+@pytest.mark.parametrize("h,dh,th,tw,mh,mw,special", [
+    (2, 64, 1, 1, 16, 16, False), (3, 32, 3, 6, 8, 16, False), (1, 64, 7, 9, 8, 16, False),
+    (3, 32, 8, 8, 16, 16, False), (2, 64, 8, 8, 16, 16, True), (2, 32, 5, 8, 8, 16, True)])
+def test_attn_long_key_forward(rnn, h, dh, th, tw, mh, mw, special):
+    import torch
+    n, tq, tk, c = 3, th * tw, mh * mw, h * dh
+    idx, nrel = rnn.rel_index(th, tw, mh, mw)
+    core = rnn.Core(h, dh, tq, tk, idx, nrel, False)
+    gen = torch.Generator(device="cuda").manual_seed(tq + tk)
+    rnd = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+    q, kv = rnd(n, tq, c), rnd(n, tk, 2 * c)
+    if special:
+        kv[0, tk - 3, 5], kv[1, 2, c + 1] = float("inf"), float("-inf")
+        kv[2, tk - 1, 2 * c - 1] = float("nan")
+    tau, rel = torch.full((h,), dh ** -0.5, device="cuda"), rnd(h * nrel) * 0.2
+    p, o = core.forward(n, q, c, 0, kv, 2 * c, 0, c, tau, rel)
+    heads = lambda t, at: t[..., at:at + c].reshape(n, -1, h, dh).transpose(1, 2).double()
+    s = heads(q, 0) @ heads(kv, 0).transpose(2, 3).contiguous() * tau.view(1, h, 1, 1)
+    bias = rel.view(h, nrel)[:, torch.as_tensor(np.asarray(idx).astype(np.int64), device="cuda")]
+    want_p = torch.softmax(s + bias.view(1, h, tq, tk), -1)
+    want_o = want_p @ heads(kv, c)
+    # scores of size 6 at most, each term's and sum's rounding 2^-24 of it; the
+    # exponential carries them into P, the sums over keys add 2^-24 sqrt(tk)
+    tol = 2.0 ** -24 * (np.sqrt(dh) + np.sqrt(tk) + 6 * 8)
+    for got, want in ((p.view(n, h, tq, tk), want_p), (o.reshape(n, tq, h, dh).transpose(1, 2),
+                                                       want_o)):
+        got, want = to_host(got), to_host(want)
+        fine = np.isfinite(want)
+        assert np.array_equal(got[~fine], want[~fine], equal_nan=True)
+        assert np.linalg.norm(got[fine] - want[fine]) < tol * np.linalg.norm(want[fine])
