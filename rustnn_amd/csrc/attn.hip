@@ -592,10 +592,8 @@ attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
 }
 
 template <int DHP, int NT>
-constexpr size_t bwd_long_words() {
-    return (size_t)(16 * NT) * (DHP + 4) > (size_t)DHP * (16 * NT + 4)
-               ? std::max<size_t>((size_t)(16 * NT) * (DHP + 4), (size_t)MAXT * 16 * NT)
-               : std::max<size_t>((size_t)DHP * (16 * NT + 4), (size_t)MAXT * 16 * NT);
+constexpr size_t bwd_long_words() {  // the staged half, or dS [64][tk]
+    return std::max<size_t>(LongTile<DHP, NT>::WORDS, (size_t)MAXT * 16 * NT);
 }
 
 template <int DHP, int NT>
@@ -890,24 +888,26 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel(AttnArgs g) {
 
 // Core::backward's query half for tq <= 64 and tk = 16 NT keys above 64
 // (the rustvit's cross-attention), one workgroup per (image, head), wave w
-// on queries [16w, 16w + 16) as in attn_bwd_kernel's phase 1: dP^T = V dO^T
-// with V's rows in LDS; dS = P o (dP - <dP, P>), with tau dS written to s2
-// ([tq][tk] per (image, head)) for the key half (attn_bwd_long_k_kernel);
-// then dSK = dS K with K^T in LDS over V's rows (K held in registers
-// meanwhile); dQ = tau dSK, set or added (ACC); the (image, head) shares of
-// dtau (sum Q . dSK, f64) and of drel (dS staged in LDS [tq][tk] over K^T and
+// on queries [16w, 16w + 16) as in attn_bwd_kernel's phase 1, its products on
+// the bf16 matrix cores (LongTile; on fp32 MFMAs 50.0 us at 128 images, 4
+// heads, 64 x 256 tokens, dh 64, so 46.0, its 158 MB being 32 us of a copy):
+// dP^T = V dO^T with V's rows in LDS;
+// dS = P o (dP - <dP, P>), with tau dS written to s2 ([tq][tk] per (image,
+// head)) for the key half (attn_bwd_long_k_kernel); then dSK = dS K with K's
+// columns in LDS (K in registers meanwhile, its loads out as V's halves are
+// stored); dQ = tau dSK, set or added (ACC); the (image, head) shares of
+// dtau (sum Q . dSK, f64) and of drel (dS staged in LDS [tq][tk] over K and
 // gathered through the inverse index, each slot's positions in ascending
 // order) into g.dtau_part / g.drel_part.
 template <int DHP, int NT, bool ACC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
 attn_bwd_long_q_kernel(AttnArgs g, float *__restrict__ s2) {
-    constexpr int KSL = DHP / 4, NDT = DHP / 16, TK = 16 * NT, KS = DHP + 4, VS = TK + 4;
-    constexpr int AW0 = TK * KS > DHP * VS ? TK * KS : DHP * VS;
-    constexpr int AW = AW0 > MAXT * TK ? AW0 : MAXT * TK;  // also dS [64][tk]
-    constexpr int G = DHP / 4, CPT = TK * G / 256;
+    constexpr int NDT = DHP / 16, TK = 16 * NT;
+    using T = LongTile<DHP, NT>;
+    constexpr int AW = T::WORDS > (size_t)MAXT * TK ? (int)T::WORDS : MAXT * TK;
     static_assert(AW % 2 == 0, "8-byte aligned reduction slots");
     extern __shared__ float smem[];
-    float *A = smem;                                         // V rows, then K^T
+    float *A = smem;                                         // V, then K, then dS
     double *dred = reinterpret_cast<double *>(smem + AW);    // [4]
     const int tid = threadIdx.x, lane = tid & 63, w = wave_index();
     const int l16 = lane & 15, grp = lane >> 4;
@@ -922,61 +922,30 @@ attn_bwd_long_q_kernel(AttnArgs g, float *__restrict__ s2) {
     const bool qlive = qi < tq;
     const float tau = g.tau[hd];
     const long long prow = ((long long)img * g.h + hd) * tq;
+    const float *orow = ob + (long long)min(qi, tq - 1) * c;
 
+    T kv;
+#pragma unroll
+    for (int hh = 0; hh < T::NH; hh++) kv.load_rows(hh, vb, g.kvstride, tid);
+    Bf3 of[DHP / 32];
+    T::lane_row(orow, qlive, grp, of);
     float4 pv4[NT];
-    {
-        const float *pr = g.p + (prow + min(qi, tq - 1)) * TK + 4 * grp;
-#pragma unroll
-        for (int t = 0; t < NT; t++) pv4[t] = *reinterpret_cast<const float4 *>(pr + 16 * t);
-    }
-    float4 oraw[KSL / 4];
-#pragma unroll
-    for (int i = 0; i < KSL; i += 4) oraw[i / 4] = load4<true>(ob, c, qi, tq, grp * KSL + i, dh);
-    float4 kv4[CPT];
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, cc = (i % G) * 4;
-        kv4[j] = load4<true>(vb, g.kvstride, r, TK, cc, dh);
-    }
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, cc = (i % G) * 4;
-        *reinterpret_cast<float4 *>(A + r * KS + cc) = kv4[j];
-    }
-    __syncthreads();
-
-    float os[KSL];
-#pragma unroll
-    for (int i = 0; i < KSL; i += 4) {
-        const float4 t4 = mask4(oraw[i / 4], qlive, grp * KSL + i, dh);
-        os[i] = t4.x;
-        os[i + 1] = t4.y;
-        os[i + 2] = t4.z;
-        os[i + 3] = t4.w;
-    }
-    // dP^T = V dO^T (attn.rs:272-278): the score-tile layout of P
     f32x4 dp[NT];
+    // dP^T = V dO^T (attn.rs:272-278): the score-tile layout of P
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        dp[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const float *vr = A + (16 * t + l16) * KS + grp * KSL;
+    for (int hh = 0; hh < T::NH; hh++) {
+        if (hh) __syncthreads();  // every wave is done with the half before
+        kv.store_rows(hh, A, tid);
+        if (hh == 0) {
+            const float *pr = g.p + (prow + min(qi, tq - 1)) * TK + 4 * grp;
 #pragma unroll
-        for (int s = 0; s < KSL; s += 4) {
-            const float4 a = lds4(vr + s);
-            dp[t] = mfma16(a.x, os[s], dp[t]);
-            dp[t] = mfma16(a.y, os[s + 1], dp[t]);
-            dp[t] = mfma16(a.z, os[s + 2], dp[t]);
-            dp[t] = mfma16(a.w, os[s + 3], dp[t]);
+            for (int t = 0; t < NT; t++) pv4[t] = *reinterpret_cast<const float4 *>(pr + 16 * t);
         }
+        kv.load_cols(hh, kb, g.kvstride, tid);
+        __syncthreads();
+        T::times_rows(A, hh, l16, grp, of, dp);
     }
-    // K next, once dO's slice is dead (the registers are scarce): only dS K
-    // needs it, so its latency overlaps dS and its stores
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, cc = (i % G) * 4;
-        kv4[j] = load4<true>(kb, g.kvstride, r, TK, cc, dh);
-    }
+    if (T::nonfinite(dp)) T::slow_rows(vb, g.kvstride, orow, qlive, l16, grp, dp);
     // dS = P o (dP - <dP, P>) (attn.rs:280-290)
     float pv[NT][4];
 #pragma unroll
@@ -1004,47 +973,47 @@ attn_bwd_long_q_kernel(AttnArgs g, float *__restrict__ s2) {
             *reinterpret_cast<float4 *>(d2 + 16 * t) =
                 make_float4(dp[t][0] * tau, dp[t][1] * tau, dp[t][2] * tau, dp[t][3] * tau);
     }
-    __syncthreads();  // every wave is done with V's rows
+    // dSK = dS K (attn.rs:316-323, before the tau scaling)
+    f32x4 acc[NDT][2];
 #pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int i = tid + 256 * j, r = i / G, cc = (i % G) * 4;
-        A[(cc + 0) * VS + r] = kv4[j].x;
-        A[(cc + 1) * VS + r] = kv4[j].y;
-        A[(cc + 2) * VS + r] = kv4[j].z;
-        A[(cc + 3) * VS + r] = kv4[j].w;
-    }
-    // Q (for dtau) and the old dQ: loaded late, the registers are scarce
+    for (int dt = 0; dt < NDT; dt++) acc[dt][0] = acc[dt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     float oq[NDT][4], qv[NDT][4];
 #pragma unroll
-    for (int dt = 0; dt < NDT; dt++) {
-        if constexpr (ACC) old4(oq[dt], dqi, g.qstride, r0, tq, 16 * dt + l16, dh);
+    for (int hh = 0; hh < T::NH; hh++) {
+        __syncthreads();  // every wave is done with V, or K's half before
+        kv.store_cols(hh, A, tid);
+        if (hh == T::NH - 1) {
+            // Q (for dtau) and the old dQ: loaded late, the registers are scarce
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-            qv[dt][v] = qb[(long long)min(r0 + v, tq - 1) * g.qstride + 16 * dt + l16];
+            for (int dt = 0; dt < NDT; dt++) {
+                if constexpr (ACC) old4(oq[dt], dqi, g.qstride, r0, tq, 16 * dt + l16, dh);
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    qv[dt][v] = qb[(long long)min(r0 + v, tq - 1) * g.qstride + 16 * dt + l16];
+            }
+        }
+        __syncthreads();
+        T::times_cols(A, hh, l16, grp, dp, acc);
     }
-    __syncthreads();
-    // dSK = dS K (attn.rs:316-323, before the tau scaling); dQ = tau dSK;
-    // dtau += Q . dSK
+    f32x4 dsk[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++) dsk[dt] = acc[dt][0] + acc[dt][1];
+    if (T::nonfinite(dsk)) {
+        T::slow_cols(kb, g.kvstride, l16, grp, dp, acc);
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) dsk[dt] = acc[dt][0];
+    }
+    // dQ = tau dSK; dtau += Q . dSK
     double tpart = 0.0;
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++) {
-        f32x4 dsk = {0.f, 0.f, 0.f, 0.f};
-        const float *kr = A + (16 * dt + l16) * VS + 4 * grp;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const float4 b = lds4(kr + 16 * t);
-            dsk = mfma16(dp[t][0], b.x, dsk);
-            dsk = mfma16(dp[t][1], b.y, dsk);
-            dsk = mfma16(dp[t][2], b.z, dsk);
-            dsk = mfma16(dp[t][3], b.w, dsk);
-        }
-        tpart += (double)(dsk[0] * qv[dt][0]) + (double)(dsk[1] * qv[dt][1]) +
-                 (double)(dsk[2] * qv[dt][2]) + (double)(dsk[3] * qv[dt][3]);
-        store4<ACC>(dqi, g.qstride, r0, tq, 16 * dt + l16, dh, oq[dt], dsk, tau);
+        tpart += (double)(dsk[dt][0] * qv[dt][0]) + (double)(dsk[dt][1] * qv[dt][1]) +
+                 (double)(dsk[dt][2] * qv[dt][2]) + (double)(dsk[dt][3] * qv[dt][3]);
+        store4<ACC>(dqi, g.qstride, r0, tq, 16 * dt + l16, dh, oq[dt], dsk[dt], tau);
     }
     tpart = wave_sum_d(tpart);
     if (lane == 0) dred[w] = tpart;
-    __syncthreads();  // every wave is done with K^T; the dtau shares are in dred
+    __syncthreads();  // every wave is done with K; the dtau shares are in dred
     if (tid == 0)
         g.dtau_part[(long long)img * g.h + hd] = ((dred[0] + dred[1]) + dred[2]) + dred[3];
     // dS in LDS as [tq][tk] (position q*tk + k, as the inverse index numbers
