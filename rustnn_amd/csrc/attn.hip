@@ -328,13 +328,14 @@ struct LongTile {
             const int i = tid + 256 * j;
             const float *x = &v[hh][4 * j];
             uint2 *d = reinterpret_cast<uint2 *>(lds) + (i / G) * RS * 2 + i % G;
-            float r[4], q[4];
+            float u[4], r[4], q[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                r[e] = bf3_rest(x[e]);
+                u[e] = x[e] * BF3_UP;
+                r[e] = bf3_rest(u[e]);
                 q[e] = bf3_rest(r[e]);
             }
-            d[0] = make_uint2(bf3_top2(x[0], x[1]), bf3_top2(x[2], x[3]));
+            d[0] = make_uint2(bf3_top2(u[0], u[1]), bf3_top2(u[2], u[3]));
             d[HK * RS * 2] = make_uint2(bf3_top2(r[0], r[1]), bf3_top2(r[2], r[3]));
             d[2 * HK * RS * 2] = make_uint2(bf3_top2(q[0], q[1]), bf3_top2(q[2], q[3]));
         }
@@ -410,8 +411,8 @@ struct LongTile {
                     c[1][k] = pick(a1, f[u], c[1][k]);
                 });
             }
-            out[8 * hh + t] = c[0][0] + c[0][1];
-            out[8 * hh + t + 1] = c[1][0] + c[1][1];
+            out[8 * hh + t] = (c[0][0] + c[0][1]) * BF3_DOWN;
+            out[8 * hh + t + 1] = (c[1][0] + c[1][1]) * BF3_DOWN;
         }
     }
     // acc[dt] += st (the lane's row, the half's keys) times columns 16 dt ..;
@@ -574,7 +575,7 @@ attn_fwd_long_kernel(AttnArgs g, const uint32_t *__restrict__ relidx) {
     }
     f32x4 o[DHP / 16];
 #pragma unroll
-    for (int dt = 0; dt < DHP / 16; dt++) o[dt] = acc[dt][0] + acc[dt][1];
+    for (int dt = 0; dt < DHP / 16; dt++) o[dt] = (acc[dt][0] + acc[dt][1]) * BF3_DOWN;
     if (T::nonfinite(o)) {
         T::slow_cols(vb, g.kvstride, l16, grp, st, acc);
 #pragma unroll
@@ -997,7 +998,7 @@ attn_bwd_long_q_kernel(AttnArgs g, float *__restrict__ s2) {
     }
     f32x4 dsk[NDT];
 #pragma unroll
-    for (int dt = 0; dt < NDT; dt++) dsk[dt] = acc[dt][0] + acc[dt][1];
+    for (int dt = 0; dt < NDT; dt++) dsk[dt] = (acc[dt][0] + acc[dt][1]) * BF3_DOWN;
     if (T::nonfinite(dsk)) {
         T::slow_cols(kb, g.kvstride, l16, grp, dp, acc);
 #pragma unroll
@@ -1188,8 +1189,8 @@ __global__ __launch_bounds__(256) void attn_bwd_long_k_kernel(AttnArgs g,
         bool bad = false;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
-            av[dt][0] += av[dt][1];
-            ak[dt][0] += ak[dt][1];
+            av[dt][0] = (av[dt][0] + av[dt][1]) * BF3_DOWN;
+            ak[dt][0] = (ak[dt][0] + ak[dt][1]) * BF3_DOWN;
 #pragma unroll
             for (int v = 0; v < 4; v++)
                 bad = bad || bf3_nonfinite(av[dt][0][v]) || bf3_nonfinite(ak[dt][0][v]);

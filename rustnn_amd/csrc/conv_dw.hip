@@ -559,9 +559,11 @@ __device__ __forceinline__ void dw_mfma_wave(const DwArgs &g, float *smem, float
     if constexpr (K == 3) {
         bool bad = false;
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int t = 0; t < NT; t++) {
+            acc[t] *= BF3_DOWN;
 #pragma unroll
             for (int v = 0; v < 16; v++) bad = bad || bf3_nonfinite(acc[t][v]);
+        }
         if (__any(bad)) dw_slow<S, T0, NT>(g, z, cob, cib, wq, lane, acc);
     }
     if constexpr (K == 1) {

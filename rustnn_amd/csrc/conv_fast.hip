@@ -768,7 +768,7 @@ __attribute__((amdgpu_waves_per_eu(EPI || (K == 3 && !(DX && S == 2)) ? 4 : 1)))
                 for (int mb = 0; mb < MB; mb++)
 #pragma unroll
                     for (int j = 0; j < NPW; j++) {
-                        acc[c][mb][j][0] += acc[c][mb][j][1];
+                        acc[c][mb][j][0] = (acc[c][mb][j][0] + acc[c][mb][j][1]) * BF3_DOWN;
 #pragma unroll
                         for (int v = 0; v < 16; v++)
                             bad = bad || bf3_nonfinite(acc[c][mb][j][0][v]);

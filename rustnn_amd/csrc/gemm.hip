@@ -425,14 +425,14 @@ struct DmaTile {
         // Odd shares multiply -A (subtracted in the exchange); a tile without
         // shares turns the sign of its sums every few stages: the matrix
         // core's rounding toward -inf cancels (mfma_split.h).
-        uint32_t neg = NACC == 1 && WK > 1 && (wk() & 1) ? 0x80000000u : 0u;
+        float up = NACC == 1 && WK > 1 && (wk() & 1) ? -BF3_UP : BF3_UP;
         const int flip = min(8, max(1, nk / 4));
         int turn = flip;
         for (int it = 0; it < nk; it++) {
             if constexpr (NACC == 1 && WK == 1)
                 if (turn-- == 0) {
                     turn = flip - 1;
-                    neg ^= 0x80000000u;
+                    up = -up;
                     bf3_negate<TM, TN>(sum);
                 }
             __syncthreads();
@@ -450,15 +450,9 @@ struct DmaTile {
 #pragma unroll
                         for (int e = 0; e < 8; e++) rs[i] += (double)x[i][e];
                 }
-                if constexpr (NACC == 1)
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int e = 0; e < 8; e++)
-                            x[i][e] = __uint_as_float(__float_as_uint(x[i][e]) ^ neg);
                 Bf3 p[TM + TN];
 #pragma unroll
-                for (int i = 0; i < TM + TN; i++) p[i] = bf3_split(x[i]);
+                for (int i = 0; i < TM + TN; i++) p[i] = bf3_split(x[i], i < TM ? up : BF3_UP);
                 bf3_products([&](auto pick, auto kind) {
                     auto &t = NACC == 2 && decltype(kind)::value ? part : sum;
 #pragma unroll
@@ -504,7 +498,7 @@ struct DmaTile {
                         t = NACC == 1 && (s & 1) ? t - u : t + u;
                     }
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[o][4 * e4 + e] = t[e];
+                    for (int e = 0; e < 4; e++) acc[o][4 * e4 + e] = t[e] * BF3_DOWN;
                 }
             if (rsum && k == 0)
 #pragma unroll
@@ -513,11 +507,12 @@ struct DmaTile {
                     for (int i = 0; i < TM; i++)
                         rs[i] += xr[((s * WM * WN + w0) * TM + i) * 64 + lane];
         } else {
-            if (neg) bf3_negate<TM, TN>(sum);
+            const float down = up < 0.f ? -BF3_DOWN : BF3_DOWN;
 #pragma unroll
             for (int o = 0; o < NG; o++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[o][e] = sum[o / (2 * TN)][o / 2 % TN][8 * (o & 1) + e];
+                for (int e = 0; e < 8; e++)
+                    acc[o][e] = sum[o / (2 * TN)][o / 2 % TN][8 * (o & 1) + e] * down;
         }
         // An operand's infinity has no split (its parts are inf and NaN), and
         // part sums can overflow where the values' do not: groups that are

@@ -275,3 +275,38 @@ def test_attn_long_key_forward(rnn, h, dh, th, tw, mh, mw, special):
         fine = np.isfinite(want)
         assert np.array_equal(got[~fine], want[~fine], equal_nan=True)
         assert np.linalg.norm(got[fine] - want[fine]) < tol * np.linalg.norm(want[fine])
+
+
+@pytest.mark.parametrize("dh,th,mh", [(32, 4, 8), (64, 8, 16)])
+@pytest.mark.parametrize("sq,sk,sv,so", [(1.0, 1.0, 1e-36, 1.0), (1.0, 1.0, 1e-36, 1e30),
+                                         (1e-38, 1e30, 1.0, 1e-36), (1e28, 1e-41, 1.0, 1e-8)])
+def test_attn_long_key_exponent_range(rnn, dh, th, mh, sq, sk, sv, so):
+    """Q, K, V and dO far from 1, down to denormal ones."""
+    import torch
+    n, h, tw = 2, 2, 8
+    tq, tk, c = th * tw, mh * 16, h * dh
+    idx, nrel = rnn.rel_index(th, tw, mh, 16)
+    core = rnn.Core(h, dh, tq, tk, idx, nrel, False)
+    gen = torch.Generator(device="cuda").manual_seed(tk + dh)
+    rnd = lambda s, *sh: (torch.randn(sh, generator=gen, device="cuda").double() * s).float()
+    q, do = rnd(sq, n, tq, c), rnd(so, n, tq, c)
+    kv = torch.cat([rnd(sk, n, tk, c), rnd(sv, n, tk, c)], -1)
+    tau, rel = torch.full((h,), dh ** -0.5, device="cuda"), rnd(0.2, h * nrel)
+    lay = (c, 0, kv, 2 * c, 0, c)
+    p, o = core.forward(n, q, *lay, tau, rel)
+    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+    core.backward(n, q, *lay, tau, p, do, dq, dkv, torch.zeros_like(tau), torch.zeros_like(rel),
+                  set_dq=True, set_dkv=True)
+    heads = lambda t, at=0: t[..., at:at + c].reshape(n, -1, h, dh).transpose(1, 2).double()
+    t = lambda a: a.transpose(2, 3).contiguous()
+    Q, K, V, O = heads(q), heads(kv), heads(kv, c), heads(do)
+    P = p.view(n, h, tq, tk).double()
+    dp = O @ t(V)
+    ds = P * (dp - (P * dp).sum(-1, keepdim=True)) * tau.view(1, h, 1, 1)
+    # sums of at most tk products, dS from sums of dh; the spacing of denormals
+    tol = 2.0 ** -24 * (np.sqrt(tk) + 4 * np.sqrt(dh) + 8)
+    for got, want in ((heads(o.view(n, tq, c)), P @ V), (heads(dq), ds @ K),
+                      (heads(dkv), t(ds) @ Q), (heads(dkv, c), t(P) @ O)):
+        got, want = to_host(got.contiguous()), to_host(want.contiguous())
+        size = np.linalg.norm(want) + 2.0 ** -145 * np.sqrt(want.size) / tol
+        assert np.linalg.norm(got - want) < tol * size

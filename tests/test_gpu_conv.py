@@ -355,3 +355,32 @@ def test_conv_dw_split(rnn, n, cin, cout, s, h, w):
         got = to_host(dw).reshape(cout, cin, 9)
         assert np.isfinite(np.delete(got, 2, axis=1)).all() and not np.isnan(got[:, 2, 4]).any()
         assert (~np.isfinite(got[:, 2])).any()
+
+
+@pytest.mark.parametrize("s", [1, 2])
+@pytest.mark.parametrize("sx,sw,sdy", [(1e-36, 1.0, 1.0), (1e-36, 1e30, 1e5), (3e-39, 1e30, 1e5),
+                                       (1.0, 1e-36, 1e-36), (1e30, 1e-41, 1e-41)])
+def test_conv_split_exponent_range(rnn, s, sx, sw, sdy):
+    """Forward, dX and dW of values far from 1, down to denormal ones."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(11)
+    n, cin, cout, h = 4, 20, 40, 16
+    sp = rnn.ConvSpec.make(cin, cout, 3, s, 1, h, h)
+    rnd = lambda sh, f: (torch.randn(sh, generator=g, device="cuda").double() * f).float()
+    x, wt, dy = rnd((n, cin, h, h), sx), rnd((cout, cin, 3, 3), sw), rnd((n, cout, sp.oh, sp.ow),
+                                                                         sdy)
+    xd, wd = x.double().requires_grad_(True), wt.double().requires_grad_(True)
+    cols = torch.nn.functional.unfold(xd, 3, padding=1, stride=s).permute(1, 0, 2)
+    y = (wd.reshape(cout, -1) @ cols.reshape(9 * cin, -1)).view(cout, n, sp.oh, sp.ow)
+    y = y.permute(1, 0, 2, 3)
+    dx, dw = torch.autograd.grad(y, [xd, wd], dy.double())
+    got_dw = torch.zeros(wt.numel(), device="cuda")
+    rnn.conv2d_backward_w(sp, n, dy, x, got_dw)
+    for got, want, k in ((rnn.conv2d_forward(sp, n, x, wt.view(-1)), y.detach(), 9 * cin),
+                         (rnn.conv2d_backward_x(sp, n, dy, wt.view(-1)), dx, 9 * cout),
+                         (got_dw, dw, n * sp.hw)):
+        w = to_host(want.contiguous())
+        # as test_conv_split_matches_float64, and the spacing of denormal results
+        tol = (2.0 ** -24 * np.sqrt(k) + 2.0 ** -22) * np.linalg.norm(w) + 2.0 ** -149 * np.sqrt(
+            w.size)
+        assert np.linalg.norm(to_host(got).astype(np.float64).ravel() - w.ravel()) < tol

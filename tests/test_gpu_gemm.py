@@ -307,3 +307,21 @@ def test_linear_backward_ragged_bias(rnn, rows, fin, fout):
     assert rel_frob(to_host(dw) - 1, to_host(d.T @ x.double())) < 2 * tol(rows)
     assert rel_frob(to_host(db), to_host(d.sum(0) + 1)) < 2.0 ** -23
     assert rel_frob(to_host(dx), to_host(d @ w.double())) < tol(fout)
+
+
+# Operands far from 1, down to denormal ones, whose lower parts have no bf16 of
+# their own exponent: 32 x 64, 64 x 64, 128 x 128, 256 x 128 and ragged tiles.
+@pytest.mark.parametrize("m,n,k", [(64, 64, 64), (2048, 640, 64), (2048, 2048, 1024),
+                                   (16384, 1024, 32), (65, 67, 63)])
+@pytest.mark.parametrize("sa,sb", [(1e-36, 1.0), (1e-36, 1e30), (1e30, 3e-39), (1e-41, 1e30),
+                                   (1e25, 1e10)])
+def test_matmul_split_exponent_range(rnn, m, n, k, sa, sb):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    rnd = lambda r, c, s: (torch.randn((r, c), generator=g, device="cuda").double() * s).float()
+    a, b = rnd(m, k, sa), rnd(k, n, sb)
+    c = torch.empty((m, n), device="cuda")
+    rnn.matmul(m, n, k, a, False, b, False, c)
+    # as test_matmul_split_tiles; results from 1e24 on are fp32 products
+    want = a.double() @ b.double()
+    assert rel_frob(to_host(c), to_host(want)) < 2.0 ** -24 * np.sqrt(k) + 2.0 ** -22
