@@ -450,9 +450,14 @@ struct DmaTile {
 #pragma unroll
                         for (int e = 0; e < 8; e++) rs[i] += (double)x[i][e];
                 }
+                // A rounded: what the split leaves out has no common sign (same-
+                // sign sums were 4.1e-8 too small with both cut off), for 1-2%:
+                // 8192 x 256 x 768 28.3 -> 28.9 us, 4096^3 795 -> 805
                 Bf3 p[TM + TN];
 #pragma unroll
-                for (int i = 0; i < TM + TN; i++) p[i] = bf3_split(x[i], i < TM ? up : BF3_UP);
+                for (int i = 0; i < TM; i++) p[i] = bf3_split_near<NACC == 2>(x[i], up);
+#pragma unroll
+                for (int j = TM; j < TM + TN; j++) p[j] = bf3_split(x[j]);
                 bf3_products([&](auto pick, auto kind) {
                     auto &t = NACC == 2 && decltype(kind)::value ? part : sum;
 #pragma unroll

@@ -4,9 +4,13 @@
 // bits each: its leading 8 bits, those of the remainder, and the rest (cut
 // off, not rounded, so that the largest float's leading part stays finite).
 // Of the nine part products of a x b the three smallest (mid lo, lo mid, lo
-// lo: below 2^-23 of the product) are left out; the other six are exact in
-// the matrix core and summed in its fp32 accumulator, sixteen k values and
-// two roundings an instruction where v_mfma_f32_32x32x2f32 takes two.
+// lo) are left out; the other six are exact in the matrix core and summed in
+// its fp32 accumulator, sixteen k values and two roundings an instruction where
+// v_mfma_f32_32x32x2f32 takes two.  What is left out is below 2^-21 of the
+// product with both operands cut off (mid < 2^-7, lo < 2^-15 of the leading
+// bit), always of the product's sign, so that it adds up over k; below 2^-22
+// and of no common sign with one operand's leading part rounded to nearest
+// instead (|mid| <= 2^-8, |lo| < 2^-16), as every caller does.
 //
 // Measured on MI355X.  Rate: the bf16 pipe sustains 1.79 PFLOP/s from
 // registers, six products 298 TFLOP/s of fp32 work against the fp32 pipe's
@@ -90,21 +94,35 @@ __device__ __forceinline__ Bf3 bf3_split_round(const float (&x)[8]) {
 }
 
 // The same with the leading part alone rounded, which already takes the common
-// sign away, for one integer add a float more than bf3_split.  On the weights
+// sign away (1 + 2^-7 - 2^-23 squared: 4.7e-7 too small cut off, 2e-9 this way;
+// sums of positive products at any k 4.1e-8 / below 1e-9).  On the weights
 // of the 3x3 convolutions: logits of 17 ResNets of 8 to 20 layers 1.047 times
 // the fp32 pipe's error against 64 bits cut off, 0.996 this way, for 1% of the
-// time (a ResNet-20 step 1953 -> 1973 us).
+// time (a ResNet-20 step 1953 -> 1973 us).  CVT: rounded by a bf16 conversion
+// (ties to even) instead of an integer add (away from zero), three
+// instructions a pair of floats less and a longer chain: 512^3 (32 x 64 tiles)
+// 9.5 us against 10.1, 2048^3 (128 x 128) 118.6 against 116.2.
 // An infinity's or NaN's remainder is a NaN.
+template <bool CVT = false>
 __device__ __forceinline__ Bf3 bf3_split_near(const float (&x)[8], float up = BF3_UP) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     Bf3 p;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const float xa = x[2 * j] * up, xb = x[2 * j + 1] * up;
-        const float a = __uint_as_float(__float_as_uint(xa) + 0x8000u);
-        const float b = __uint_as_float(__float_as_uint(xb) + 0x8000u);
-        p.hi[j] = bf3_top2(a, b);
-        const float ra = xa - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
-        const float rb = xb - __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
+        float a, b;  // the leading parts
+        if constexpr (CVT) {
+            const bf16x2 v = {(__bf16)xa, (__bf16)xb};
+            const uint32_t u = __builtin_bit_cast(uint32_t, v);
+            p.hi[j] = u;
+            a = __uint_as_float(u << 16);
+            b = __uint_as_float(u & 0xFFFF0000u);
+        } else {
+            a = __uint_as_float((__float_as_uint(xa) + 0x8000u) & 0xFFFF0000u);
+            b = __uint_as_float((__float_as_uint(xb) + 0x8000u) & 0xFFFF0000u);
+            p.hi[j] = bf3_top2(a, b);
+        }
+        const float ra = xa - a, rb = xb - b;
         p.mid[j] = bf3_top2(ra, rb);
         p.lo[j] = bf3_top2(bf3_rest(ra), bf3_rest(rb));
     }

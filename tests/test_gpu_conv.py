@@ -298,7 +298,8 @@ def test_conv_split_matches_float64(rnn, n, cin, cout, s, h, w):
     y = (wd.reshape(cout, -1) @ cols).view(dy.shape)
     dx, = torch.autograd.grad(y, xd, dy.double())
     # k sums of rounded products as a random walk: 2^-24 sqrt(k) of the result,
-    # with 2^-23 for the part products left out
+    # with 2^-23 for the part products left out (below 2^-22 of their product
+    # each, 2^-24 in the root mean square over random operands)
     tol = lambda k: 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23
     for p in (False, True):
         wp = [rnn.conv_pack_weights(sp, d, wt.view(-1)) for d in (0, 1)] if p else None

@@ -270,7 +270,8 @@ def test_matmul_split_tiles(rnn, m, n, k, at, bt):
     want = (a.T if at else a).double() @ (b.T if bt else b).double()
     # k sums of rounded products, each rounding 2^-24 of a partial sum: as a
     # random walk 2^-24 sqrt(k) of the result, with 2^-23 for the part
-    # products left out
+    # products left out (below 2^-22 of their product each, 2^-24 in the root
+    # mean square over random operands)
     assert rel_frob(to_host(c), to_host(want)) < 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23
 
 
@@ -325,3 +326,26 @@ def test_matmul_split_exponent_range(rnn, m, n, k, sa, sb):
     # as test_matmul_split_tiles; results from 1e24 on are fp32 products
     want = a.double() @ b.double()
     assert rel_frob(to_host(c), to_host(want)) < 2.0 ** -24 * np.sqrt(k) + 2.0 ** -22
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 512, 16), (512, 512, 256), (513, 515, 65), (8192, 256, 48),
+                                   (2048, 2048, 1024), (16384, 1024, 64)])
+def test_matmul_split_same_sign(rnn, m, n, k):
+    """What the split leaves out does not add up over terms of one sign."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    a = torch.randn((m, k), generator=g, device="cuda").abs()
+    b = torch.randn((k, n), generator=g, device="cuda").abs()
+    c = torch.empty((m, n), device="cuda")
+    rnn.matmul(m, n, k, a, False, b, False, c)
+    want = a.double() @ b.double()
+    # each result's error is a random walk of sqrt(k) roundings, their mean over
+    # rows and columns that share operands at most its 1/sqrt(min(m, n)) part
+    tol = 2.0 ** -24 * np.sqrt(k) / np.sqrt(min(m, n)) + 2.0 ** -27
+    assert abs(((c.double() - want) / want).mean().item()) < tol
+    # a mantissa whose parts below the leading one are as large as they get
+    x = 1.0 + 2.0 ** -7 - 2.0 ** -23
+    a.fill_(x)
+    b.fill_(x)
+    rnn.matmul(m, n, k, a, False, b, False, c)
+    assert rel_frob(to_host(c), np.full((m, n), k * x * x)) < 2.0 ** -22
