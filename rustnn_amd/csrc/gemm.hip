@@ -8,8 +8,9 @@
 //   * gemm_dma_kernel (operands under 2 GiB): producer waves DMA the slabs
 //     from HBM straight into a multi-stage LDS ring, 16 bytes a lane where
 //     every operand quad is whole, else one float; the products run on the
-//     bf16 matrix cores, each float in three exact parts (mfma_split.h);
-//   * gemm_kernel (any shape): the 4 waves load a slab into
+//     bf16 matrix cores, each float in three exact parts (mfma_split.h), those
+//     of a short k on the fp32 ones;
+//   * gemm_kernel (larger operands; ragged ones of a short k): the 4 waves load a slab into
 //     registers and store it k-contiguous (16 k values + 4 pad floats a row)
 //     into a double-buffered LDS tile, multiplied by v_mfma_f32_32x32x2f32
 //     (k order inside a block of 8 permuted identically for A and B: step s
@@ -262,22 +263,32 @@ struct DmaOperand {
     uint32_t off[PER];
 
     // First word of DMA u of this lane in a stage's slab.
-    __device__ __forceinline__ static int word(int u, int wave, int lane) {
-        return ((u * NP + wave) * 64 + lane) * VW;
+    static constexpr uint32_t STEP = 64 * NP * VW;  // words between its DMAs
+    static_assert(STEP % (KMAJOR ? BK : R) == 0, "whole rows between a lane's DMAs");
+    __device__ __forceinline__ static uint32_t word(int u, int wave, int lane) {
+        return (uint32_t)(wave * 64 + lane) * VW + u * STEP;
     }
     // The k of word j, relative to the stage.
-    __device__ __forceinline__ static int kof(int j) {
-        if (KMAJOR) return ((j % BK / 4) ^ kswz<BK>(j / BK)) * 4 + j % 4;
+    __device__ __forceinline__ static uint32_t kof(uint32_t j) {
+        if (KMAJOR) return ((j % BK / 4) ^ (uint32_t)kswz<BK>(j / BK)) * 4 + j % 4;
         return j / R;
     }
+    // One vector multiply an operand, since nothing else runs before the first
+    // DMA (a 64 x 64 x 4 product 4.1 -> 3.9 us).
     __device__ __forceinline__ void init(int ld, int rows, int r0, int wave, int lane) {
+        const uint32_t j0 = word(0, wave, lane);
+        if (KMAJOR) {
+            const uint32_t r = r0 + j0 / BK, at = r * (uint32_t)ld;
 #pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int j = word(u, wave, lane);
-            const int row = r0 + (KMAJOR ? j / BK : j % R);
-            off[u] = row >= rows ? DMA_OOB
-                     : KMAJOR    ? (uint32_t)(row * ld + kof(j)) * 4u
-                                 : (uint32_t)(kof(j) * ld + row) * 4u;
+            for (int u = 0; u < PER; u++) {
+                const uint32_t o = at + u * (STEP / BK) * (uint32_t)ld + kof(j0 + u * STEP);
+                off[u] = r + u * (STEP / BK) < (uint32_t)rows ? o * 4u : DMA_OOB;
+            }
+        } else {
+            const uint32_t c = r0 + j0 % R, at = kof(j0) * (uint32_t)ld + c;
+#pragma unroll
+            for (int u = 0; u < PER; u++)
+                off[u] = c < (uint32_t)rows ? (at + u * (STEP / R) * (uint32_t)ld) * 4u : DMA_OOB;
         }
     }
     // Issues this thread's DMAs of k values k0 .. k0 + BK (of kz) into lds.
@@ -288,7 +299,7 @@ struct DmaOperand {
 #pragma unroll
         for (int u = 0; u < PER; u++) {
             uint32_t o = off[u];
-            if (!whole && k0 + kof(word(u, wave, lane)) >= kz) o = DMA_OOB;
+            if (!whole && k0 + (int)kof(word(u, wave, lane)) >= kz) o = DMA_OOB;
             const lds_ptr_t to = (lds_ptr_t)(lds + word(u, wave, 0));
             if constexpr (VW == 4)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, to, 16, o, so, 0, 0);
@@ -330,8 +341,10 @@ struct DmaOperand {
 // stage it has landed (each producer waited for its own DMAs) and every
 // compute wave is done with stage it - 1, whose buffer the producers then
 // refill with stage it + NS - 1.
+// F32: the products on the fp32 matrix cores (NACC = 2: k steps alternate
+// between two accumulators).
 template <int BM, int BN, int BK, int NS, int WM, int WN, int WK, int NP, int NACC, int VW,
-          bool AT, bool BT>
+          bool AT, bool BT, bool F32 = false>
 struct DmaTile {
     static constexpr int NC = WM * WN * WK;
     using OA = DmaOperand<BM, BK, !AT, NP, VW>;
@@ -346,22 +359,23 @@ struct DmaTile {
     static constexpr int OCC = ((int)(160 * 1024 / LDS_BYTES) * (NC + NP) + 3) / 4;
     static constexpr int NG = TM * TN * 2 / WK;  // accumulator groups a wave keeps
     static_assert(TM * TN * 2 % WK == 0 && BK % (16 * WK) == 0, "wave layout");
+    static_assert(!F32 || WK == 1, "the exchange of shares scales the split's sums");
     float acc[NG][8];
     // With rsum, the f64 sums of the A values this lane multiplies: row
     // wm*WTM + 32i + lr, stage by stage in k order (of share 0: of all k).
     double rs[TM];
 
-    __device__ __forceinline__ static int wk() { return wave_index() / (WM * WN); }
-    __device__ __forceinline__ static int wm() { return wave_index() / WN % WM; }
-    __device__ __forceinline__ static int wn() { return wave_index() % WN; }
-    __device__ __forceinline__ static int row0() { return wm() * WTM; }
+    // This wave's place, read once: a readfirstlane an element of the epilogue,
+    // which the compiler may not move, took 0.3 us of a launch.
+    const int wave = wave_index(), wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+    const int row0 = wm * WTM;
     // Tile row and column of element 0 of kept group o (before the lane's part).
-    __device__ __forceinline__ static int grow(int o) {
-        const int g = wk() * NG + o;
-        return row0() + g / (2 * TN) * 32 + (g & 1) * 16;
+    __device__ __forceinline__ int grow(int o) const {
+        const int g = wk * NG + o;
+        return row0 + g / (2 * TN) * 32 + (g & 1) * 16;
     }
-    __device__ __forceinline__ static int gcol(int o) {
-        return wn() * WTN + (wk() * NG + o) / 2 % TN * 32;
+    __device__ __forceinline__ int gcol(int o) const {
+        return wn * WTN + (wk * NG + o) / 2 % TN * 32;
     }
     // The row of element e of a group, past grow(), in lane half lh.
     __device__ __forceinline__ static int erow(int e, int lh) {
@@ -373,7 +387,7 @@ struct DmaTile {
     // (extents below 2^31 bytes, checked by the host).
     __device__ __forceinline__ bool run(const float *A, int lda, int M, const float *B, int ldb,
                                         int N, int kz, int m0, int n0, bool rsum, float *lds) {
-        const int lane = threadIdx.x & 63, wave = wave_index();
+        const int lane = threadIdx.x & 63;
         const int nk = (kz + BK - 1) / BK;
         if (wave >= NC) {
             const int pw = wave - NC;
@@ -421,15 +435,15 @@ struct DmaTile {
 #pragma unroll
                 for (int v = 0; v < 16; v++) sum[i][j][v] = part[i][j][v] = 0.f;
         constexpr int NSTEP = BK / 16 / WK;
-        const int s0 = wk() * NSTEP, ra0 = row0() + lr, rb0 = wn() * WTN + lr;
+        const int s0 = wk * NSTEP, ra0 = row0 + lr, rb0 = wn * WTN + lr;
         // Odd shares multiply -A (subtracted in the exchange); a tile without
         // shares turns the sign of its sums every few stages: the matrix
         // core's rounding toward -inf cancels (mfma_split.h).
-        float up = NACC == 1 && WK > 1 && (wk() & 1) ? -BF3_UP : BF3_UP;
+        float up = NACC == 1 && WK > 1 && (wk & 1) ? -BF3_UP : BF3_UP;
         const int flip = min(8, max(1, nk / 4));
         int turn = flip;
         for (int it = 0; it < nk; it++) {
-            if constexpr (NACC == 1 && WK == 1)
+            if constexpr (NACC == 1 && WK == 1 && !F32)
                 if (turn-- == 0) {
                     turn = flip - 1;
                     up = -up;
@@ -437,6 +451,39 @@ struct DmaTile {
                 }
             __syncthreads();
             const float *As = lds + (it % NS) * STAGE, *Bs = As + OA::WORDS;
+            if constexpr (F32) {
+                float x[NSTEP][TM + TN][8];
+#pragma unroll
+                for (int u = 0; u < NSTEP; u++) {
+#pragma unroll
+                    for (int i = 0; i < TM; i++) OA::frag(As, ra0 + 32 * i, s0 + u, lh, x[u][i]);
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        OB::frag(Bs, rb0 + 32 * j, s0 + u, lh, x[u][TM + j]);
+                }
+                // the stage's reads go out ahead of its MFMAs
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < NSTEP; u++) {
+                    if (rsum) {
+#pragma unroll
+                        for (int i = 0; i < TM; i++)
+#pragma unroll
+                            for (int e = 0; e < 8; e++) rs[i] += (double)x[u][i][e];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        auto &t = NACC == 2 && (e & 1) ? part : sum;
+#pragma unroll
+                        for (int i = 0; i < TM; i++)
+#pragma unroll
+                            for (int j = 0; j < TN; j++)
+                                t[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                    x[u][i][e], x[u][TM + j][e], t[i][j], 0, 0, 0);
+                    }
+                }
+                continue;
+            }
 #pragma unroll
             for (int u = 0; u < NSTEP; u++) {
                 float x[TM + TN][8];
@@ -450,14 +497,14 @@ struct DmaTile {
 #pragma unroll
                         for (int e = 0; e < 8; e++) rs[i] += (double)x[i][e];
                 }
-                // A rounded: what the split leaves out has no common sign (same-
-                // sign sums were 4.1e-8 too small with both cut off), for 1-2%:
-                // 8192 x 256 x 768 28.3 -> 28.9 us, 4096^3 795 -> 805
+                // B rounded: what the split leaves out has no common sign (same-
+                // sign sums were 4.1e-8 too small with both cut off), for 2-3%:
+                // 8192 x 256 x 768 28.3 -> 29.3 us, 4096^3 795 -> 808
                 Bf3 p[TM + TN];
 #pragma unroll
-                for (int i = 0; i < TM; i++) p[i] = bf3_split_near<NACC == 2>(x[i], up);
+                for (int i = 0; i < TM; i++) p[i] = bf3_split(x[i], up);
 #pragma unroll
-                for (int j = TM; j < TM + TN; j++) p[j] = bf3_split(x[j]);
+                for (int j = TM; j < TM + TN; j++) p[j] = bf3_split_near<NACC == 2>(x[j]);
                 bf3_products([&](auto pick, auto kind) {
                     auto &t = NACC == 2 && decltype(kind)::value ? part : sum;
 #pragma unroll
@@ -490,7 +537,7 @@ struct DmaTile {
 #pragma unroll
                 for (int i = 0; i < TM; i++) xr[(wave * TM + i) * 64 + lane] = rs[i];
             __syncthreads();
-            const int w0 = wave % (WM * WN), k = wk();
+            const int w0 = wave % (WM * WN), k = wk;
 #pragma unroll
             for (int o = 0; o < NG; o++)
 #pragma unroll
@@ -512,7 +559,7 @@ struct DmaTile {
                     for (int i = 0; i < TM; i++)
                         rs[i] += xr[((s * WM * WN + w0) * TM + i) * 64 + lane];
         } else {
-            const float down = up < 0.f ? -BF3_DOWN : BF3_DOWN;
+            const float down = F32 ? 1.f : up < 0.f ? -BF3_DOWN : BF3_DOWN;
 #pragma unroll
             for (int o = 0; o < NG; o++)
 #pragma unroll
@@ -522,12 +569,14 @@ struct DmaTile {
         // An operand's infinity has no split (its parts are inf and NaN), and
         // part sums can overflow where the values' do not: groups that are
         // not finite are taken again on the fp32 matrix cores.
-        bool bad = false;
+        if constexpr (!F32) {
+            bool bad = false;
 #pragma unroll
-        for (int o = 0; o < NG; o++)
+            for (int o = 0; o < NG; o++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) bad = bad || bf3_nonfinite(acc[o][e]);
-        if (__any(bad)) slow(A, lda, M, B, ldb, N, kz, m0, n0);
+                for (int e = 0; e < 8; e++) bad = bad || bf3_nonfinite(acc[o][e]);
+            if (__any(bad)) slow(A, lda, M, B, ldb, N, kz, m0, n0);
+        }
         return true;
     }
 
@@ -595,6 +644,15 @@ template <bool AT, bool BT>
 using Tile32u = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, 1, AT, BT>;
 template <bool AT, bool BT>
 using Tile64u = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, 1, AT, BT>;
+// Short k: the fp32 matrix cores, four 32 x 32 sub-tiles.  A split of a stage
+// or two is not paid back (us, this tile / the split ones): 465 products of 49
+// x 196 x 32 14.7 / 17.0, 512 of 64 x 256 x 64 22.0 / 25.2, 8192 x 256 x 32
+// 6.0 / 6.8, 1024 x 1024 x 96 5.6 / 6.1 (4096 x 4096 x 16 24.2 against the
+// 256 x 128 tile's 18.2); and up to k = 4 its sums are nearer to
+// 64 bits (k = 1 2.5e-8 / 4.0e-8, 2 3.1e-8 / 3.9e-8, 4 4.1e-8 / 4.0e-8, 8
+// 4.8e-8 / 4.0e-8).
+template <bool AT, bool BT>
+using Tile64f = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT, true>;
 // Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile.
 template <bool AT, bool BT>
 using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, 4, AT, BT>;
@@ -613,8 +671,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(Gemm
     const int m0 = (tl / gx) * BM, n0 = (tl % gx) * BN;
     // RS: the compute waves of the first column tile also sum A's values
     const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
-    const bool rsum = RS && n0 == 0 && Tile::wn() == 0;
     Tile t;
+    const bool rsum = RS && n0 == 0 && t.wn == 0;
     if (!t.run(g.a + zoff(g, z, g.stride_a, g.stride_a2), g.lda, g.M,
                g.b + zoff(g, z, g.stride_b, g.stride_b2), g.ldb, g.N, kz, m0, n0,
                rsum, lds))
@@ -625,8 +683,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(Gemm
             // the two lane halves' sums, added in half order on both halves
             const double o = __shfl_xor(t.rs[i], 32, 64);
             const double s = lh == 0 ? t.rs[i] + o : o + t.rs[i];
-            const int row = m0 + Tile::row0() + i * 32 + lr;
-            if (lh == 0 && Tile::wk() == 0 && row < g.M) {
+            const int row = m0 + t.row0 + i * 32 + lr;
+            if (lh == 0 && t.wk == 0 && row < g.M) {
                 if (g.rsum_part)
                     g.rsum_part[z * g.M + row] = s;
                 else
@@ -656,8 +714,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(Gemm
     }
 #pragma unroll
     for (int o = 0; o < Tile::NG; o++) {
-        const int col = n0 + Tile::gcol(o) + lr, colc = min(col, g.N - 1);
-        const int row0 = m0 + Tile::grow(o);
+        const int col = n0 + t.gcol(o) + lr, colc = min(col, g.N - 1);
+        const int row0 = m0 + t.grow(o);
         const float bj = bias ? g.bias[colc] : 0.f, lj = res ? g.res_l[colc] : 0.f;
         float old[8], mv[8];
 #pragma unroll
@@ -990,10 +1048,18 @@ static bool dma_enabled() {
     return on;
 }
 
+// Operands whose quads are not whole with a k this short stay on gemm_kernel,
+// for its time and (up to k = 4) its rounding, as at Tile64f: 511 x 513 x 31
+// 4.9 us against 5.7, 8191 x 255 x 31 6.6 / 8.1, x 47 7.8 / 8.8, x 63 9.0 / 8.8,
+// 4095 x 4097 x 47 42.4 / 42.3, x 63 51.6 / 42.5.
+constexpr size_t RAGGED_SHORT_K = 48;
+
 // Whether C += A^T B (A [k x m], B [k x n]) takes the direct-to-LDS kernel,
 // which can then also sum A's columns (the row sums of A^T).
-static bool dw_rowsum_ok(size_t m, size_t n, size_t k) {
-    return dma_enabled() && dma_extent_ok(m, n, k, k, (int)m, 1, (int)n, 0);
+static bool dw_rowsum_ok(size_t m, size_t n, size_t k, const float *a, const float *b) {
+    if (!dma_enabled()) return false;
+    if (dma_ok(1, m, n, k, k, a, 0, (int)m, 1, b, 0, (int)n, 0)) return true;
+    return k > RAGGED_SHORT_K && dma_extent_ok(m, n, k, k, (int)m, 1, (int)n, 0);
 }
 
 // rs_out / rs_part: the row sums of op(A) (A^T B layout and the direct-to-LDS
@@ -1046,19 +1112,27 @@ static int gemm_enqueue(rnn_ctx *ctx, size_t count, size_t m, size_t n, size_t k
         // definitions): 256 x 128 from two tiles a CU (at 1.5, 16384 x 768,
         // the 64 x 64 grid is faster), 128 x 128 from one a CU where k is
         // long enough to pay for its ramp, 32 x 64 where 64 x 64 tiles would
-        // leave CUs without one.
+        // give a CU no more than one (1024^3 21.0 us against 23.2, 4096 x 256
+        // x 256 8.4 against 9.1; with 1.25 a CU, 2048 x 640 x 256, 12.1 against
+        // 10.9).  The fp32 tile for a k that a split does not pay for: one or
+        // two stages, four where the 32 x 64 tiles, more than one a CU, would
+        // take a second round.
         const size_t cus = (size_t)ctx->num_cus;
         const size_t tiles256 = rnn_div_up(m, 256) * rnn_div_up(n, 128) * count;
         const size_t tiles64 = rnn_div_up(m, 64) * rnn_div_up(n, 64) * count;
-        if (m >= 256 && n >= 128 && tiles256 >= 2 * cus)
+        const bool one = tiles64 > cus / 2 && tiles64 <= cus;
+        if (m >= 256 && n >= 128 && tiles256 >= 2 * cus && kchunk > 4)
             return launch_dma<Tile256>(ctx, g, (int)count, at, bt);
         if (m >= 128 && n >= 128 && tiles128 >= cus && kchunk >= 1024)
             return launch_dma<Tile128>(ctx, g, (int)count, at, bt);
-        if (tiles64 < cus) return launch_dma<Tile32>(ctx, g, (int)count, at, bt);
+        if (kchunk <= (one ? 128 : 64)) return launch_dma<Tile64f>(ctx, g, (int)count, at, bt);
+        if (tiles64 <= cus) return launch_dma<Tile32>(ctx, g, (int)count, at, bt);
         return launch_dma<Tile64>(ctx, g, (int)count, at, bt);
     }
-    if (dma_enabled() && dma_extent_ok(m, n, kchunk, ktotal, lda, at, ldb, bt)) {
-        // quads that are not whole: the aligned rule's line between the tiles
+    if (dma_enabled() && dma_extent_ok(m, n, kchunk, ktotal, lda, at, ldb, bt) &&
+        (kchunk > RAGGED_SHORT_K || rs_out || rs_part)) {
+        // quads that are not whole: 32 x 64 tiles where 64 x 64 ones would
+        // leave CUs without one
         if (rnn_div_up(m, 64) * rnn_div_up(n, 64) * count < (size_t)ctx->num_cus)
             return launch_dma<Tile32u>(ctx, g, (int)count, at, bt);
         return launch_dma<Tile64u>(ctx, g, (int)count, at, bt);
@@ -1302,7 +1376,7 @@ int rnn_linear_backward_ex(rnn_ctx *ctx, size_t rows, size_t fin, size_t fout, c
     // (linear.rs:70-89), summed in f64 by the dW GEMM itself when it takes
     // the direct-to-LDS kernel, else by the column-sum kernels
     int rc;
-    if (db && rows && fout && fin && dw_rowsum_ok(fout, fin, rows)) {
+    if (db && rows && fout && fin && dw_rowsum_ok(fout, fin, rows, dy, x)) {
         rc = gemm_splitk(ctx, fout, fin, rows, dy, 1, x, 0, dw, 1, db, true);
         if (rc == -1)
             rc = gemm_enqueue(ctx, 1, fout, fin, rows, rows, dy, 0, (int)fout, 1, x, 0, (int)fin,

@@ -349,3 +349,64 @@ def test_matmul_split_same_sign(rnn, m, n, k):
     b.fill_(x)
     rnn.matmul(m, n, k, a, False, b, False, c)
     assert rel_frob(to_host(c), np.full((m, n), k * x * x)) < 2.0 ** -22
+
+
+# Short k, which takes the fp32 matrix cores: one product is rounded once, and
+# sums of a few are no further off than a chain of fp32 roundings.
+@pytest.mark.parametrize("m,n", [(4, 4), (64, 68), (8192, 256), (4096, 4096), (1, 3), (511, 513)])
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("k", [1, 2, 4, 5])
+def test_matmul_short_k(rnn, m, n, k, at, bt):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn((k, m) if at else (m, k), generator=g, device="cuda")
+    b = torch.randn((n, k) if bt else (k, n), generator=g, device="cuda")
+    c = torch.full((m, n), 7.0, device="cuda")
+    rnn.matmul(m, n, k, a, at, b, bt, c)
+    want = (a.T if at else a).double() @ (b.T if bt else b).double()
+    if k == 1:
+        assert torch.equal(c, want.float())
+    elif m * n > 256:
+        # rounding j of k is 2^-24 / sqrt(3) of a partial sum of j of the k terms
+        # at most, 0.7 of that where mantissas are spread over a binade
+        tol = 2.0 ** -24 / np.sqrt(3) * np.sqrt((k + 1) / 2)
+        assert ((c.double() - want).norm() / want.norm()).item() < tol
+
+
+# Both sides of the lines between the tiles: fp32 and split ones at k = 64 / 68
+# and, with 129 to 256 tiles, 128 / 132; 32 x 64 and 64 x 64 ones at 256 and 272
+# tiles; ragged sizes at k = 48 / 49.  With infinities and a NaN.
+@pytest.mark.parametrize("m,n,k", [(512, 512, 64), (512, 512, 68), (1024, 1020, 128),
+                                   (1024, 1020, 132), (1024, 1088, 68), (2048, 1028, 132),
+                                   (255, 257, 48), (255, 257, 49), (2047, 1029, 131)])
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False)])
+def test_matmul_tile_lines(rnn, m, n, k, at, bt):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randint(-3, 4, (k, m) if at else (m, k), generator=g, device="cuda").float()
+    b = torch.randint(-3, 4, (n, k) if bt else (k, n), generator=g, device="cuda").float()
+    c = torch.empty((m, n), device="cuda")
+    for special in (False, True):
+        if special:
+            av, bv = a.T if at else a, b.T if bt else b
+            av[5, 3], av[m - 1, k - 1] = float("inf"), float("nan")
+            bv[2, 9], bv[k - 1, n - 2] = float("-inf"), float("inf")
+        rnn.matmul(m, n, k, a, at, b, bt, c)
+        want = ((a.T if at else a).double() @ (b.T if bt else b).double()).float()
+        assert np.array_equal(to_host(c), to_host(want), equal_nan=True)
+
+
+@pytest.mark.parametrize("rows,fin,fout", [(1, 32, 64), (3, 33, 31), (48, 33, 31), (49, 33, 31),
+                                           (64, 64, 128)])
+def test_linear_backward_few_rows(rnn, rows, fin, fout):
+    """dW and db of a short batch, with db beside dW and in a sum of its own."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows + fin)
+    dy = torch.randint(-3, 4, (rows, fout), generator=g, device="cuda").float()
+    x = torch.randint(-3, 4, (rows, fin), generator=g, device="cuda").float()
+    w = torch.randint(-3, 4, (fout, fin), generator=g, device="cuda").float()
+    dw, db = torch.ones(fout * fin, device="cuda"), torch.ones(fout, device="cuda")
+    dx = rnn.linear_backward(rows, fin, fout, dy, x, w, dw, db)
+    assert torch.equal(dw.view(fout, fin), dy.T.contiguous() @ x + 1)
+    assert torch.equal(db, dy.sum(0) + 1)
+    assert torch.equal(dx.view(rows, fin), dy @ w)
