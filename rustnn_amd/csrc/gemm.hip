@@ -653,9 +653,12 @@ using Tile64u = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, 1, AT, BT>;
 // 4.8e-8 / 4.0e-8).
 template <bool AT, bool BT>
 using Tile64f = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT, true>;
-// Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile.
+// Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile, one
+// accumulator, so that two workgroups fit a CU by registers too (the optimiser's
+// step over the rustvit's parameters, fp32 pipe 360 us: with two accumulators
+// and one workgroup 378, this way 346; five 704 x 256 matrices 245 / 212 / 213).
 template <bool AT, bool BT>
-using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, 4, AT, BT>;
+using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 1, 4, AT, BT>;
 
 template <class Tile, bool RS>
 __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(GemmArgs g) {
@@ -870,8 +873,8 @@ __device__ __forceinline__ void ns_tile_dma(const NsGemmProb &p, uint32_t z, int
 
 using NsTile = TileNs<false, false>;
 
-__global__ __launch_bounds__(NsTile::THREADS, 3) void ns_gemm_dma_kernel(const NsGemmProb *__restrict__ probs,
-                                                          int nprob, float alpha, float beta) {
+__global__ __launch_bounds__(NsTile::THREADS, NsTile::OCC) void ns_gemm_dma_kernel(
+    const NsGemmProb *__restrict__ probs, int nprob, float alpha, float beta) {
     extern __shared__ float lds[];
     int lo = 0, hi = nprob - 1;
     while (lo < hi) {
