@@ -644,13 +644,16 @@ template <bool AT, bool BT>
 using Tile32u = DmaTile<32, 64, 64, 3, 1, 1, 4, 4, 2, 1, AT, BT>;
 template <bool AT, bool BT>
 using Tile64u = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 1, 1, AT, BT>;
-// Short k: the fp32 matrix cores, four 32 x 32 sub-tiles.  A split of a stage
-// or two is not paid back (us, this tile / the split ones): 465 products of 49
-// x 196 x 32 14.7 / 17.0, 512 of 64 x 256 x 64 22.0 / 25.2, 8192 x 256 x 32
-// 6.0 / 6.8, 1024 x 1024 x 96 5.6 / 6.1 (4096 x 4096 x 16 24.2 against the
-// 256 x 128 tile's 18.2); and up to k = 4 its sums are nearer to
-// 64 bits (k = 1 2.5e-8 / 4.0e-8, 2 3.1e-8 / 3.9e-8, 4 4.1e-8 / 4.0e-8, 8
-// 4.8e-8 / 4.0e-8).
+// Short k: four 32 x 32 sub-tiles, no shares to exchange.  Split (us, this tile
+// / the 64 x 64 one above): 465 products of 49 x 196 x 32 14.3 / 15.9, 512 of
+// 64 x 256 x 64 21.1 / 23.5, 8192 x 256 x 32 5.9 / 6.3, 1024 x 1024 x 96 6.1 /
+// 6.5; at k = 144 and 196 no faster.
+template <bool AT, bool BT>
+using Tile64s = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT>;
+// The same on the fp32 matrix cores: nearer to 64 bits up to k = 4 (k = 1 2.5e-8
+// / 4.0e-8 split, 2 3.1e-8 / 3.9e-8, 4 4.1e-8 / 4.0e-8, 8 4.8e-8 / 4.1e-8, 24
+// 7.0e-8 / 4.6e-8), and in a grid of at most one tile a CU faster where k is a
+// stage (64 x 64 x 16 3.6 us / 3.9, 1024 x 1024 x 16 4.4 / 4.7).
 template <bool AT, bool BT>
 using Tile64f = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT, true>;
 // Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile, one
@@ -1052,10 +1055,10 @@ static bool dma_enabled() {
 }
 
 // Operands whose quads are not whole with a k this short stay on gemm_kernel,
-// for its time and (up to k = 4) its rounding, as at Tile64f: 511 x 513 x 31
-// 4.9 us against 5.7, 8191 x 255 x 31 6.6 / 8.1, x 47 7.8 / 8.8, x 63 9.0 / 8.8,
-// 4095 x 4097 x 47 42.4 / 42.3, x 63 51.6 / 42.5.
-constexpr size_t RAGGED_SHORT_K = 48;
+// for its time (511 x 513 x 7 4.2 us against 4.8, 8191 x 255 x 7 5.6 / 6.7, x 31
+// 6.7 / 6.8) and its rounding (against 64 bits at k = 1 2.5e-8 / 3.7e-8, 8
+// 5.4e-8 / 4.1e-8, 16 7.4e-8 / 4.4e-8).
+constexpr size_t RAGGED_SHORT_K = 12;
 
 // Whether C += A^T B (A [k x m], B [k x n]) takes the direct-to-LDS kernel,
 // which can then also sum A's columns (the row sums of A^T).
@@ -1117,18 +1120,22 @@ static int gemm_enqueue(rnn_ctx *ctx, size_t count, size_t m, size_t n, size_t k
         // long enough to pay for its ramp, 32 x 64 where 64 x 64 tiles would
         // give a CU no more than one (1024^3 21.0 us against 23.2, 4096 x 256
         // x 256 8.4 against 9.1; with 1.25 a CU, 2048 x 640 x 256, 12.1 against
-        // 10.9).  The fp32 tile for a k that a split does not pay for: one or
-        // two stages, four where the 32 x 64 tiles, more than one a CU, would
-        // take a second round.
+        // 10.9).  Before the last two, the tiles for a short k: up to 64, or
+        // 128 where the 32 x 64 tiles, more than one a CU, take a second round
+        // (1024 x 1024 x 96 6.1 / 6.5); on the fp32 cores up to 4, and up to
+        // 24, where its error is still below that of the split with both
+        // operands cut off, in a grid of one tile a CU.
         const size_t cus = (size_t)ctx->num_cus;
         const size_t tiles256 = rnn_div_up(m, 256) * rnn_div_up(n, 128) * count;
         const size_t tiles64 = rnn_div_up(m, 64) * rnn_div_up(n, 64) * count;
-        const bool one = tiles64 > cus / 2 && tiles64 <= cus;
-        if (m >= 256 && n >= 128 && tiles256 >= 2 * cus && kchunk > 4)
+        if (kchunk <= (tiles64 <= cus ? 24 : 4))
+            return launch_dma<Tile64f>(ctx, g, (int)count, at, bt);
+        if (m >= 256 && n >= 128 && tiles256 >= 2 * cus)
             return launch_dma<Tile256>(ctx, g, (int)count, at, bt);
         if (m >= 128 && n >= 128 && tiles128 >= cus && kchunk >= 1024)
             return launch_dma<Tile128>(ctx, g, (int)count, at, bt);
-        if (kchunk <= (one ? 128 : 64)) return launch_dma<Tile64f>(ctx, g, (int)count, at, bt);
+        if (2 * tiles64 > cus && kchunk <= (tiles64 <= cus ? 128 : 64))
+            return launch_dma<Tile64s>(ctx, g, (int)count, at, bt);
         if (tiles64 <= cus) return launch_dma<Tile32>(ctx, g, (int)count, at, bt);
         return launch_dma<Tile64>(ctx, g, (int)count, at, bt);
     }

@@ -351,8 +351,8 @@ def test_matmul_split_same_sign(rnn, m, n, k):
     assert rel_frob(to_host(c), np.full((m, n), k * x * x)) < 2.0 ** -22
 
 
-# Short k, which takes the fp32 matrix cores: one product is rounded once, and
-# sums of a few are no further off than a chain of fp32 roundings.
+# Short k: one product is rounded once, and sums of a few are no further off
+# than a chain of fp32 roundings.
 @pytest.mark.parametrize("m,n", [(4, 4), (64, 68), (8192, 256), (4096, 4096), (1, 3), (511, 513)])
 @pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("k", [1, 2, 4, 5])
@@ -373,12 +373,14 @@ def test_matmul_short_k(rnn, m, n, k, at, bt):
         assert ((c.double() - want).norm() / want.norm()).item() < tol
 
 
-# Both sides of the lines between the tiles: fp32 and split ones at k = 64 / 68
-# and, with 129 to 256 tiles, 128 / 132; 32 x 64 and 64 x 64 ones at 256 and 272
-# tiles; ragged sizes at k = 48 / 49.  With infinities and a NaN.
-@pytest.mark.parametrize("m,n,k", [(512, 512, 64), (512, 512, 68), (1024, 1020, 128),
-                                   (1024, 1020, 132), (1024, 1088, 68), (2048, 1028, 132),
-                                   (255, 257, 48), (255, 257, 49), (2047, 1029, 131)])
+# Both sides of the lines between the tiles: fp32 and split ones at k = 4 / 8
+# and, with up to 256 tiles, 24 / 28; tiles without shares up to k = 64, or 128;
+# 32 x 64 and 64 x 64 ones at 256 and 272 tiles; ragged sizes at k = 12 / 13.
+# With infinities and a NaN.
+@pytest.mark.parametrize("m,n,k", [(1024, 1088, 4), (1024, 1088, 8), (512, 512, 24), (512, 512, 28),
+                                   (1024, 1020, 128), (1024, 1020, 132), (1024, 1088, 64),
+                                   (1024, 1088, 68), (255, 257, 12), (255, 257, 13),
+                                   (2047, 1029, 131)])
 @pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False)])
 def test_matmul_tile_lines(rnn, m, n, k, at, bt):
     import torch
