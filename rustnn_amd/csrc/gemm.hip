@@ -656,12 +656,18 @@ using Tile64s = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT>;
 // stage (64 x 64 x 16 3.6 us / 3.9, 1024 x 1024 x 16 4.4 / 4.7).
 template <bool AT, bool BT>
 using Tile64f = DmaTile<64, 64, 32, 3, 2, 2, 1, 4, 2, 4, AT, BT, true>;
-// Newton-Schulz: few tiles, long k; eight compute waves a 64 x 64 tile, one
-// accumulator, so that two workgroups fit a CU by registers too (the optimiser's
-// step over the rustvit's parameters, fp32 pipe 360 us: with two accumulators
-// and one workgroup 378, this way 346; five 704 x 256 matrices 245 / 212 / 213).
+// Newton-Schulz, 64 x 64 tiles and two accumulators.  TileNs, for a launch of at
+// most one tile a CU: eight compute waves.  TileNs2, for more: four, so that two
+// workgroups fit a CU by registers (us, fp32 pipe / TileNs / TileNs2: the
+// optimiser's step over the rustvit's parameters, 452 and 1462 tiles a launch,
+// 361 / 382 / 350; six 1152 x 512 matrices, 216 and 864 tiles, 385 / 383 / 386;
+// five 704 x 256, 50 and 220 tiles, 236 / 224 / 244).  With one accumulator two
+// workgroups of eight fit, 338 us of the step, but the results are 1.4 times
+// as far from 64 bits (five 704 x 256 2.2e-7; 1.6e-7 / 1.7e-7, fp32 3.5e-7).
 template <bool AT, bool BT>
-using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 1, 4, AT, BT>;
+using TileNs = DmaTile<64, 64, 64, 2, 2, 1, 4, 4, 2, 4, AT, BT>;
+template <bool AT, bool BT>
+using TileNs2 = DmaTile<64, 64, 32, 3, 2, 1, 2, 4, 2, 4, AT, BT>;
 
 template <class Tile, bool RS>
 __global__ __launch_bounds__(Tile::THREADS, Tile::OCC) void gemm_dma_kernel(GemmArgs g) {
@@ -849,12 +855,11 @@ __global__ __launch_bounds__(256) void ns_gemm_kernel(const NsGemmProb *__restri
 }
 
 // ns_gemm_kernel on the direct-to-LDS tile (every operand of every problem
-// of the launch with whole 16-byte quads): 8 waves, 64 x 64 tiles.
-template <bool AT, bool BT>
+// of the launch with whole 16-byte quads), 64 x 64 tiles.
+template <class Tile>
 __device__ __forceinline__ void ns_tile_dma(const NsGemmProb &p, uint32_t z, int ti, int tj,
                                             float alpha, float beta, float *lds) {
 #pragma clang fp contract(off)
-    using Tile = TileNs<AT, BT>;
     const int m0 = ti * 64, n0 = tj * 64;
     Tile t;
     if (!t.run(p.a + z * p.stride_a, p.lda, p.M, p.b + z * p.stride_b, p.ldb, p.N, p.K, m0, n0,
@@ -863,20 +868,35 @@ __device__ __forceinline__ void ns_tile_dma(const NsGemmProb &p, uint32_t z, int
     float *Cp = p.c + z * p.stride_c;
     const float *Ep = p.e ? p.e + z * p.stride_c : nullptr;
     const bool mirror = p.sym && ti != tj;
-    t.each([&](int rr, int cc, float val) {
-        const int row = m0 + rr, col = n0 + cc;
-        if (row < p.M && col < p.N) {
-            const long long o = (long long)row * p.ldc + col;
-            const float v = Ep ? alpha * Ep[o] + beta * val : val;
-            Cp[o] = v;
-            if (mirror) Cp[(long long)col * p.ldc + row] = v;
+    // E is loaded eight elements at a time ahead of the stores: one by one each
+    // load waited behind the store before it (the optimiser's step 380 us, so
+    // 364; five 704 x 256 matrices 222 / 204)
+    const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+#pragma unroll
+    for (int o = 0; o < Tile::NG; o++) {
+        const int row0 = m0 + t.grow(o), col = n0 + t.gcol(o) + lr;
+        float old[8];
+        if (Ep)
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                old[e] = Ep[(long long)min(row0 + Tile::erow(e, lh), p.M - 1) * p.ldc +
+                            min(col, p.N - 1)];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int row = row0 + Tile::erow(e, lh);
+            if (row < p.M && col < p.N) {
+                const float v = Ep ? alpha * old[e] + beta * t.acc[o][e] : t.acc[o][e];
+                Cp[(long long)row * p.ldc + col] = v;
+                if (mirror) Cp[(long long)col * p.ldc + row] = v;
+            }
         }
-    });
+    }
 }
 
-using NsTile = TileNs<false, false>;
-
-__global__ __launch_bounds__(NsTile::THREADS, NsTile::OCC) void ns_gemm_dma_kernel(
+// WGS: workgroups on a CU.
+template <template <bool, bool> class Tile, int WGS>
+__global__ __launch_bounds__((Tile<false, false>::THREADS), (WGS * Tile<false, false>::THREADS / 256))
+void ns_gemm_dma_kernel(
     const NsGemmProb *__restrict__ probs, int nprob, float alpha, float beta) {
     extern __shared__ float lds[];
     int lo = 0, hi = nprob - 1;
@@ -901,11 +921,11 @@ __global__ __launch_bounds__(NsTile::THREADS, NsTile::OCC) void ns_gemm_dma_kern
         tj = (int)(r % p.tn);
     }
     if (p.lay == NS_LAY_NT)
-        ns_tile_dma<false, true>(p, z, ti, tj, alpha, beta, lds);
+        ns_tile_dma<Tile<false, true>>(p, z, ti, tj, alpha, beta, lds);
     else if (p.lay == NS_LAY_TN)
-        ns_tile_dma<true, false>(p, z, ti, tj, alpha, beta, lds);
+        ns_tile_dma<Tile<true, false>>(p, z, ti, tj, alpha, beta, lds);
     else
-        ns_tile_dma<false, false>(p, z, ti, tj, alpha, beta, lds);
+        ns_tile_dma<Tile<false, false>>(p, z, ti, tj, alpha, beta, lds);
 }
 
 __global__ void fill_kernel(float *p, long long n, float v) {
@@ -1001,6 +1021,20 @@ int launch_dma(rnn_ctx *ctx, const GemmArgs &g, int count, bool at, bool bt) {
     if (!at && bt) return launch_dma_t<Tile<false, true>, false>(ctx, g, count);
     if (at && !bt) return launch_dma_t<Tile<true, false>, false>(ctx, g, count);
     return launch_dma_t<Tile<true, true>, false>(ctx, g, count);
+}
+
+template <template <bool, bool> class Tile, int WGS>
+void launch_ns_dma(rnn_ctx *ctx, dim3 grid, const NsGemmProb *probs, int nprob, float alpha,
+                   float beta) {
+    using T = Tile<false, false>;
+    static bool attr = false;
+    if (!attr) {
+        attr = true;
+        (void)hipFuncSetAttribute((const void *)ns_gemm_dma_kernel<Tile, WGS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::LDS_BYTES);
+    }
+    hipLaunchKernelGGL((ns_gemm_dma_kernel<Tile, WGS>), grid, dim3(T::THREADS), T::LDS_BYTES,
+                       ctx->stream, probs, nprob, alpha, beta);
 }
 
 template <int BM, int BN>
@@ -1167,15 +1201,10 @@ int rnn_ns_gemm_launch(rnn_ctx *ctx, const NsGemmProb *probs, int nprob, size_t 
     if (ntiles > 0x7fffffffu) return rnn_fail(ctx, RNN_E_UNSUPPORTED, "ns_gemm: too many tiles");
     const dim3 grid((unsigned)ntiles);
     if (vec == 2) {
-        static bool attr = false;
-        if (!attr) {
-            attr = true;
-            (void)hipFuncSetAttribute((const void *)ns_gemm_dma_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)NsTile::LDS_BYTES);
-        }
-        hipLaunchKernelGGL(ns_gemm_dma_kernel, grid, dim3(NsTile::THREADS), NsTile::LDS_BYTES,
-                           ctx->stream, probs, nprob, alpha, beta);
+        if (ntiles <= (size_t)ctx->num_cus)
+            launch_ns_dma<TileNs, 1>(ctx, grid, probs, nprob, alpha, beta);
+        else
+            launch_ns_dma<TileNs2, 2>(ctx, grid, probs, nprob, alpha, beta);
     } else if (vec)
         hipLaunchKernelGGL(ns_gemm_kernel<true>, grid, dim3(256), 0, ctx->stream, probs, nprob,
                            alpha, beta);

@@ -51,6 +51,24 @@ def test_newton_schulz(rnn, orc, count, rows, cols):
             i, rel_frob(got[i], exact), rel_frob(want, exact))
 
 
+@pytest.mark.parametrize("count,rows,cols", [(4, 512, 512), (2, 1028, 516), (3, 516, 1028)])
+def test_newton_schulz_around_one_tile_a_cu(rnn, count, rows, cols):
+    """Grids of exactly one 64 x 64 tile a CU, and above: two tilings."""
+    from rustnn_amd.optim import newton_schulz
+    rng = np.random.default_rng(rows)
+    g = rng.standard_normal(count * rows * cols).astype(np.float32)
+    G = to_dev(g)
+    newton_schulz(G, rows, cols, 3)
+    got = to_host(G).reshape(count, -1)
+    # nine products of at most 1028 terms, each a random walk of 2^-24 sqrt(k)
+    # and 2^-22 for what the split leaves out; errors of X grow by 3.4445 a step
+    # at most and shrink again where X nears orthogonality
+    tol = 9 * (2.0 ** -24 * np.sqrt(1028) + 2.0 ** -22)
+    for i in range(count):
+        exact = ns_f64(g[i * rows * cols:(i + 1) * rows * cols], rows, cols, 3)
+        assert rel_frob(got[i], exact) < tol
+
+
 def _params(rng, specs):
     """specs: (len, rows, cols, decay); values / grads ~N(0,1)."""
     out = []
