@@ -732,6 +732,11 @@ int rnn_dbg_resnet_buffer(rnn_resnet *net, size_t block, int which, const float 
  * exists to time that kernel alone (benchmarks). */
 int rnn_dbg_resnet_dw_group(rnn_resnet *net, int launch, double *flops);
 int rnn_dbg_im2col(rnn_ctx *ctx, const rnn_conv_spec *sp, const float *x_img, float *col);
+/* The tile of the specialised forward (dx = 0) or dX kernel for n images on a
+ * chip of `cus` CUs: plan[6] = output rows, images, source channels a stage,
+ * 32-position groups a wave, waves along output channels, window positions.
+ * RNN_E_UNSUPPORTED: the generic kernel.  Host only. */
+int rnn_dbg_conv_plan(const rnn_conv_spec *sp, int dx, size_t n, size_t cus, int *plan);
 /* PackedA::pack / pack_t (gemm.rs:54-113) into out[nb*256*mpad] (positions the
  * reference never writes are left untouched). */
 int rnn_dbg_pack_a(rnn_ctx *ctx, const float *a, size_t m, size_t k, int transposed, float *out);

@@ -158,6 +158,7 @@ def lib():
                                               _vp]),
             "rnn_dbg_resnet_buffer": (_i, [_vp, _sz, _i, P(_vp), P(_sz)]),
             "rnn_dbg_resnet_dw_group": (_i, [_vp, _i, P(C.c_double)]),
+            "rnn_dbg_conv_plan": (_i, [P(ConvSpec), _i, _sz, _sz, P(_i)]),
             "rnn_dbg_im2col": (_i, [_vp, P(ConvSpec), _vp, _vp]),
             "rnn_dbg_pack_a": (_i, [_vp, _vp, _sz, _sz, _i, _vp]),
             "rnn_dbg_pack_b": (_i, [_vp, _vp, _sz, _sz, _i, _vp]),
@@ -749,6 +750,14 @@ class Linear:
 
 
 # ------------------------------------------------------------------ debug exports
+def dbg_conv_plan(sp: ConvSpec, dx, n, cus=256):
+    """The specialised kernel's tile for a forward or dX of n images, as
+    rnn_dbg_conv_plan; None where the generic kernel runs."""
+    plan = (_i * 6)()
+    rc = lib().rnn_dbg_conv_plan(C.byref(sp), int(dx), n, cus, plan)
+    return None if rc else tuple(plan)
+
+
 def dbg_im2col(sp: ConvSpec, x_img, ctx=None):
     ctx = ctx or default_ctx()
     col = _new(sp.ckk * sp.hw, x_img)

@@ -941,7 +941,8 @@ static bool plan_ok(FastPlan &p, int CS, int GA, int GB, FastArgs &a) {
 // two 32-position groups per wave where that leaves two items a CU (32 -> 32
 // @32x32, 512 items: 23.4 us), else 128 positions (64 -> 64 @16x16, 256 or 512
 // items: 23.5 / 20.3; 48 -> 80 @23x29, 37 images: 25.2 / 21.2; one 32x32 image
-// 13.9 / 9.5); 1x1 forward takes 256 positions when an image has as many;
+// 13.9 / 9.5), but always 256 for a row of more than 128, which fits no other
+// tile (one 160x160 image 32 -> 32: PLAN_US us, 57.1 on the generic kernel); 1x1 forward takes 256 positions when an image has as many;
 // strided 3x3 forward takes 64 positions with the waves split two ways along
 // output channels, so every wave has a 32x32 block.  A plan that does not fit
 // falls back to shrinking the tile.
@@ -969,7 +970,7 @@ static bool choose_plan(int CS, int CD, int GA, int GB, size_t n, size_t cus, Fa
     int npos = 128;
     if (T::KK == 9 && T::NCLS == 1 && T::IS == 1) {
         const size_t tiles = n * (size_t)((GA + std::max(1, 256 / GB) - 1) / std::max(1, 256 / GB));
-        if (GA * GB >= 256 && tiles * ((CD + 31) / 32) >= 2 * cus) {
+        if (GB > 128 || (GA * GB >= 256 && tiles * ((CD + 31) / 32) >= 2 * cus)) {
             r.NPW = 2;
             npos = 256;
         }
@@ -1240,6 +1241,31 @@ int rnn_conv_fast_parts(const rnn_ctx *ctx, const rnn_conv_spec *sp, size_t n) {
     RNN_CONV_CASE(1, 1, 0)
 #undef RNN_CONV_CASE
     return -1;
+}
+
+template <int K, int S, int P, bool DX>
+static int plan_of(const rnn_conv_spec *sp, size_t n, size_t cus, int *plan) {
+    FastArgs a;
+    FastPlan p;
+    if (!setup<K, S, P, DX>(sp, n, cus, a, p)) return RNN_E_UNSUPPORTED;
+    const int v[6] = {p.TR, p.IMGS, p.CH, p.NPW, p.WM, a.plane};
+    std::copy(v, v + 6, plan);
+    return RNN_OK;
+}
+
+extern "C" int rnn_dbg_conv_plan(const rnn_conv_spec *sp, int dx, size_t n, size_t cus, int *plan) {
+    if (!sp || !plan) return RNN_E_NULL;
+    const int k = sp->k, s = sp->stride, p = sp->pad;
+#define RNN_CONV_CASE(K_, S_, P_)                                        \
+    if (k == K_ && s == S_ && p == P_)                                   \
+        return dx ? plan_of<K_, S_, P_, true>(sp, n, cus, plan)          \
+                  : plan_of<K_, S_, P_, false>(sp, n, cus, plan);
+    RNN_CONV_CASE(3, 1, 1)
+    RNN_CONV_CASE(3, 2, 1)
+    RNN_CONV_CASE(1, 2, 0)
+    RNN_CONV_CASE(1, 1, 0)
+#undef RNN_CONV_CASE
+    return RNN_E_UNSUPPORTED;
 }
 
 int rnn_conv_pack_geo(const rnn_conv_spec *sp, int dx, PackGeo *pg) {

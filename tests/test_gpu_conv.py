@@ -385,3 +385,46 @@ def test_conv_split_exponent_range(rnn, s, sx, sw, sdy):
         tol = (2.0 ** -24 * np.sqrt(k) + 2.0 ** -22) * np.linalg.norm(w) + 2.0 ** -149 * np.sqrt(
             w.size)
         assert np.linalg.norm(to_host(got).astype(np.float64).ravel() - w.ravel()) < tol
+
+
+# Two 32-position groups a wave: a stage of the batch's own network, rows of 129
+# and of 254 (three window groups a producer wave, the widest), a ragged tile.
+@pytest.mark.parametrize("n,cin,cout,h,w,groups", [(128, 9, 33, 32, 32, 2), (1, 8, 40, 160, 160, 2),
+                                                   (2, 5, 31, 9, 129, 2), (1, 16, 24, 3, 254, 3)])
+def test_conv_split_two_groups(rnn, n, cin, cout, h, w, groups):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + cin + cout)
+    sp = rnn.ConvSpec.make(cin, cout, 3, 1, 1, h, w)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for d in (0, 1):
+        plan = rnn.dbg_conv_plan(sp, d, n, cus)
+        assert plan[3] == 2 and -(-plan[5] // 256) == groups
+    x = torch.randn((n, cin, h, w), generator=g, device="cuda")
+    wt = torch.randn((cout, cin, 3, 3), generator=g, device="cuda")
+    dy = torch.randn((n, cout, h, w), generator=g, device="cuda")
+    xd, wd = x.double().requires_grad_(True), wt.double()
+    y = (wd.reshape(cout, -1) @ torch.nn.functional.unfold(xd, 3, padding=1)).view(dy.shape)
+    dx, = torch.autograd.grad(y, xd, dy.double())
+    tol = lambda k: 2.0 ** -24 * np.sqrt(k) + 2.0 ** -23  # as test_conv_split_matches_float64
+    fwd = [rnn.conv2d_forward(sp, n, x, wt.view(-1)),
+           rnn.conv2d_forward_packed(sp, n, x, wt.view(-1),
+                                     rnn.conv_pack_weights(sp, 0, wt.view(-1)))]
+    bwd = [rnn.conv2d_backward_x(sp, n, dy, wt.view(-1)),
+           rnn.conv2d_backward_x_packed(sp, n, dy, wt.view(-1),
+                                        rnn.conv_pack_weights(sp, 1, wt.view(-1)))]
+    for a, b in zip(fwd, bwd):
+        assert rel_frob(to_host(a), to_host(y)) < tol(9 * cin)
+        assert rel_frob(to_host(b), to_host(dx)) < tol(9 * cout)
+    # an infinity, a NaN and the largest float among integers: exact
+    x = torch.randint(1, 4, x.shape, generator=g, device="cuda").float()
+    wt = torch.randint(1, 4, wt.shape, generator=g, device="cuda").float()
+    x[0, 1, 0, 5], x[n - 1, 2, h - 1, w - 1] = float("inf"), float("nan")
+    x[0, 3, 2, w - 2], wt[:, 3] = torch.finfo(torch.float32).max, 1.0
+    want = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), padding=1)
+    got = rnn.conv2d_forward(sp, n, x, wt.view(-1))
+    # (sums with the largest float round in another order: equal where they are
+    # infinite, NaN or without it)
+    got, want = to_host(got).reshape(want.shape), want.float().numpy()
+    big = np.isfinite(want) & (want > 1e30)
+    assert np.allclose(got[big], want[big], rtol=2.0 ** -22)
+    assert np.array_equal(np.where(big, 0, got), np.where(big, 0, want), equal_nan=True)
