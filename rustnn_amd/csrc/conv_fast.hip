@@ -23,7 +23,7 @@
 // 32 -> 32 @32x32 29.8 / 28.4 -> 23.4 / 22.9; 64 -> 64 @16x16 28.3 / 28.0 ->
 // 20.3 / 20.5; 128 -> 128 @8x8 28.4 / 28.5 -> 23.6 / 23.3; 96 -> 96 @16x16
 // 69.1 / 68.9 -> 37.5 / 37.7; stride 2 64 -> 128 @16x16 18.7 / 29.6 -> 20.4 /
-// 26.3.  Without loads and splitting 17-21 us are left of the stride-1 ones:
+// 24.0.  Without loads and splitting 17-21 us are left of the stride-1 ones:
 // the ramp, LDS reads and MFMAs.  Errors against 64 bits 2-3 times smaller
 // (32 -> 32 2.1e-7 / 3.0e-7 -> 0.9e-7 / 1.1e-7).
 //
@@ -627,7 +627,7 @@ __device__ __forceinline__ void store_stats(
 // 3x3 only: U window groups per producer wave, PK packed weights.
 template <int K, int S, int P, bool DX, int NPW, int MB, int WM, int EPI, int U, bool PK>
 __global__ __launch_bounds__(64 * FAST_NW * 2)
-__attribute__((amdgpu_waves_per_eu(EPI || (K == 3 && !(DX && S == 2)) ? 4 : 1))) void conv_fast_kernel(FastArgs g) {
+__attribute__((amdgpu_waves_per_eu((K == 3 ? S == 1 : EPI) ? 4 : 1))) void conv_fast_kernel(FastArgs g) {
     using T = ConvTaps<K, S, P, DX>;
     constexpr int NCLS = T::NCLS;
     // 1x1: a wave with a single output block alternates two accumulators so
@@ -942,10 +942,16 @@ static bool plan_ok(FastPlan &p, int CS, int GA, int GB, FastArgs &a) {
 // @32x32, 512 items: 23.4 us), else 128 positions (64 -> 64 @16x16, 256 or 512
 // items: 23.5 / 20.3; 48 -> 80 @23x29, 37 images: 25.2 / 21.2; one 32x32 image
 // 13.9 / 9.5), but always 256 for a row of more than 128, which fits no other
-// tile (one 160x160 image 32 -> 32: PLAN_US us, 57.1 on the generic kernel); 1x1 forward takes 256 positions when an image has as many;
-// strided 3x3 forward takes 64 positions with the waves split two ways along
-// output channels, so every wave has a 32x32 block.  A plan that does not fit
-// falls back to shrinking the tile.
+// tile (one 160x160 image 32 -> 32: 16.2 us, 57.1 on the generic kernel); 1x1
+// forward takes 256 positions when an image has as many;
+// strided 3x3 forward splits the waves two ways along output channels, so that
+// every wave has a 32x32 block at 64 positions, two at 128 where that leaves a
+// CU one item (us, fp32 pipe / 64 / 128: 32 -> 64 @32x32, 256 items, 18.9 / 22.1
+// / 19.9; 48 -> 96 @32x32 47.2 / 49.2 / 40.0; 128 -> 256 @16x16 60.0 / 61.9 /
+// 48.8; 64 -> 128 @16x16, 128 items, 18.6 / 20.7 / 28.3); 32 positions where 64
+// leave half of the CUs without one (32 images 32 -> 64 @32x32 11.8 / 13.5 /
+// 11.1 at 32, one image 11.4 / 12.9 / 10.4).  A plan that does not fit falls
+// back to shrinking the tile.
 template <int K, int S, int P, bool DX>
 static bool choose_plan(int CS, int CD, int GA, int GB, size_t n, size_t cus, FastPlan &best,
                         FastArgs &a) {
@@ -976,7 +982,21 @@ static bool choose_plan(int CS, int CD, int GA, int GB, size_t n, size_t cus, Fa
         }
     } else if (strided) {
         npos = 64;
-        if (CD > 32) r.WM = 2;
+        if (CD > 32) {
+            r.WM = 2;
+            auto tile = [&](int np, FastPlan &q) -> size_t {  // sets it; work items
+                q.TR = GA * GB <= np ? GA : std::max(1, np / GB);
+                q.IMGS = GA * GB <= np ? std::max(1, np / (GA * GB)) : 1;
+                return (n + q.IMGS - 1) / q.IMGS * ((GA + q.TR - 1) / q.TR) * ((CD + 63) / 64);
+            };
+            FastPlan q = r;
+            q.NPW = 2;
+            if (tile(128, q) >= cus && plan_ok<K, S, P, DX>(q, CS, GA, GB, a)) {
+                best = q;
+                return true;
+            }
+            if (2 * tile(64, q) <= cus) npos = 32;
+        }
     } else if (T::KK == 1 && T::NCLS == 1 && GA * GB >= 256) {
         r.NPW = 2;
         npos = 256;

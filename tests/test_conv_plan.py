@@ -25,3 +25,13 @@ def test_wide_rows_take_two_groups_a_wave():
                          (128, 32, 32, 2)):
         sp = R.ConvSpec.make(32, 32, 3, 1, 1, h, w)
         assert [R.dbg_conv_plan(sp, d, n)[3] for d in (0, 1)] == [npw, npw], (n, h, w)
+
+
+def test_strided_tiles_by_items():
+    """128 positions from one item a CU on, 32 where 64 idle half of the chip."""
+    for n, cin, cout, h, npos, npw in ((128, 32, 64, 32, 128, 2), (128, 64, 128, 16, 64, 1),
+                                       (32, 32, 64, 32, 32, 1), (1, 32, 64, 32, 32, 1),
+                                       (33, 32, 64, 32, 64, 1), (128, 16, 32, 32, 64, 1)):
+        sp = R.ConvSpec.make(cin, cout, 3, 2, 1, h, h)
+        plan = R.dbg_conv_plan(sp, 0, n)
+        assert (plan[0] * plan[1] * sp.ow, plan[3]) == (npos, npw), (n, cin, h, plan)

@@ -428,3 +428,31 @@ def test_conv_split_two_groups(rnn, n, cin, cout, h, w, groups):
     big = np.isfinite(want) & (want > 1e30)
     assert np.allclose(got[big], want[big], rtol=2.0 ** -22)
     assert np.array_equal(np.where(big, 0, got), np.where(big, 0, want), equal_nan=True)
+
+
+# The strided forward's tiles of 128, 64 and 32 positions, with a last tile of
+# fewer rows or images and channel blocks off 64.
+@pytest.mark.parametrize("n,cin,cout,h,w,npos", [(130, 9, 65, 31, 32, 128), (513, 7, 40, 15, 13, 128),
+                                                 (60, 8, 70, 17, 16, 64), (3, 10, 33, 19, 30, 32),
+                                                 (1, 8, 64, 5, 6, 32)])
+def test_conv_split_strided_forward(rnn, n, cin, cout, h, w, npos):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + cin + cout)
+    sp = rnn.ConvSpec.make(cin, cout, 3, 2, 1, h, w)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    plan = rnn.dbg_conv_plan(sp, 0, n, cus)
+    assert plan[3] == (2 if npos == 128 else 1) and plan[0] * plan[1] * sp.ow <= npos
+    x = torch.randn((n, cin, h, w), generator=g, device="cuda")
+    wt = torch.randn((cout, cin, 3, 3), generator=g, device="cuda")
+    y = wt.double().reshape(cout, -1) @ torch.nn.functional.unfold(x.double(), 3, padding=1, stride=2)
+    tol = 2.0 ** -24 * np.sqrt(9 * cin) + 2.0 ** -23  # as test_conv_split_matches_float64
+    for got in (rnn.conv2d_forward(sp, n, x, wt.view(-1)),
+                rnn.conv2d_forward_packed(sp, n, x, wt.view(-1),
+                                          rnn.conv_pack_weights(sp, 0, wt.view(-1)))):
+        assert rel_frob(to_host(got).ravel(), to_host(y).ravel()) < tol
+    x[n - 1, 1, h // 2, w // 2], x[0, 2, 0, 0] = float("inf"), float("nan")
+    want = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), stride=2, padding=1)
+    got, want = to_host(rnn.conv2d_forward(sp, n, x, wt.view(-1))).ravel(), want.numpy().ravel()
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
+    assert rel_frob(got[fine], want[fine]) < tol
