@@ -1091,6 +1091,10 @@ static PackGeo pack_geo(const FastArgs &a) {
     return pg;
 }
 
+// A kernel as a type, so that launch's static state is one of its own.
+template <void (*F)(FastArgs)>
+using Kern = std::integral_constant<void (*)(FastArgs), F>;
+
 template <int K, int S, int P, bool DX>
 static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src, const float *w,
                   const float *wp, float *dst, const ConvStats *cs) {
@@ -1127,9 +1131,12 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
             return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: no LDS for the store-pass sums");
     }
     // Persistent grid: as many workgroups as fit on the chip at once.
-    auto run = [&](auto kern) -> int {
-        (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
+    auto run = [&](auto kc) -> int {
+        constexpr auto kern = decltype(kc)::value;
+        // once an instance, not a host call a launch
+        static const hipError_t attr = hipFuncSetAttribute(
+            (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)attr;
         int occ = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, 64 * FAST_NW * 2, p.lds) !=
                 hipSuccess ||
@@ -1149,12 +1156,12 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
                 constexpr int N = decltype(nc)::value, M = decltype(mc)::value;
                 const int u = (a.ppw + FAST_NW - 1) / FAST_NW;
                 if (wp)
-                    return u == 1   ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, true>)
-                           : u == 2 ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, true>)
-                                    : run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, true>);
-                return u == 1   ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, false>)
-                       : u == 2 ? run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, false>)
-                                : run(conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, false>);
+                    return u == 1   ? run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, true>>{})
+                           : u == 2 ? run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, true>>{})
+                                    : run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, true>>{});
+                return u == 1   ? run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 1, false>>{})
+                       : u == 2 ? run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 2, false>>{})
+                                : run(Kern<conv_fast_kernel<K, S, P, DX, N, 1, M, E, 3, false>>{});
             };
             using one = std::integral_constant<int, 1>;
             using two = std::integral_constant<int, 2>;
@@ -1166,8 +1173,8 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
             return split(one{}, one{});
         } else {
             if constexpr (T::NCLS == 1)
-                if (p.NPW == 2) return run(conv_fast_kernel<K, S, P, DX, 2, 1, 1, E, 1, false>);
-            return run(conv_fast_kernel<K, S, P, DX, 1, 1, 1, E, 1, false>);
+                if (p.NPW == 2) return run(Kern<conv_fast_kernel<K, S, P, DX, 2, 1, 1, E, 1, false>>{});
+            return run(Kern<conv_fast_kernel<K, S, P, DX, 1, 1, 1, E, 1, false>>{});
         }
     };
     if constexpr (!DX)
