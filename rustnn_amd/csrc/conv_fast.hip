@@ -42,14 +42,9 @@ namespace {
 
 constexpr int FAST_NW = 4;  // waves per workgroup
 
-// Window DMA rows of 16 positions that one wave stages per channel quad:
-// row u of wave w covers window positions (w + 4u)*16 .. +16.  Row u is issued
-// at tap u % KK of a step, so its per-lane source offsets sit in a register
-// table indexed at compile time.
-template <int KK>
-struct WinRows {
-    static constexpr int MAX = KK == 1 ? 4 : KK;
-};
+// 1x1: window DMA rows of 16 positions that one wave stages per channel quad:
+// row u of wave w covers window positions (w + 4u)*16 .. +16.
+constexpr int WIN_ROWS = 4;
 
 struct FastArgs {
     const float *src;  // [N][CS][HS][WS]
@@ -71,7 +66,6 @@ struct FastArgs {
     int xwords;        // LDS words of the window: CH * plane (3x3: 3 parts of 8 bf16: 12 * plane)
     int stage;         // LDS words of one stage: window, then weight slabs
     TileGeo geo;       // window geometry in positions (chs unused)
-    int tapoff[9];     // window-position offset of each tap
     // 3x3: the two taps of each k step (one per lane half; -1 none) and their
     // window-position offsets
     int ptap[10], poff[10];
@@ -116,24 +110,21 @@ __device__ __forceinline__ StageDMA stage_dma(const FastArgs &g, int item, int c
 }
 
 // Per-lane constants of the DMA rows (computed once per workgroup).
-template <int KK>
 struct LaneDMA {
-    int toff[WinRows<KK>::MAX];   // window row u: element offset in the tile, channel lane&3
-    int tmeta[WinRows<KK>::MAX];  // window row ty | img << 8 (ty = 255: no source element)
-    int wl;                       // weight row: (lane/4)*sm + (lane%4)*sc
+    int toff[WIN_ROWS];   // window row u: element offset in the tile, channel lane&3
+    int tmeta[WIN_ROWS];  // window row ty | img << 8 (ty = 255: no source element)
+    int wl;               // weight row: (lane/4)*sm + (lane%4)*sc
     // Per work item: byte offset of window row u for channel lane&3 of
     // channel 0, or an offset >= 2^31 (beyond any buffer) when the row has
     // no source data.  A stage adds its channel's byte offset.
-    uint32_t roff[WinRows<KK>::MAX];
+    uint32_t roff[WIN_ROWS];
 };
 
-template <int KK>
-__device__ __forceinline__ void lane_dma_init(const FastArgs &g, LaneDMA<KK> &L, int wave,
-                                              int lane) {
+__device__ __forceinline__ void lane_dma_init(const FastArgs &g, LaneDMA &L, int wave, int lane) {
     const TileGeo &t = g.geo;
     const int i = lane & 3;
 #pragma unroll
-    for (int u = 0; u < WinRows<KK>::MAX; u++) {
+    for (int u = 0; u < WIN_ROWS; u++) {
         const int pos = (wave + FAST_NW * u) * 16 + (lane >> 2);
         const uint32_t mi = g.m_imgs, mt = g.m_tiwp;  // FastDiv magic multipliers
         const int img = (int)(mi ? __umulhi((uint32_t)pos, mi) : (uint32_t)pos);
@@ -150,11 +141,11 @@ __device__ __forceinline__ void lane_dma_init(const FastArgs &g, LaneDMA<KK> &L,
     L.wl = (lane >> 2) * g.sm + i * g.sc;
 }
 
-// Weight rows (mb, q, TT) of stage d gathered from W in [cout][cin][k][k]
-// order: 64-word row `wave` of each slab, lane l = wave*16 + lane/4.
-template <int KK, int SL, int TT>
+// 1x1 weight rows (mb, q) of stage d gathered from W in [cout][cin] order:
+// 64-word row `wave` of each slab, lane l = wave*16 + lane/4.
+template <int SL>
 __device__ __forceinline__ void issue_w_gather(const FastArgs &g, const StageDMA &d,
-                                               const LaneDMA<KK> &L, __amdgpu_buffer_rsrc_t rs_w,
+                                               const LaneDMA &L, __amdgpu_buffer_rsrc_t rs_w,
                                                int q, int wave, int lane) {
     const int CP = g.CH >> 1, cq = g.CH >> 3;
 #pragma unroll
@@ -162,18 +153,17 @@ __device__ __forceinline__ void issue_w_gather(const FastArgs &g, const StageDMA
         const int mrel = mb * 32 + (wave & 1) * 16;
         const int cbase = d.c0 + (wave >> 1) * CP + 4 * q;
         const bool ok = (lane >> 2) < d.mlim - mrel && (lane & 3) < g.CS - cbase;
-        const int e = L.wl + (d.grp * SL * 32 + mrel) * g.sm + cbase * g.sc + TT;
+        const int e = L.wl + (d.grp * SL * 32 + mrel) * g.sm + cbase * g.sc;
         const uint32_t off = max((uint32_t)e * 4u, ok ? 0u : DMA_OOB);
-        float *dst = d.buf + g.xwords + ((mb * cq + q) * KK + TT) * 256 + wave * 64;
+        float *dst = d.buf + g.xwords + (mb * cq + q) * 256 + wave * 64;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr_t)dst, 4, off, 0, 0, 0);
     }
 }
 
 // The per-item window row offsets (LaneDMA::roff) of stage d's work item.
-template <int KK>
-__device__ __forceinline__ void item_rows(const FastArgs &g, const StageDMA &d, LaneDMA<KK> &L) {
+__device__ __forceinline__ void item_rows(const FastArgs &g, const StageDMA &d, LaneDMA &L) {
 #pragma unroll
-    for (int u = 0; u < WinRows<KK>::MAX; u++) {
+    for (int u = 0; u < WIN_ROWS; u++) {
         const int ty = L.tmeta[u] & 255, img = L.tmeta[u] >> 8;
         const bool rowok = (unsigned)(ty - d.ylo) < (unsigned)(d.yhi - d.ylo) && img < d.nimg;
         L.roff[u] = rowok ? (uint32_t)(L.toff[u] + d.ebase) * 4u : 0x80000000u;
@@ -215,10 +205,9 @@ struct ConvPairs {
     }
 };
 
-// s_waitcnt lgkmcnt(0) / vmcnt(0) alone, and a barrier that waits for this
-// wave's LDS accesses only (loads into registers stay in flight across it).
+// s_waitcnt lgkmcnt(0) alone, and a barrier that waits for this wave's LDS
+// accesses only (loads into registers stay in flight across it).
 __device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
     wait_lds();
@@ -447,65 +436,56 @@ __device__ __forceinline__ void compute_slow(
     }
 }
 
-// One stage of the GEMM on the MFMA waves: (quad q, tap t) steps over the
-// window `xs` and the weight slabs of the current buffer, the operands of the
-// next step read from LDS while the MFMAs of the current one run.
-template <int K, int S, int P, bool DX, int NPW, int MB, int WM, int NACC>
-__device__ __forceinline__ void compute_stage(
-    const FastArgs &g, const float *__restrict__ xs, const int (&vb)[NPW],
-    f32x16 (&acc)[ConvTaps<K, S, P, DX>::NCLS][MB][NPW][NACC], int wave, int lane) {
-    using T = ConvTaps<K, S, P, DX>;
-    constexpr int KK = T::KK;
+// One 1x1 stage of the GEMM on the MFMA waves: channel quads of the window `xs`
+// and the weight slabs of the current buffer, the operands of the next quad
+// read from LDS while the MFMAs of the current one run.
+template <int NCLS, int NPW, int MB, int WM, int NACC>
+__device__ __forceinline__ void compute_stage(const FastArgs &g, const float *__restrict__ xs,
+                                              const int (&vb)[NPW],
+                                              f32x16 (&acc)[NCLS][MB][NPW][NACC], int wave,
+                                              int lane) {
     const int CQ = g.CH >> 3;
-    const int wslab = CQ * KK * 256;
+    const int wslab = CQ * 256;
     const float *ws = xs + g.xwords + lane * 4;
     constexpr int WP = FAST_NW / WM;  // waves along positions
     const float *wsw = ws + (wave / WP) * MB * wslab;  // this wave's m-blocks
 
-    auto fetch = [&](int q, int t, float4 *fa, float4 *fb) {
+    auto fetch = [&](int q, float4 *fa, float4 *fb) {
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
-            fa[mb] = *reinterpret_cast<const float4 *>(wsw + mb * wslab + (q * KK + t) * 256);
-        const float *xq = xs + (q * g.plane + g.tapoff[t]) * 4;
+            fa[mb] = *reinterpret_cast<const float4 *>(wsw + mb * wslab + q * 256);
+        const float *xq = xs + q * g.plane * 4;
 #pragma unroll
         for (int j = 0; j < NPW; j++) fb[j] = *reinterpret_cast<const float4 *>(xq + vb[j]);
     };
     float4 ca[MB], cb[NPW];
-    fetch(0, 0, ca, cb);
+    fetch(0, ca, cb);
     for (int q = 0; q < CQ; q++) {
-        static_for<0, KK>([&](auto tc) {
-            constexpr int t = decltype(tc)::value;
-            constexpr int c = T::cls(t);
-            float4 na[MB], nb[NPW];
-            if (t + 1 < KK)
-                fetch(q, t + 1 < KK ? t + 1 : 0, na, nb);
-            else if (q + 1 < CQ)
-                fetch(q + 1, 0, na, nb);
+        float4 na[MB], nb[NPW];
+        if (q + 1 < CQ) fetch(q + 1, na, nb);
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++)
+            for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-                    for (int j = 0; j < NPW; j++)
-                        acc[c][mb][j][i % NACC] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                            ca[mb][i], cb[j][i], acc[c][mb][j][i % NACC], 0, 0, 0);
+                for (int j = 0; j < NPW; j++)
+                    acc[0][mb][j][i % NACC] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                        ca[mb][i], cb[j][i], acc[0][mb][j][i % NACC], 0, 0, 0);
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) ca[mb] = na[mb];
+        for (int mb = 0; mb < MB; mb++) ca[mb] = na[mb];
 #pragma unroll
-            for (int j = 0; j < NPW; j++) cb[j] = nb[j];
-        });
+        for (int j = 0; j < NPW; j++) cb[j] = nb[j];
     }
 }
 
-// All DMA of stage `chunk` of the work item described by d (its window
+// All DMA of 1x1 stage `chunk` of the work item described by d (its window
 // rows in L.roff) into `buf`, issued by producer wave `dw`: the window rows
 // u = dw, dw + 4, ... of every channel quad, then the weights -- contiguous
 // 1 KiB slabs of the packed copy, 16 bytes a lane, or gathered from W.
-template <int K, int S, int P, bool DX, int SL>
+template <int SL>
 __device__ __forceinline__ void issue_stage(const FastArgs &g, StageDMA d, float *buf, int chunk,
-                                            const LaneDMA<ConvTaps<K, S, P, DX>::KK> &L,
-                                            __amdgpu_buffer_rsrc_t rs_w, int dw, int lane) {
-    constexpr int KK = ConvTaps<K, S, P, DX>::KK;
+                                            const LaneDMA &L, __amdgpu_buffer_rsrc_t rs_w, int dw,
+                                            int lane) {
     const int cq = g.CH >> 3;
     d.buf = buf;
     d.c0 = chunk * g.CH;
@@ -517,27 +497,23 @@ __device__ __forceinline__ void issue_stage(const FastArgs &g, StageDMA d, float
         const uint32_t chbad = g.CS - cb >= 4 ? 0u : ((lane & 3) >= g.CS - cb ? 0x80000000u : 0u);
         float *row0 = buf + (hq * g.plane + dw * 16) * 4;
 #pragma unroll
-        for (int u = 0; u < WinRows<KK>::MAX; u++)
+        for (int u = 0; u < WIN_ROWS; u++)
             if (u < g.ppw)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
                     d.rs, (lds_ptr_t)(row0 + FAST_NW * u * 64), 4, (L.roff[u] + cbytes) | chbad, 0,
                     0, 0);
     }
     if (g.wp) {
-        const int per = cq * KK;
         const __amdgpu_buffer_rsrc_t rs_p = make_rsrc(g.wp, (uint32_t)g.wpbytes);
-        for (int k = dw; k < SL * per; k += FAST_NW) {
-            const int mb = k / per, r = k - mb * per;
+        for (int k = dw; k < SL * cq; k += FAST_NW) {
+            const int mb = k / cq, r = k - mb * cq;
             const uint32_t src =
-                (uint32_t)(((d.grp * SL + mb) * g.nchunks + chunk) * per + r) * 1024u;
+                (uint32_t)(((d.grp * SL + mb) * g.nchunks + chunk) * cq + r) * 1024u;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_p, (lds_ptr_t)(buf + g.xwords + k * 256),
                                                      16, src + (uint32_t)lane * 16u, 0, 0, 0);
         }
     } else {
-        for (int q = 0; q < cq; q++)
-            static_for<0, KK>([&](auto tc) {
-                issue_w_gather<KK, SL, decltype(tc)::value>(g, d, L, rs_w, q, dw, lane);
-            });
+        for (int q = 0; q < cq; q++) issue_w_gather<SL>(g, d, L, rs_w, q, dw, lane);
     }
 }
 
@@ -689,22 +665,22 @@ __attribute__((amdgpu_waves_per_eu((K == 3 ? S == 1 : EPI) ? 4 : 1))) void conv_
             return;
         } else {
         const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(g.w, (uint32_t)g.wbytes);
-        LaneDMA<T::KK> L;
-        lane_dma_init<T::KK>(g, L, dw, lane);
+        LaneDMA L;
+        lane_dma_init(g, L, dw, lane);
         StageDMA d = stage_dma<K, S, P, DX, SL>(g, blockIdx.x, 0, smem);
-        item_rows<T::KK>(g, d, L);
-        issue_stage<K, S, P, DX, SL>(g, d, smem, 0, L, rs_w, dw, lane);
+        item_rows(g, d, L);
+        issue_stage<SL>(g, d, smem, 0, L, rs_w, dw, lane);
         int s = 0;
         for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
             for (int chunk = 0; chunk < g.nchunks; chunk++, s++) {
                 dma_wait_barrier();
                 float *nbuf = smem + ((s + 1) & 1) * g.stage;
                 if (chunk + 1 < g.nchunks) {
-                    issue_stage<K, S, P, DX, SL>(g, d, nbuf, chunk + 1, L, rs_w, dw, lane);
+                    issue_stage<SL>(g, d, nbuf, chunk + 1, L, rs_w, dw, lane);
                 } else if (item + (int)gridDim.x < nitems) {
                     d = stage_dma<K, S, P, DX, SL>(g, item + gridDim.x, 0, nbuf);
-                    item_rows<T::KK>(g, d, L);
-                    issue_stage<K, S, P, DX, SL>(g, d, nbuf, 0, L, rs_w, dw, lane);
+                    item_rows(g, d, L);
+                    issue_stage<SL>(g, d, nbuf, 0, L, rs_w, dw, lane);
                 }
             }
             if constexpr (EPI != 0) __syncthreads();  // the compute waves' store-pass sums
@@ -753,8 +729,7 @@ __attribute__((amdgpu_waves_per_eu((K == 3 ? S == 1 : EPI) ? 4 : 1))) void conv_
                 continue;
             } else {
             dma_wait_barrier();
-            compute_stage<K, S, P, DX, NPW, MB, WM, NACC>(g, smem + (s & 1) * g.stage, vb, acc,
-                                                          wave, lane);
+            compute_stage<NCLS, NPW, MB, WM, NACC>(g, smem + (s & 1) * g.stage, vb, acc, wave, lane);
             }
         }
         // acc row 8*(v/4) + 4*h + v%4 = output channel in the block, column = position.
@@ -862,7 +837,7 @@ struct FastPlan {
 };
 
 // Window geometry of a plan; returns the LDS bytes (two stage buffers), or
-// 0 when the window does not fit the per-wave DMA row tables.
+// 0 when the window does not fit the producers' registers.
 template <int K, int S, int P, bool DX>
 static size_t plan_geometry(const FastPlan &p, int GB, FastArgs &a) {
     using T = ConvTaps<K, S, P, DX>;
@@ -891,24 +866,19 @@ static size_t plan_geometry(const FastPlan &p, int GB, FastArgs &a) {
     tilegeo_finish(t);
     a.plane = (p.IMGS * t.imgs + 63) / 64 * 64;
     a.ppw = a.plane / 64;
-    if (a.ppw > (K == 3 ? SPLIT_U * FAST_NW : WinRows<T::KK>::MAX) || t.TIH > 254 || p.IMGS > 255)
+    if (a.ppw > (K == 3 ? SPLIT_U * FAST_NW : WIN_ROWS) || t.TIH > 254 || p.IMGS > 255)
         return 0;
     a.dymin = dymin;
     a.dxmin = dxmin;
-    for (int i = 0; i < 9; i++) {
-        a.tapoff[i] = 0;
-        if (i < T::KK) {
-            const int dyp = T::dy(i) - dymin, dxp = T::dx(i) - dxmin;
-            a.tapoff[i] = dyp * t.TIWP + (t.deint ? (dxp & 1) * t.HALF + (dxp >> 1) : dxp);
-        }
-    }
     a.m_imgs = t.fd_imgstr.m;
     a.m_tiwp = t.fd_tiwp.m;
     if constexpr (K == 3) {
         constexpr ConvPairs<S, P, DX> cp;
         for (int i = 0; i < 10; i++) {
+            const int tap = cp.t[i] >= 0 ? cp.t[i] : cp.t[i & ~1];
+            const int dyp = T::dy(tap) - dymin, dxp = T::dx(tap) - dxmin;
             a.ptap[i] = cp.t[i];
-            a.poff[i] = a.tapoff[cp.t[i] >= 0 ? cp.t[i] : cp.t[i & ~1]];
+            a.poff[i] = dyp * t.TIWP + (t.deint ? (dxp & 1) * t.HALF + (dxp >> 1) : dxp);
         }
         a.xwords = 12 * a.plane;
         a.stage = a.xwords + p.WM * p.MB * 5 * 3 * 256;
@@ -1193,11 +1163,10 @@ static int parts_of(const rnn_ctx *ctx, const rnn_conv_spec *sp, size_t n) {
 }
 
 
-// Packs W for the forward (dx = 0) or dX (dx = 1) kernel: slab order
-// [m-block][chunk][quad][tap][lane][4], the layout the kernel's LDS weight
-// slabs take, zero-filled beyond the channels, so that a stage's weights are
-// one contiguous copy.  Lane L of slab (q, t) holds rows m = 32*mblk + L%32
-// and channels c = chunk*CH + (L/32)*CH/2 + 4q + i.
+// Packs W for the forward (dx = 0) or dX (dx = 1) kernel in the order in which
+// the kernel stages it (PackGeo: 1x1 [m-block][chunk][quad][lane][4], 3x3
+// [m-block][chunk][tap pair][lane][8]), zero-filled beyond the channels, so that
+// a stage's weights are one contiguous read.
 __global__ __launch_bounds__(256) void conv_pack_kernel(const float *__restrict__ w, PackGeo g,
                                                         float *wp) {
     for (int r = blockIdx.x; r < g.slabs(); r += gridDim.x)
