@@ -475,8 +475,8 @@ __device__ __forceinline__ void dw_compute(const DwArgs &g, const float *__restr
     }
 }
 
-// A 3x3 wave's sums again with fp32 MFMAs from global memory: for values that
-// are not finite in the split (see bf3_nonfinite).
+// A 3x3 wave's sums again with fp32 MFMAs from global memory: for a few pixels,
+// and for values that are not finite in the split (see bf3_nonfinite).
 template <int S, int T0, int NT>
 __device__ __forceinline__ void dw_slow(const DwArgs &g, int z, int cob, int cib, int wave,
                                         int lane, f32x16 (&acc)[NT]) {
@@ -557,7 +557,9 @@ __device__ __forceinline__ void dw_mfma_wave(const DwArgs &g, float *smem, float
         }
     }
     if constexpr (K == 3) {
-        bool bad = false;
+        // sums of up to eight pixels are nearer to 64 bits in fp32 (one: 2.6e-8,
+        // split 3.0e-8; eight: 4.3e-8 / 4.4e-8; sixteen: 5.2e-8 / 4.7e-8)
+        bool bad = (long long)g.N * g.OH * g.OW <= 8;
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             acc[t] *= BF3_DOWN;

@@ -310,3 +310,23 @@ def test_attn_long_key_exponent_range(rnn, dh, th, mh, sq, sk, sv, so):
         got, want = to_host(got.contiguous()), to_host(want.contiguous())
         size = np.linalg.norm(want) + 2.0 ** -145 * np.sqrt(want.size) / tol
         assert np.linalg.norm(got - want) < tol * size
+
+
+def test_attn_long_key_one_query(rnn):
+    """One query: dV and dK are single products, rounded once (dV = P dO)."""
+    import torch
+    n, h, dh, tk = 3, 2, 64, 256
+    c = h * dh
+    idx, nrel = rnn.rel_index(1, 1, 16, 16)
+    core = rnn.Core(h, dh, 1, tk, idx, nrel, False)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+    q, kv, do = rnd(n, 1, c), rnd(n, tk, 2 * c), rnd(n, 1, c)
+    tau, rel = torch.full((h,), 0.125, device="cuda"), rnd(h * nrel) * 0.2
+    lay = (c, 0, kv, 2 * c, 0, c)
+    p, _ = core.forward(n, q, *lay, tau, rel)
+    dkv = torch.empty_like(kv)
+    core.backward(n, q, *lay, tau, p, do, torch.empty_like(q), dkv, torch.zeros_like(tau),
+                  torch.zeros_like(rel), set_dq=True, set_dkv=True)
+    want = p.view(n, h, tk, 1) * do.view(n, h, 1, dh)
+    assert torch.equal(dkv[..., c:].reshape(n, tk, h, dh).transpose(1, 2), want)

@@ -456,3 +456,17 @@ def test_conv_split_strided_forward(rnn, n, cin, cout, h, w, npos):
     fine = np.isfinite(want)
     assert np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
     assert rel_frob(got[fine], want[fine]) < tol
+
+
+@pytest.mark.parametrize("cin,cout,s,h", [(33, 40, 1, 1), (8, 16, 2, 2)])
+def test_conv_dw_one_pixel(rnn, cin, cout, s, h):
+    """One output pixel: each weight's gradient is one product, rounded once."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(cin)
+    sp = rnn.ConvSpec.make(cin, cout, 3, s, 1, h, h)
+    x = torch.randn((1, cin, h, h), generator=g, device="cuda")
+    dy = torch.randn((1, cout, 1, 1), generator=g, device="cuda")
+    dw = torch.zeros(cout * cin * 9, device="cuda")
+    rnn.conv2d_backward_w(sp, 1, dy, x, dw)
+    cols = torch.nn.functional.unfold(x, 3, padding=1, stride=s).view(-1)
+    assert torch.equal(dw.view(cout, -1), dy.view(-1, 1) * cols)
