@@ -412,3 +412,47 @@ def test_linear_backward_few_rows(rnn, rows, fin, fout):
     assert torch.equal(dw.view(fout, fin), dy.T.contiguous() @ x + 1)
     assert torch.equal(db, dy.sum(0) + 1)
     assert torch.equal(dx.view(rows, fin), dy @ w)
+
+
+_REGISTER_KERNEL = """
+import sys
+import torch
+import rustnn_amd as R
+worst = 0.0
+for m, n, k in ((64, 64, 64), (132, 68, 36), (2176, 2176, 48), (1, 1, 1), (33, 65, 67),
+                (2177, 2177, 31), (70, 31, 2051)):
+    for at in (False, True):
+        for bt in (False, True):
+            g = torch.Generator(device="cuda").manual_seed(m + n + k)
+            a = torch.randint(-3, 4, (k, m) if at else (m, k), generator=g, device="cuda").float()
+            b = torch.randint(-3, 4, (n, k) if bt else (k, n), generator=g, device="cuda").float()
+            want = ((a.T if at else a).double() @ (b.T if bt else b).double()).float()
+            for acc in (False, True):
+                c = torch.full((m, n), 7.0, device="cuda")
+                R.matmul(m, n, k, a, at, b, bt, c, acc)
+                assert torch.equal(c, want + 7.0 if acc else want), (m, n, k, at, bt, acc)
+for rows, fin, fout in ((64, 32, 48), (35, 33, 31), (2050, 130, 67)):
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, w, dy = (torch.randint(-3, 4, sh, generator=g, device="cuda").float()
+                for sh in ((rows, fin), (fout, fin), (rows, fout)))
+    bias = torch.arange(fout, device="cuda").float()
+    y = R.linear_forward(rows, fin, fout, x, w, bias)
+    assert torch.equal(y.view(rows, fout), x @ w.T.contiguous() + bias)
+    dw, db = torch.ones(fout * fin, device="cuda"), torch.ones(fout, device="cuda")
+    dx = R.linear_backward(rows, fin, fout, dy, x, w, dw, db)
+    assert torch.equal(dx.view(rows, fin), dy @ w) and torch.equal(db, dy.sum(0) + 1)
+    assert torch.equal(dw.view(fout, fin), dy.T.contiguous() @ x + 1)
+print("register kernel ok", flush=True)
+"""
+
+
+def test_register_staged_kernel():
+    """gemm_kernel, which operands of 2 GiB and more take, at every tile,
+    layout and alignment: a process in which no product takes the other one."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _REGISTER_KERNEL], cwd=root, capture_output=True,
+                       text=True, timeout=100, env=dict(os.environ, RNN_GEMM_NODMA="1"))
+    assert r.returncode == 0 and "register kernel ok" in r.stdout, r.stderr[-2000:]
