@@ -180,10 +180,13 @@ def step_profile_table():
 
 
 def template_base(t):
-    """A conv_fast_kernel template without its last argument (the store-pass
+    """A conv_fast_kernel template without its eighth argument (the store-pass
     statistics flag: the step's forward convs take the batch statistics in
     the store pass, the sweep's forward ops do not), else t."""
-    return t.rsplit(",", 1)[0] if t.startswith("conv_fast_kernel<") else t
+    if not t.startswith("conv_fast_kernel<"):
+        return t
+    args = t[len("conv_fast_kernel<"):-1].split(", ")
+    return f"conv_fast_kernel<{', '.join(args[:7] + args[8:])}>"
 
 
 def profile_kernels(op):
@@ -1102,7 +1105,7 @@ def main():
         if template_base(t_dom) != t_dom:
             roof["step_template_note"] = (
                 "the step runs this kernel with the batch statistics taken in its store pass "
-                "(last template argument 1); the sweep op above runs it without them")
+                "(eighth template argument 1); the sweep op above runs it without them")
     roof["candidates"] = candidates
     roof["share_note"] = ("launch time of every launch of the template per step / step time "
                           "(live timings of each kernel alone)")
