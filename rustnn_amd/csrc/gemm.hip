@@ -624,7 +624,9 @@ struct DmaTile {
 // 8.6 / 9.9 / 21 / 36; 8192 x 768 x 256 34.6 -> 38 / 30.2 / 37 / 32; 8192 x
 // 256 x 768 32.1 -> 29 / 26.6 / 38 / 63; 16384 x 768 x 256 69.2 -> 78 / 56.4 /
 // 62 / 63; 2048^3 148 -> 148 / 113 / 103 / 156; 4096^3 1280 -> 1202 / 918 /
-// 818 / 766 (179 TFLOP/s).  NACC: a second accumulator for the smaller part
+// 818 / 766 (179 TFLOP/s); with operands scaled, B rounded and the wave's place
+// read once 512^3 8.8, 8192 x 768 x 256 29.6, 8192 x 256 x 768 27.6, 2048^3 107,
+// 4096^3 784.  NACC: a second accumulator for the smaller part
 // products (mfma_split.h) where the registers allow it; on the 64 x 64 tile
 // it costs a workgroup a CU (8192 x 768 x 256 31.7 -> 32.5 us).
 template <bool AT, bool BT>
