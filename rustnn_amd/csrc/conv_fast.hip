@@ -1072,7 +1072,7 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
     FastArgs a;
     FastPlan p;
     if (!setup<K, S, P, DX>(sp, (size_t)n, (size_t)ctx->num_cus, a, p))
-        return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: no LDS tiling for a %dx%d grid", a.GA, a.GB);
+        return RNN_E_UNSUPPORTED;  // no LDS tiling for the grid
     a.src = src;
     a.w = w;
     a.dst = dst;
@@ -1081,7 +1081,7 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
     const long long pbytes = (long long)pack_geo<K, S, P, DX>(a).floats() * 4;
     if ((long long)p.IMGS * a.CS * a.HS * a.WS * 4 >= 0x7FFFFFF0ll || wbytes >= 0x7FFFFFF0ll ||
         pbytes >= 0x7FFFFFF0ll)
-        return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: tile source or weights beyond 2 GiB");
+        return RNN_E_UNSUPPORTED;  // tile source or weights beyond 2 GiB
     a.wbytes = (int)wbytes;
     a.wp = wp;
     a.wpbytes = (int)pbytes;
@@ -1089,7 +1089,7 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
     a.ntiles = a.tiles_a * ((n + p.IMGS - 1) / p.IMGS);
     a.ngroups = (nmblk + p.MB * p.WM - 1) / (p.MB * p.WM);
     const long long nitems = (long long)a.ntiles * a.ngroups;
-    if (nitems > 0x7fffffffll) return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: too many tiles");
+    if (nitems > 0x7fffffffll) return RNN_E_UNSUPPORTED;
     const bool stats = cs != nullptr;
     if (stats) {
         if (DX || !cs->part)
@@ -1097,8 +1097,7 @@ static int launch(rnn_ctx *ctx, const rnn_conv_spec *sp, int n, const float *src
         a.stats = *cs;
         a.npart = a.ntiles;
         p.lds += epi_lds(p);
-        if (p.lds > 160 * 1024)
-            return rnn_fail(ctx, RNN_E_UNSUPPORTED, "conv: no LDS for the store-pass sums");
+        if (p.lds > 160 * 1024) return RNN_E_UNSUPPORTED;  // no LDS for the store-pass sums
     }
     // Persistent grid: as many workgroups as fit on the chip at once.
     auto run = [&](auto kc) -> int {
@@ -1207,7 +1206,8 @@ static int geo_of(const rnn_conv_spec *sp, PackGeo *pg) {
 
 // Forward (dx = 0) or dX (dx = 1) through the specialised kernels; returns
 // RNN_E_UNSUPPORTED (without recording an error) when (k, stride, pad) has no
-// specialisation, so the caller can take the generic per-class path.  wp:
+// specialisation or the shape no tile, so the caller can take the generic
+// per-class path.  wp:
 // the weights packed by rnn_conv_pack for this direction, or null.
 int rnn_conv_fast(rnn_ctx *ctx, int dx, const rnn_conv_spec *sp, size_t n, const float *src,
                   const float *w, const float *wp, float *dst, const ConvStats *stats) {

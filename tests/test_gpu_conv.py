@@ -470,3 +470,21 @@ def test_conv_dw_one_pixel(rnn, cin, cout, s, h):
     rnn.conv2d_backward_w(sp, 1, dy, x, dw)
     cols = torch.nn.functional.unfold(x, 3, padding=1, stride=s).view(-1)
     assert torch.equal(dw.view(cout, -1), dy.view(-1, 1) * cols)
+
+
+def test_conv_without_a_tile_records_no_error(rnn):
+    """A row that no tile fits runs on the generic kernel, and is no error."""
+    import torch
+    ctx = rnn.Context()
+    sp = rnn.ConvSpec.make(4, 8, 3, 1, 1, 3, 256)
+    assert rnn.dbg_conv_plan(sp, 0, 1) is None and rnn.dbg_conv_plan(sp, 1, 1) is None
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-3, 4, (1, 4, 3, 256), generator=g, device="cuda").float()
+    wt = torch.randint(-3, 4, (8, 4, 3, 3), generator=g, device="cuda").float()
+    y = rnn.conv2d_forward(sp, 1, x, wt.view(-1), ctx=ctx)
+    dx = rnn.conv2d_backward_x(sp, 1, y, wt.view(-1), ctx=ctx)
+    want = torch.nn.functional.conv2d(x.cpu(), wt.cpu(), padding=1)
+    back = torch.nn.functional.conv_transpose2d(want, wt.cpu(), padding=1)
+    assert np.array_equal(to_host(y).ravel(), want.numpy().ravel())
+    assert np.array_equal(to_host(dx).ravel(), back.numpy().ravel())
+    assert rnn.lib().rnn_ctx_last_error(ctx.h) == b""
